@@ -157,6 +157,9 @@ int build_image(gprm_ctx* c, std::vector<char>* out) {
   img.off_adj = (int)off;   off = align16(off + 2 * nadj);
   img.off_spheres = (int)off; off = align16(off + 32 * (size_t)N);
   img.bytes = (int)off;
+  off = (off + 63) & ~(size_t)63;
+  img.off_polyrecs = (long long)off; off += sizeof(PolyRec) * (size_t)N;
+  img.off_pairrecs = (long long)off; off = align16(off + 8 * (size_t)M);
   out->assign(off, 0);
   char* b = out->data();
   for (int k = 0; k < N; ++k) {
@@ -207,17 +210,28 @@ int build_image(gprm_ctx* c, std::vector<char>* out) {
     for (int i = 0; i < p.n(); ++i)
       for (int a = 0; a < 3; ++a) h[a] = std::max(h[a], std::fabs((double)p.verts[3 * i + a] - (double)c[a]));
     const float rf = up(std::sqrt(r2));
-    // w of the second record: |c|_1 + r, the polytope's magnitude term of the
-    // bound test's margin in its own frame (the world frame for obstacles)
-    const float mag = (float)(std::fabs((double)c[0]) + std::fabs((double)c[1]) + std::fabs((double)c[2]) + rf);
-    float sp[8] = {c[0], c[1], c[2], rf, up(h[0]), up(h[1]), up(h[2]), mag};
+    // w of the second record: the radius with the bound test's margins for a
+    // polytope at rest in the world frame (bound_radius in kernels.hip)
+    const double mag = std::fabs((double)c[0]) + std::fabs((double)c[1]) + std::fabs((double)c[2]) + (double)rf;
+    const float rb = up((double)rf * (1.0 + 0x1p-8) + 0x1p-9 * mag);
+    float sp[8] = {c[0], c[1], c[2], rf, up(h[0]), up(h[1]), up(h[2]), rb};
     std::memcpy(b + img.off_spheres + 32 * (size_t)k, sp, 32);
+    PolyRec rec{};
+    for (int a = 0; a < 3; ++a) {
+      rec.v[a] = p.verts[a];
+      rec.c[a] = c[a];
+      rec.h[a] = sp[4 + a];
+    }
+    rec.r = rf;
+    rec.rb = s.sys[k] == 0 ? rb : rf;
+    rec.frame = s.sys[k];
+    std::memcpy(b + (size_t)img.off_polyrecs + sizeof(rec) * (size_t)k, &rec, sizeof(rec));
   }
   std::vector<int> order(M);
   for (int i = 0; i < M; ++i) order[i] = i;
   std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
-    int kx = s.sys[s.to[x]] * 256 + s.sys[s.from[x]], ky = s.sys[s.to[y]] * 256 + s.sys[s.from[y]];
-    return kx < ky;
+    const int kx = s.sys[s.to[x]] * 256 + s.sys[s.from[x]], ky = s.sys[s.to[y]] * 256 + s.sys[s.from[y]];
+    return kx != ky ? kx < ky : s.to[x] < s.to[y];  // runs of one Q polytope
   });
   // The kernel keeps the last P frame and the last Q frame of a segment.
   // Within a block of equal Q frame, the pairs whose P is also a moving link
@@ -278,6 +292,8 @@ int build_image(gprm_ctx* c, std::vector<char>* out) {
     int pr[4] = {vbase[s.from[i]] | (vbase[s.to[i]] << 16), s.sys[s.from[i]] | (s.sys[s.to[i]] << 8), i,
                  s.from[i] | (s.to[i] << 16)};
     std::memcpy(b + img.off_pairs + 16 * (size_t)j, pr, 16);
+    const int rec[2] = {pr[3], i};
+    std::memcpy(b + (size_t)img.off_pairrecs + 8 * (size_t)j, rec, 8);
   }
   return GPRM_OK;
 }

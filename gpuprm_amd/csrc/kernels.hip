@@ -41,6 +41,15 @@ struct T12 {
 
 __device__ __forceinline__ V3 v3(float4 a) { return V3{a.x, a.y, a.z}; }
 
+// Pointers that a kernel loads from memory (the multi-scene task tables) are
+// generic to the compiler, and their accesses flat ones, which wait for LDS
+// and global memory together.  The kernels' hot accesses name the address
+// space instead.
+#define GAS __attribute__((address_space(1)))
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ V3 v3(f32x4 a) { return V3{a.x, a.y, a.z}; }
+__device__ __forceinline__ GAS f32x4* global_f4(float4* p) { return (GAS f32x4*)p; }
+
 // sprod (geo4.h:130-132)
 __device__ __forceinline__ float dot3(const V3& u, const V3& v) {
   return (u.x * v.x + u.y * v.y) + u.z * v.z;
@@ -154,8 +163,8 @@ __device__ __forceinline__ void fk_store(const DevRobot& rb, const float* q, flo
 // quad-planar, float4 j (0..2) of link s of item i at
 // frames4[((s - 1) 3 + j) stride + i].
 __device__ __forceinline__ T12 load_frame(const float* __restrict__ frames, int item, long long stride, int sys) {
-  const float4* f = reinterpret_cast<const float4*>(frames) + (size_t)(sys - 1) * 3 * stride + item;
-  const float4 a = f[0], b = f[stride], c = f[2 * stride];
+  const GAS f32x4* f = (const GAS f32x4*)frames + (size_t)(sys - 1) * 3 * stride + item;
+  const f32x4 a = f[0], b = f[stride], c = f[2 * stride];
   T12 t;
   t.m[0] = a.x; t.m[1] = a.y; t.m[2] = a.z;  t.m[3] = a.w;
   t.m[4] = b.x; t.m[5] = b.y; t.m[6] = b.z;  t.m[7] = b.w;
@@ -167,6 +176,26 @@ __device__ __forceinline__ T12 load_frame(const float* __restrict__ frames, int 
 // double 1e-6 (collision4.h:20,242,296).  float(1e-6) = 0x1.0c6f7ap-20 lies
 // below 1e-6, so both become exact float comparisons with it.
 constexpr float kEpsBelow = 0x1.0c6f7ap-20f;
+
+// ---- bound arithmetic ------------------------------------------------------
+// The bound tests' own products: they only have to stay inside the tests'
+// margins, so they use fused multiply-adds.
+__device__ __forceinline__ float b_dot(const V3& u, const V3& v) {
+  return __builtin_fmaf(u.z, v.z, __builtin_fmaf(u.y, v.y, u.x * v.x));
+}
+__device__ __forceinline__ V3 b_apply(const T12& t, const V3& u) {
+  const float* c = t.m;
+  V3 r;
+  r.x = __builtin_fmaf(c[6], u.z, __builtin_fmaf(c[3], u.y, __builtin_fmaf(c[0], u.x, c[9])));
+  r.y = __builtin_fmaf(c[7], u.z, __builtin_fmaf(c[4], u.y, __builtin_fmaf(c[1], u.x, c[10])));
+  r.z = __builtin_fmaf(c[8], u.z, __builtin_fmaf(c[5], u.y, __builtin_fmaf(c[2], u.x, c[11])));
+  return r;
+}
+// A bounding sphere's radius with the bound tests' margins in it: r (1 +
+// 2^-8) + 2^-9 (|c|_1 + r), c its centre in the world frame.
+__device__ __forceinline__ float bound_radius(const V3& c, float r) {
+  return __builtin_fmaf(r, 1.0f + 0x1p-8f, 0x1p-9f * ((fabsf(c.x) + fabsf(c.y)) + (fabsf(c.z) + r)));
+}
 
 // ----------------------------------------------------------------------------
 // kinematics kernels
@@ -598,7 +627,7 @@ __global__ void fill_u32_kernel(unsigned int* p, unsigned int v, long long n) {
 struct Lds {
   const float4* verts;          // (x, y, z, info bits): info = row offset << 8 | degree
   const int4* pairs;            // (vbP | vbQ << 16, sysP | sysQ << 8, CRS index, kP | kQ << 16)
-  const float4* spheres;        // per polytope, own frame: (centre, sphere radius), (box half extents, |c|_1 + r)
+  const float4* spheres;        // per polytope, own frame: (centre, sphere radius), (box half extents, radius with margins)
   const unsigned short* adj;    // rows of 4k neighbour ids, padded with the row's own vertex
 };
 
@@ -664,9 +693,10 @@ __device__ __forceinline__ V2 mult23(const Orth& o, const V3& x) {
 // repeats, as in the reference, where the repetition test comes first; the
 // scan stops changing ra/rb where find_half_plane returns false.
 constexpr int kHistBatch = 2;  // history loads in flight (four spill registers at five waves per SIMD)
-__device__ __forceinline__ int sva_slow(float4* __restrict__ H, size_t hs, int& k, int l, int pq, const V3& r,
+template <class HP>
+__device__ __forceinline__ int sva_slow(HP H, size_t hs, int& k, int l, int pq, const V3& r,
                                         float dp, V3& S, V3& w) {
-  H[k * hs] = make_float4(r.x, r.y, r.z, __int_as_float(pq));
+  H[k * hs] = f32x4{r.x, r.y, r.z, __int_as_float(pq)};
   // find_half_plane returns at once (w unchanged) when w.r > 0
   const bool scan = k >= 2 && !(dot3(w, r) > 0);
   Orth o{};
@@ -682,10 +712,13 @@ __device__ __forceinline__ int sva_slow(float4* __restrict__ H, size_t hs, int& 
   V3 r0{0.0f, 0.0f, 0.0f};
   V2 ra{0.0f, 0.0f}, rb{0.0f, 0.0f};
   for (int j0 = 0; j0 < k; j0 += kHistBatch) {
-    float4 e[kHistBatch];
+    f32x4 e[kHistBatch];
 #pragma unroll
     for (int u = 0; u < kHistBatch; ++u)
-      e[u] = j0 + u < k ? H[(j0 + u) * hs] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      {
+      e[u] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      if (j0 + u < k) e[u] = H[(j0 + u) * hs];
+    }
 #pragma unroll
     for (int u = 0; u < kHistBatch; ++u) {
       const int j = j0 + u;
@@ -772,6 +805,24 @@ __device__ __forceinline__ Lds scene_global(const SceneImg& img) {
   return L;
 }
 
+// The records of a (wave-uniform) pair and polytope: scalar loads, constant
+// for the launch.
+typedef int i32x2 __attribute__((ext_vector_type(2)));
+typedef int i32x16 __attribute__((ext_vector_type(16)));
+__device__ __forceinline__ i32x2 load_pairrec(const SceneImg& img, int pair) {
+  const unsigned long long p = reinterpret_cast<unsigned long long>(img.blob) + (unsigned long long)img.off_pairrecs +
+                               8ull * (unsigned)pair;
+  return *(const __attribute__((address_space(4))) i32x2*)p;
+}
+__device__ __forceinline__ i32x16 load_polyrec(const SceneImg& img, int poly) {
+  const unsigned long long p = reinterpret_cast<unsigned long long>(img.blob) + (unsigned long long)img.off_polyrecs +
+                               sizeof(PolyRec) * (unsigned)poly;
+  return *(const __attribute__((address_space(4))) i32x16*)p;
+}
+__device__ __forceinline__ V3 rec_v3(const i32x16& r, int at) {
+  return V3{__int_as_float(r[at]), __int_as_float(r[at + 1]), __int_as_float(r[at + 2])};
+}
+
 // Deferred pair tests of one wave: a ring of CAP = sva_ring_cap(BLOCK)
 // entries in LDS, (item, pair) in ent and the item's edge (edge mode) in
 // edge.  Phase B starts as soon as CAP - 64 entries wait, so the ring never
@@ -800,7 +851,7 @@ __device__ __forceinline__ unsigned sva_unit_count(const SvaArgs& A, int nitems)
 // the ring is empty.  The gate is re-read when a pair is taken.
 template <int EDGE, int CAP>
 __device__ __forceinline__ void sva_drain(const SvaArgs& A, const Lds& L, const Ring& R,
-                                          float4* __restrict__ H, size_t hs, unsigned& d_head, unsigned d_tail,
+                                          GAS f32x4* H, size_t hs, unsigned& d_head, unsigned d_tail,
                                           unsigned& n_sep, unsigned& n_col, unsigned& n_dropped, unsigned& n_iter) {
   const int lane = threadIdx.x & 63;
   const unsigned long long lt_mask = (1ull << lane) - 1ull;
@@ -828,9 +879,9 @@ __device__ __forceinline__ void sva_drain(const SvaArgs& A, const Lds& L, const 
       int gv;
       if (EDGE) {
         bedge = R.edge[slot];
-        gv = __hip_atomic_load(&A.edge_res[bedge], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        gv = __hip_atomic_load((GAS int*)A.edge_res + bedge, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       } else {
-        gv = __hip_atomic_load(&A.word[bitem], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        gv = __hip_atomic_load((GAS int*)A.word + bitem, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
       vbP = pd.x & 0xffff;
       vbQ = pd.x >> 16;
@@ -896,9 +947,10 @@ __device__ __forceinline__ void sva_drain(const SvaArgs& A, const Lds& L, const 
       if (code != 0) {
         ++n_col;
         if (EDGE) {
-          __hip_atomic_store(&A.edge_res[bedge], code, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          __hip_atomic_store((GAS int*)A.edge_res + bedge, code, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         } else {
-          atomicMin(&A.word[bitem], ((crs + 1) << 4) | (code + 1));
+          __hip_atomic_fetch_min((GAS int*)A.word + bitem, ((crs + 1) << 4) | (code + 1), __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_AGENT);
         }
       } else {
         ++n_sep;
@@ -923,17 +975,21 @@ __device__ __forceinline__ void sva_drain(const SvaArgs& A, const Lds& L, const 
 // the wave's units (the same in every lane).
 template <int EDGE, int CAP>
 __device__ __forceinline__ void sva_units(const SvaArgs& A, const Lds& L, const Ring& R,
-                                          float4* __restrict__ H, size_t hs, SvaCounts& cnt) {
+                                          GAS f32x4* H, size_t hs, SvaCounts& cnt) {
   const int lane = threadIdx.x & 63;
   const unsigned long long lt_mask = (1ull << lane) - 1ull;
-  const int nitems = A.nitems >= 0 ? A.nitems : *A.nitems_dev;
+  // the same in every lane, as are the unit indices derived from it: said by
+  // readfirstlane, so that the pair loop and the records stay scalar also
+  // where the arguments were loaded from memory
+  const int nitems = __builtin_amdgcn_readfirstlane(A.nitems >= 0 ? A.nitems : *A.nitems_dev);
   const int M = A.img.M;
   const int PC = A.pairs_per_unit;
   const unsigned ngroups = (unsigned)((nitems + 63) >> 6);
   const unsigned nunits = sva_unit_count(A, nitems);
 
   unsigned d_head = 0, d_tail = 0;  // the ring's cursors (the same in every lane)
-  unsigned n_sep = 0, n_col = 0, n_dropped = 0, n_units = 0, n_iter = 0, n_bound = 0, n_claimed = 0;
+  unsigned n_sep = 0, n_col = 0, n_dropped = 0, n_units = 0, n_iter = 0, n_claimed = 0;
+  unsigned s_dropped = 0, s_bound = 0;  // the wave's, in scalar registers
 
   // Point mode with the codes written here: a unit is complete once the
   // ring holds none of its deferred pairs, which is certain whenever the
@@ -958,15 +1014,15 @@ __device__ __forceinline__ void sva_units(const SvaArgs& A, const Lds& L, const 
       // times slower.)
       __builtin_amdgcn_s_waitcnt(0);
       if (lane == 0)
-        old = __hip_atomic_fetch_add(&A.group_done[g], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        old = __hip_atomic_fetch_add((GAS int*)A.group_done + g, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       old = __shfl(old, 0, 64);
       if (old == A.units_per_item - 1) {
         // every unit of the group has finished: the words are final (the
         // loads below are issued after the count came back)
         const int it = (int)(g << 6) + lane;
         if (it < nitems) {
-          const int w = __hip_atomic_load(&A.word[it], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          A.codes[it] = w == 0x7fffffff ? 0 : (w & 15) - 1;
+          const int w = __hip_atomic_load((GAS int*)A.word + it, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          ((GAS int*)A.codes)[it] = w == 0x7fffffff ? 0 : (w & 15) - 1;
         }
       }
     }
@@ -1011,9 +1067,9 @@ __device__ __forceinline__ void sva_units(const SvaArgs& A, const Lds& L, const 
       unsigned b = 0xffffffffu;
       if (lane == 0) {
         bool go = true;
-        if (left < nwaves) go = __hip_atomic_load(A.counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) <
+        if (left < nwaves) go = __hip_atomic_load((GAS unsigned*)A.counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) <
                                 nunits - nstatic;
-        if (go) b = atomicAdd(A.counter, k);
+        if (go) b = __hip_atomic_fetch_add((GAS unsigned*)A.counter, k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
       b = __builtin_amdgcn_readfirstlane(b);
       if (b == 0xffffffffu || b >= nunits - nstatic) break;
@@ -1029,89 +1085,84 @@ __device__ __forceinline__ void sva_units(const SvaArgs& A, const Lds& L, const 
     const int p0 = (int)ch * PC, p1 = min(M, p0 + PC);
     // early exit: in edge mode once any sample of the edge is blocked; in
     // point mode for pairs after (in CRS order) a pair known to collide,
-    // since the reference returns the first colliding pair's code.  The gate
-    // is read lazily so that its memory latency overlaps pair work: the
-    // item's word (point mode) or edge index (edge mode) is loaded here, the
-    // edge's result two pairs later, and the gate is consulted from the
-    // unit's fourth pair on.
+    // since the reference returns the first colliding pair's code.
     int edge = 0, gate = 0x7fffffff;
+    bool open_item = active;
     if (active) {
-      if (EDGE) edge = A.item_edge[item];
-      else gate = __hip_atomic_load(&A.word[item], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> 4;
+      if (EDGE) {
+        edge = ((const GAS int*)A.item_edge)[item];
+        open_item = __hip_atomic_load((GAS int*)A.edge_res + edge, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0;
+      } else {
+        gate = __hip_atomic_load((GAS int*)A.word + item, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> 4;
+      }
     }
+    // the lanes whose item is in the launch, and those of them that are open
+    const unsigned long long act = __ballot(active), opn = EDGE ? __ballot(open_item) : act;
     // The unit's pairs run in segments that end where the ring is drained.
     // The caches are local to a segment, so nothing of them is live across
     // a drain, which has registers of its own.
     int pair = p0;
+    if (EDGE && opn == 0ull) {
+      s_dropped += (unsigned)__popcll(act) * (unsigned)(p1 - p0);
+      pair = p1;
+    }
     while (pair < p1) {
-      // wave-uniform caches: the frames of links fsP, fsQ; Q's world bounds for
-      // polytope ckQ and its start vertex cvQ
-      T12 tp, tq;
-#pragma unroll
-      for (int i = 0; i < 12; ++i) tp.m[i] = tq.m[i] = 0.0f;
-      int fsP = -1, fsQ = -1, ckQ = -1, cvQ = -1;
+      // wave-uniform cache: Q's world bounds for polytope ckQ and its start
+      // vertex
+      int ckQ = -1;
       V3 cQw{0, 0, 0}, PqW{0, 0, 0};
       // Q's box axes in the world frame, times its half extents
       V3 aQ0{0, 0, 0}, aQ1{0, 0, 0}, aQ2{0, 0, 0};
-      float magQ = 0.0f, rQ = 0.0f;
+      float RQ = 0.0f, rQ = 0.0f;
+      // the pair's operands are in scalar registers, loaded a pair ahead (its
+      // record two pairs ahead), so they cost no vector instruction.  LDS
+      // reads moved to scalar registers, selects between the frames, lane
+      // counters and unfused products had made 110 vector instructions a
+      // pair; now it is about 30, and 25 more where the boxes are needed
+      // (4.28 -> 3.57 ms for 4M configurations of the 7-DOF scene, 3.83 ->
+      // 3.26 ms for the 6-DOF roadmap's edges).
+      i32x2 pr1 = load_pairrec(A.img, pair), pr2 = load_pairrec(A.img, min(pair + 1, M - 1));
+      i32x16 poly1 = load_polyrec(A.img, pr1[0] & 0xffff);
       for (; pair < p1; ++pair) {
-        // the record is the same in every lane: keep it in scalar registers
-        const int4 pdv = L.pairs[pair];
-        const int4 pd = make_int4(__builtin_amdgcn_readfirstlane(pdv.x), __builtin_amdgcn_readfirstlane(pdv.y),
-                                  __builtin_amdgcn_readfirstlane(pdv.z), __builtin_amdgcn_readfirstlane(pdv.w));
-        const int crs = pd.z;
-        const int vbP = pd.x & 0xffff, vbQ = pd.x >> 16;
-        const int sP = pd.y & 255, sQ = pd.y >> 8;
-        const bool sysP0 = sP == 0, sysQ0 = sQ == 0;
-        // the cache tags are wave-uniform: compared as scalars
-        // (readfirstlane).  Frames are loaded by every lane: an inactive
-        // lane's item is below the plane stride (the item count rounded up
-        // to 64), and what it computes from them is masked out below.
-        if (!sysP0 && sP != __builtin_amdgcn_readfirstlane(fsP)) {
-          tp = load_frame(A.frames, item, A.fstride, sP);
-          fsP = sP;
-        }
-        if (!sysQ0 && sQ != __builtin_amdgcn_readfirstlane(fsQ)) {
-          tq = load_frame(A.frames, item, A.fstride, sQ);
-          fsQ = sQ;
-          ckQ = cvQ = -1;
-        }
-        const int kP = pd.w & 0xffff, kQ = pd.w >> 16;
-        if (vbQ != __builtin_amdgcn_readfirstlane(cvQ)) {
-          const V3 vq = v3(L.verts[vbQ]);
-          PqW = sysQ0 ? vq : t_apply(tq, vq);
-          cvQ = vbQ;
-        }
-        if (kQ != __builtin_amdgcn_readfirstlane(ckQ)) {
-          const float4 b0 = L.spheres[2 * kQ], b1 = L.spheres[2 * kQ + 1];
-          cQw = sysQ0 ? v3(b0) : t_apply(tq, v3(b0));
-          magQ = fabsf(cQw.x) + fabsf(cQw.y) + fabsf(cQw.z) + b0.w;
-          rQ = b0.w;
-          if (sysQ0) {
-            aQ0 = V3{b1.x, 0.0f, 0.0f};
-            aQ1 = V3{0.0f, b1.y, 0.0f};
-            aQ2 = V3{0.0f, 0.0f, b1.z};
+        const i32x2 pr = pr1;
+        const i32x16 cur = poly1;
+        pr1 = pr2;
+        poly1 = load_polyrec(A.img, pr1[0] & 0xffff);
+        pr2 = load_pairrec(A.img, min(pair + 2, M - 1));
+        const int crs = pr[1], kQ = (int)((unsigned)pr[0] >> 16);
+        // Frames are loaded by every lane: an inactive lane's item is below
+        // the plane stride (the item count rounded up to 64), and what it
+        // computes from them is masked out below.
+        if (kQ != ckQ) {
+          const i32x16 rq = load_polyrec(A.img, kQ);
+          const V3 hq = rec_v3(rq, 8);
+          rQ = __int_as_float(rq[7]);
+          if (rq[11] == 0) {
+            PqW = rec_v3(rq, 0);
+            cQw = rec_v3(rq, 4);
+            aQ0 = V3{hq.x, 0.0f, 0.0f};
+            aQ1 = V3{0.0f, hq.y, 0.0f};
+            aQ2 = V3{0.0f, 0.0f, hq.z};
           } else {
-            aQ0 = V3{tq.m[0] * b1.x, tq.m[1] * b1.x, tq.m[2] * b1.x};
-            aQ1 = V3{tq.m[3] * b1.y, tq.m[4] * b1.y, tq.m[5] * b1.y};
-            aQ2 = V3{tq.m[6] * b1.z, tq.m[7] * b1.z, tq.m[8] * b1.z};
+            const T12 tq = load_frame(A.frames, item, A.fstride, rq[11]);
+            PqW = b_apply(tq, rec_v3(rq, 0));
+            cQw = b_apply(tq, rec_v3(rq, 4));
+            aQ0 = V3{tq.m[0] * hq.x, tq.m[1] * hq.x, tq.m[2] * hq.x};
+            aQ1 = V3{tq.m[3] * hq.y, tq.m[4] * hq.y, tq.m[5] * hq.y};
+            aQ2 = V3{tq.m[6] * hq.z, tq.m[7] * hq.z, tq.m[8] * hq.z};
           }
+          RQ = bound_radius(cQw, rQ);
           ckQ = kQ;
         }
-        if (EDGE && pair == p0 + 2)  // an inactive lane reads edge 0's result, unused
-          gate = __hip_atomic_load(&A.edge_res[edge], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 ? 0 : 0x7fffffff;
         // Every lane evaluates the bound test (a SIMD runs the whole wave
-        // anyway); the lane's conditions (its item active, its pair not
-        // dropped by the gate) are applied to the result, which keeps the
-        // exec-mask switching out of the loop.
-        // (bitwise & on the conditions: no short-circuit branches)
-        const bool drop = active & (pair >= p0 + 4) & (EDGE ? gate == 0 : gate <= crs);
-        const bool test = active & !drop;
+        // anyway); the lane's conditions (its item open, its pair not
+        // dropped by the gate) are applied to the result.
+        const unsigned long long test = EDGE ? opn : act & __ballot(gate > crs);
         // Start of the pair (collision4.h:228-244) and the bound decision
         // of iteration 0: iteration 0 returns 0 whenever
         // S.normalize(q0 - p0) >= -1e-6 for the support vertices p0, q0
         // the climbs find, S = normalize(D) with D the difference of the
-        // two start vertices.  If the bounding boxes show S.(q - p) > 0
+        // two start vertices.  If the bounds show S.(q - p) > 0
         // with a wide margin for every vertex p of P and q of Q, that holds
         // whichever vertices the climbs would pick, so the pair test ends
         // here exactly as the reference's does (code 0, one
@@ -1120,60 +1171,74 @@ __device__ __forceinline__ void sva_units(const SvaArgs& A, const Lds& L, const 
         // the reference's iteration by orders of magnitude.  Both sides of
         // the test scale with |S|, so it runs on D itself: the reference's
         // S differs from D/|D| by a relative 1e-7, far inside the margin.
-        // The test also requires |D|_1 > 1e-5, so |D|_2 > 5.7e-6 stays
-        // clear of the reference's override of S for |D| <= 1e-6; a NaN D
-        // never passes (such pairs are deferred to the exact test).
-        const V3 vp = v3(L.verts[vbP]);
-        const V3 Pp = sysP0 ? vp : t_apply(tp, vp);
-        const V3 S{PqW.x - Pp.x, PqW.y - Pp.y, PqW.z - Pp.z};
+        // The test also requires |D|_2 > 1e-5, which stays clear of the
+        // reference's override of S for |D| <= 1e-6; a NaN D never passes
+        // (such pairs are deferred to the exact test).  Nothing here has to
+        // be the reference's float, so it may use fused multiply-adds.
         // First the bounding spheres: every vertex lies within r of its
         // polytope's centre c, so S.(q - p) >= S.(cQ - cP) - (rP + rQ)|S|.
-        // That costs a few operations once cP is in the world frame and
-        // decides most pairs; the boxes' support extents along S (sum_a
-        // |S.axis_a| h_a, axes the frame's rotation columns) are tighter
-        // and are computed only when some lane's pair the spheres leave
-        // open.  The margin is the same in both: 2^-10 of |S|_1 times the
-        // magnitudes |c|_1 + r per side (precomputed for world-frame
-        // polytopes); the spheres' comparison is made on squares (no square
-        // root), both sides non-negative, the right one inflated by 2^-8
-        // against their rounding.
-        const float4 b0 = L.spheres[2 * kP], b1 = L.spheres[2 * kP + 1];
-        const V3 cPw = sysP0 ? v3(b0) : t_apply(tp, v3(b0));
-        const float magP = sysP0 ? b1.w : fabsf(cPw.x) + fabsf(cPw.y) + fabsf(cPw.z) + b0.w;
-        const float sn1 = fabsf(S.x) + fabsf(S.y) + fabsf(S.z);
-        const float dc = dot3(S, V3{cQw.x - cPw.x, cQw.y - cPw.y, cQw.z - cPw.z});
-        const float thr = 0x1p-10f * (magQ + magP) * sn1;
-        const bool open = (sn1 > 1e-5f) & (dc > thr);
-        const float A = dc - thr, rsum = b0.w + rQ;
-        bool sep = open & (A * A > (rsum * rsum) * dot3(S, S) * (1.0f + 0x1p-8f));
-        const bool need_box = test & open & !sep;
-        if (__ballot(need_box) != 0ull) {
-          const float boxQ = (fabsf(dot3(S, aQ0)) + fabsf(dot3(S, aQ1))) + fabsf(dot3(S, aQ2));
-          float boxP;
-          if (sysP0) {
-            boxP = (fabsf(S.x) * b1.x + fabsf(S.y) * b1.y) + fabsf(S.z) * b1.z;
-          } else {
-            const V3 sp = t_apply_rot_inv(tp, S);
-            boxP = (fabsf(sp.x) * b1.x + fabsf(sp.y) * b1.y) + fabsf(sp.z) * b1.z;
+        // That costs a few operations and decides most pairs; the boxes'
+        // support extents along S (sum_a |S.axis_a| h_a, axes the frame's
+        // rotation columns) are tighter and are computed only when some
+        // lane's pair the spheres leave open.  The margin is 2^-10 of |S|_1
+        // times the magnitudes |c|_1 + r per side; for the spheres it is part
+        // of the radii (bound_radius: |S|_1 <= sqrt(3) |S|_2 and 2^-9 >
+        // sqrt(3) 2^-10), and the comparison is made on squares (no square
+        // root), the radii inflated by 2^-8 against their rounding.
+        const V3 vp = rec_v3(cur, 0), cP = rec_v3(cur, 4), hP = rec_v3(cur, 8);
+        const float rbP = __int_as_float(cur[3]), rP = __int_as_float(cur[7]);
+        const int sP = cur[11];
+        // the lanes of `test` that the bounds decide; P's half extents along
+        // S come from boxP
+        auto decided = [&](const V3& S, const V3& E, float rad, auto boxP) {
+          const float dc = b_dot(S, E), ss = b_dot(S, S);
+          const unsigned long long cand = __ballot(ss > 1e-10f) & __ballot(dc > 0.0f) & test;
+          unsigned long long sep = __ballot(dc * dc > (rad * rad) * ss) & cand;
+          if (cand != sep) {
+            const float boxQ = (fabsf(b_dot(S, aQ0)) + fabsf(b_dot(S, aQ1))) + fabsf(b_dot(S, aQ2));
+            // |cP|_1 <= |cQ|_1 + |E|_1
+            const float magQ = (fabsf(cQw.x) + fabsf(cQw.y)) + fabsf(cQw.z);
+            const float magE = (fabsf(E.x) + fabsf(E.y)) + fabsf(E.z);
+            const float mag = (magQ + magQ) + (magE + (rQ + rP));
+            const float thr = 0x1p-10f * mag * (fabsf(S.x) + fabsf(S.y) + fabsf(S.z));
+            sep |= __ballot(dc - boxQ - boxP() > thr) & cand;
           }
-          sep = sep | (open & (dc - boxQ - boxP > thr));
+          return sep;
+        };
+        unsigned long long sep;
+        if (sP == 0) {
+          const V3 S{PqW.x - vp.x, PqW.y - vp.y, PqW.z - vp.z};
+          const V3 E{cQw.x - cP.x, cQw.y - cP.y, cQw.z - cP.z};
+          sep = decided(S, E, RQ + rbP,
+                        [&]() { return (fabsf(S.x) * hP.x + fabsf(S.y) * hP.y) + fabsf(S.z) * hP.z; });
+        } else {
+          // P's frame is loaded for the pair and not kept: a kept one would
+          // have to be copied around every pair of a polytope at rest, and
+          // few of a scene's pairs have both polytopes on links
+          const T12 tp = load_frame(A.frames, item, A.fstride, sP);
+          const V3 Pp = b_apply(tp, vp), cw = b_apply(tp, cP);
+          const V3 S{PqW.x - Pp.x, PqW.y - Pp.y, PqW.z - Pp.z};
+          const V3 E{cQw.x - cw.x, cQw.y - cw.y, cQw.z - cw.z};
+          sep = decided(S, E, RQ + bound_radius(cw, rP), [&]() {
+            const V3 sp = t_apply_rot_inv(tp, S);
+            return (fabsf(sp.x) * hP.x + fabsf(sp.y) * hP.y) + fabsf(sp.z) * hP.z;
+          });
         }
-        sep = sep & test;
-        n_dropped += drop ? 1u : 0u;
-        n_bound += sep ? 1u : 0u;
-        n_sep += sep ? 1u : 0u;
-        const bool defer = test & !sep;
+        s_dropped += (unsigned)__popcll(act & ~test);
+        s_bound += (unsigned)__popcll(sep);
         // append the undecided pairs to the ring; drain it once CAP - 64 wait
-        const unsigned long long dm = __ballot(defer);
-        if (defer) {
-          const unsigned slot = (d_tail + (unsigned)__popcll(dm & lt_mask)) & (CAP - 1);
-          R.ent[slot] = make_int2(item, pair);
-          if (EDGE) R.edge[slot] = edge;
-        }
-        d_tail += (unsigned)__popcll(dm);
-        if (d_tail - d_head >= CAP - 64) {
-          ++pair;
-          break;
+        const unsigned long long dm = test & ~sep;
+        if (dm != 0ull) {
+          if ((dm >> lane) & 1ull) {
+            const unsigned slot = (d_tail + (unsigned)__popcll(dm & lt_mask)) & (CAP - 1);
+            R.ent[slot] = make_int2(item, pair);
+            if (EDGE) R.edge[slot] = edge;
+          }
+          d_tail += (unsigned)__popcll(dm);
+          if (d_tail - d_head >= CAP - 64) {
+            ++pair;
+            break;
+          }
         }
       }
       if (d_tail - d_head >= CAP - 64) {
@@ -1197,12 +1262,16 @@ __device__ __forceinline__ void sva_units(const SvaArgs& A, const Lds& L, const 
   if (d_tail != d_head) sva_drain<EDGE, CAP>(A, L, R, H, hs, d_head, d_tail, n_sep, n_col, n_dropped, n_iter);
   if (fuse) complete_pending();
 
+  if (lane == 0) {
+    n_sep += s_bound;
+    n_dropped += s_dropped;
+    cnt.bound += s_bound;
+  }
   cnt.sep += n_sep;
   cnt.col += n_col;
   cnt.dropped += n_dropped;
   cnt.units += n_units;
   cnt.iter += n_iter;
-  cnt.bound += n_bound;
   cnt.claimed += n_claimed;
 }
 
@@ -1239,7 +1308,7 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVE
   const Lds L = GS ? scene_global(A.img) : stage_scene<BLOCK>(A.img, smem + sva_ring_bytes(BLOCK) / 16);
   const Ring R = wave_ring<BLOCK>(smem);
   __syncthreads();
-  float4* __restrict__ H = A.hist + (size_t)blockIdx.x * BLOCK + threadIdx.x;
+  GAS f32x4* const H = global_f4(A.hist) + (size_t)blockIdx.x * BLOCK + threadIdx.x;
   const size_t hs = (size_t)gridDim.x * BLOCK;
   SvaCounts c;
   sva_units<EDGE, sva_ring_cap(BLOCK)>(A, L, R, H, hs, c);
@@ -1259,7 +1328,7 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVE
   extern __shared__ int4 smem[];
   __shared__ int s_live;
   if (threadIdx.x == 0) atomicMin(t_start, (unsigned long long)wall_clock64());
-  float4* __restrict__ H = tasks[0].a.hist + (size_t)blockIdx.x * BLOCK + threadIdx.x;
+  GAS f32x4* const H = global_f4(tasks[0].a.hist) + (size_t)blockIdx.x * BLOCK + threadIdx.x;
   const size_t hs = (size_t)gridDim.x * BLOCK;
   // dynamic LDS as in sva_kernel: deferral rings, then the scene image
   const Ring R = wave_ring<BLOCK>(smem);
@@ -1315,7 +1384,7 @@ __device__ void fk_frames(const DevRobot& rb, const float* q, T12* out) {
 // The full separating-vector test of one pair (collision4.h:227-332), as
 // sva_drain runs it per lane; H: this lane's iteration history, stride hs.
 __device__ int sva_pair_full(const Lds& L, const T12& tp, const T12& tq, bool sysP0, bool sysQ0, int vbP, int vbQ,
-                             float4* H, size_t hs) {
+                             f32x4* H, size_t hs) {
   const V3 vq0 = v3(L.verts[vbQ]), vp0 = v3(L.verts[vbP]);
   const V3 Pq = sysQ0 ? vq0 : t_apply(tq, vq0);
   const V3 Pp = sysP0 ? vp0 : t_apply(tp, vp0);
@@ -1349,7 +1418,7 @@ __global__ void __launch_bounds__(BLOCK) point_small_kernel(SceneImg img, DevRob
   // dynamic LDS: the scene image, the frames, the lanes' iteration history
   const Lds L = stage_scene<BLOCK>(img, smem);
   T12* frames = reinterpret_cast<T12*>(reinterpret_cast<char*>(smem) + img.bytes);
-  float4* H = reinterpret_cast<float4*>(reinterpret_cast<char*>(smem) + img.bytes + sizeof(T12) * kMaxDofDev) +
+  f32x4* H = reinterpret_cast<f32x4*>(reinterpret_cast<char*>(smem) + img.bytes + sizeof(T12) * kMaxDofDev) +
               threadIdx.x;
   __shared__ int s_word;
   const float* q = qs.q[blockIdx.x];

@@ -38,14 +38,32 @@ struct DevRobot {
 //   adj      uint16[...]   neighbour vertex ids (scene-global), rows as stored,
 //                          each padded to a multiple of 4 with the row's vertex
 //   spheres  float4[2N]    per polytope, own frame: (centre, sphere radius),
-//                          (box half extents, |centre|_1 + radius), rounded
-//                          outwards
+//                          (box half extents, the radius with the bound test's
+//                          margins for a polytope at rest), rounded outwards
+// Behind the staged image lie tables that are read through the scalar cache
+// (byte offsets, 64-byte aligned), small enough to stay in its 16 KB for
+// scenes of up to about 100 polytopes and 900 pairs:
+//   polyrecs PolyRec[N]    the bound test's operands of each polytope
+//   pairrecs int2[M]       (polytope P | polytope Q << 16, CRS index), in pair order
 struct SceneImg {
   const int4* blob;        // device pointer to the image
-  int bytes;               // image size, multiple of 16
+  int bytes;               // size of the staged part, multiple of 16
   int off_verts, off_pairs, off_adj, off_spheres;
+  long long off_polyrecs, off_pairrecs;
   int sumn, summ, M, N;
 };
+
+// Operands of a polytope in the bound test (64 bytes, one scalar load), in
+// its own frame.
+struct PolyRec {
+  float v[3], rb;  // the start vertex; the sphere radius, with the bound test's
+                   // margins if the polytope is at rest (frame 0)
+  float c[3], r;   // the bounding sphere
+  float h[3];      // the box half extents
+  int frame;       // its link, 0 for the world
+  int pad[4];
+};
+static_assert(sizeof(PolyRec) == 64, "one 64-byte scalar load");
 
 // Per-launch arguments of the separating-vector kernel.
 struct SvaArgs {
