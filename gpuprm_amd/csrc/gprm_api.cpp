@@ -123,6 +123,66 @@ void fill_robot(const Scene& s, DevRobot* rb) {
 
 size_t align16(size_t x) { return (x + 15) & ~(size_t)15; }
 
+// Certificate factor of a polytope's support scan (support in kernels.hip):
+// with w the vertex whose product with a direction d is largest, by more than
+// factor |d|_1 above every other vertex's, the hill climb in floats ends at w
+// from any start; inf if that cannot be promised, or if the climb is the
+// cheaper way (more vertices than kScanVertices).
+//   The polytope lies in the cone of the stored neighbours' edges e_i at each
+// vertex u: w - u = sum l_i e_i, l_i >= 0.  So (w - u).d <= (sum l_i) max e_i.d,
+// and u has a neighbour better by (w - u).d / L, L the largest sum l_i over
+// all u and w.  The climb's products err by at most g = 3.1 2^-24 vmax |d|_1
+// each, the scan's too: it suffices that the scan's margin exceeds
+// (2 L + 2) g.  The coefficients are checked here from the stored adjacency,
+// so a row that misses edges has no factor.
+constexpr int kScanVertices = 32, kScanDegree = 16;
+float support_factor(const Polytope& p) {
+  const float none = INFINITY;
+  const int n = p.n();
+  if (n > kScanVertices) return none;
+  auto at = [&](int v, int a) { return (double)p.verts[3 * v + a]; };
+  double vmax = 0.0, L = 0.0;
+  for (float x : p.verts) vmax = std::max(vmax, std::fabs((double)x));
+  for (int u = 0; u < n; ++u) {
+    const int deg = p.cnt[u];
+    if (deg > kScanDegree) return none;
+    double e[kScanDegree][3];
+    for (int i = 0; i < deg; ++i)
+      for (int a = 0; a < 3; ++a) e[i][a] = at(p.dest[p.dsp[u] + i], a) - at(u, a);
+    for (int w = 0; w < n; ++w) {
+      if (w == u) continue;
+      const double x[3] = {at(w, 0) - at(u, 0), at(w, 1) - at(u, 1), at(w, 2) - at(u, 2)};
+      double best = 1e300;
+      for (int i = 0; i < deg && best > 1.0; ++i)  // a neighbour: its own edge
+        if (p.dest[p.dsp[u] + i] == w) best = 1.0;
+      for (int i = 0; i < deg && best > 4.0; ++i)
+        for (int j = i + 1; j < deg && best > 4.0; ++j) {
+          const double c[3] = {e[i][1] * e[j][2] - e[i][2] * e[j][1], e[i][2] * e[j][0] - e[i][0] * e[j][2],
+                               e[i][0] * e[j][1] - e[i][1] * e[j][0]};
+          for (int k = j + 1; k < deg && best > 4.0; ++k) {
+            const double* f = e[k];
+            const double det = c[0] * f[0] + c[1] * f[1] + c[2] * f[2];
+            auto len = [](const double* v) { return std::sqrt(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]); };
+            if (!(std::fabs(det) > 1e-5 * len(e[i]) * len(e[j]) * len(f))) continue;
+            auto det3 = [](const double* p0, const double* p1, const double* p2) {
+              return p0[0] * (p1[1] * p2[2] - p1[2] * p2[1]) - p0[1] * (p1[0] * p2[2] - p1[2] * p2[0]) +
+                     p0[2] * (p1[0] * p2[1] - p1[1] * p2[0]);
+            };
+            const double li = det3(x, e[j], f) / det, lj = det3(e[i], x, f) / det, lk = det3(e[i], e[j], x) / det;
+            if (li < -1e-12 || lj < -1e-12 || lk < -1e-12) continue;
+            best = std::min(best, li + lj + lk);
+          }
+        }
+      if (best > 1e6) return none;
+      L = std::max(L, best);
+    }
+  }
+  // the products' errors, and 1e-8 vmax for the coefficients' own
+  const double f = ((2.0 * L + 2.0) * 3.41 * 0x1p-24 + 1e-8) * vmax;
+  const float r = (float)(f * (1.0 + 1e-6));
+  return std::isfinite(r) ? r : none;
+}
+
 // Pack the scene image (layout documented at SceneImg).  The kernel visits
 // pairs grouped by the frames they need; each pair keeps its index in the
 // reference's CRS order (polytope4data.h:343-357: by `from`, then as given),
@@ -155,7 +215,7 @@ int build_image(gprm_ctx* c, std::vector<char>* out) {
   img.off_verts = (int)off; off = align16(off + 16 * (size_t)sumn);
   img.off_pairs = (int)off; off = align16(off + 16 * (size_t)M);
   img.off_adj = (int)off;   off = align16(off + 2 * nadj);
-  img.off_spheres = (int)off; off = align16(off + 32 * (size_t)N);
+  img.off_hulls = (int)off; off = align16(off + 8 * (size_t)N);
   img.bytes = (int)off;
   off = (off + 63) & ~(size_t)63;
   img.off_polyrecs = (long long)off; off += sizeof(PolyRec) * (size_t)N;
@@ -210,22 +270,24 @@ int build_image(gprm_ctx* c, std::vector<char>* out) {
     for (int i = 0; i < p.n(); ++i)
       for (int a = 0; a < 3; ++a) h[a] = std::max(h[a], std::fabs((double)p.verts[3 * i + a] - (double)c[a]));
     const float rf = up(std::sqrt(r2));
-    // w of the second record: the radius with the bound test's margins for a
-    // polytope at rest in the world frame (bound_radius in kernels.hip)
+    // the radius with the bound test's margins for a polytope at rest in the
+    // world frame (bound_radius in kernels.hip)
     const double mag = std::fabs((double)c[0]) + std::fabs((double)c[1]) + std::fabs((double)c[2]) + (double)rf;
     const float rb = up((double)rf * (1.0 + 0x1p-8) + 0x1p-9 * mag);
-    float sp[8] = {c[0], c[1], c[2], rf, up(h[0]), up(h[1]), up(h[2]), rb};
-    std::memcpy(b + img.off_spheres + 32 * (size_t)k, sp, 32);
     PolyRec rec{};
     for (int a = 0; a < 3; ++a) {
       rec.v[a] = p.verts[a];
       rec.c[a] = c[a];
-      rec.h[a] = sp[4 + a];
+      rec.h[a] = up(h[a]);
     }
     rec.r = rf;
     rec.rb = s.sys[k] == 0 ? rb : rf;
     rec.frame = s.sys[k];
     std::memcpy(b + (size_t)img.off_polyrecs + sizeof(rec) * (size_t)k, &rec, sizeof(rec));
+    const float cert = support_factor(p);
+    int hull[2] = {std::isfinite(cert) ? p.n() : 0, 0};
+    std::memcpy(&hull[1], &cert, 4);
+    std::memcpy(b + img.off_hulls + 8 * (size_t)k, hull, 8);
   }
   std::vector<int> order(M);
   for (int i = 0; i < M; ++i) order[i] = i;

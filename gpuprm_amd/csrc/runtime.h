@@ -37,9 +37,9 @@ struct DevRobot {
 //                          by the frames they need
 //   adj      uint16[...]   neighbour vertex ids (scene-global), rows as stored,
 //                          each padded to a multiple of 4 with the row's vertex
-//   spheres  float4[2N]    per polytope, own frame: (centre, sphere radius),
-//                          (box half extents, the radius with the bound test's
-//                          margins for a polytope at rest), rounded outwards
+//   hulls    int2[N]       per polytope: (its vertex count, the bits of the
+//                          support scan's certificate factor; see support in
+//                          kernels.hip), (0, inf): no scan
 // Behind the staged image lie tables that are read through the scalar cache
 // (byte offsets, 64-byte aligned), small enough to stay in its 16 KB for
 // scenes of up to about 100 polytopes and 900 pairs:
@@ -48,7 +48,7 @@ struct DevRobot {
 struct SceneImg {
   const int4* blob;        // device pointer to the image
   int bytes;               // size of the staged part, multiple of 16
-  int off_verts, off_pairs, off_adj, off_spheres;
+  int off_verts, off_pairs, off_adj, off_hulls;
   long long off_polyrecs, off_pairrecs;
   int sumn, summ, M, N;
 };
