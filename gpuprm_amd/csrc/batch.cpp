@@ -108,13 +108,14 @@ struct gprm_batch {
   // multi-scene edge calls
   EdgeSignature esig;
   bool have_esig = false;
-  std::vector<long long> e_base;    // per scene: first edge in e_testnum / e_stride
-  DevBuf e_testnum, e_stride, e_max, e_total, e_clock, e_pro;
+  std::vector<long long> e_base;    // per scene: first edge in e_testnum
+  DevBuf e_testnum, e_max, e_total, e_clock, e_pro;
   int e_pro_blocks = 0, e_pro_tasks = 0;
   std::vector<int> e_plan_key;      // per scene largest testnum of the current plan
   bool have_eplan = false;
   std::vector<std::unique_ptr<EdgeStep>> e_steps;
-  DevBuf e_items, e_frames, e_ctl;  // step buffers; e_ctl: (items, work counter, units done) per task
+  size_t cull_lds = 0;  // LDS of the kinematics launches that write pair masks
+  DevBuf e_items, e_frames, e_masks, e_ctl;  // step buffers; e_ctl: (items, work counter, units done) per task
   int e_ntasks = 0;
   hipGraph_t egraph = nullptr;
   hipGraphExec_t eexec = nullptr;
@@ -327,6 +328,10 @@ int signature(gprm_batch* b, const float* const* d_q, const long long* offset, c
 
 // ---- multi-scene edge calls -------------------------------------------------
 
+// Whether the kinematics launches write scene s's pair masks (their tables
+// fit a block of kFkBlock threads).
+bool scene_masks(const gprm_batch* b, int s) { return cull_fits(b->ctx[s]->img, kFkBlock); }
+
 int edge_signature(gprm_batch* b, const float* const* d_qs, const float* const* d_qe, const long long* offset,
                    const int* n, int* const* d_res, EdgeSignature* sg) {
   const int S = (int)b->ctx.size();
@@ -356,7 +361,6 @@ EdgeArgs edge_args(gprm_batch* b, const EdgeSignature& sg, int s) {
   ea.offset = sg.off[s];
   ea.nedges = sg.n[s];
   ea.testnum = b->e_testnum.as<int>() + b->e_base[s];
-  ea.stride = b->e_stride.as<int>() + b->e_base[s];
   ea.edge_res = static_cast<int*>(const_cast<void*>(sg.res[s]));
   return ea;
 }
@@ -368,7 +372,6 @@ int edge_prepare(gprm_batch* b, const EdgeSignature& sg) {
   for (int s = 0; s < S; ++s) b->e_base[s + 1] = b->e_base[s] + sg.n[s];
   const size_t E = (size_t)std::max(1LL, b->e_base[S]);
   BHIP(b, b->e_testnum.ensure(sizeof(int) * E), "hipMalloc testnum");
-  BHIP(b, b->e_stride.ensure(sizeof(int) * E), "hipMalloc stride");
   BHIP(b, b->e_max.ensure(sizeof(int) * (size_t)S), "hipMalloc");
   BHIP(b, b->e_total.ensure(sizeof(unsigned long long) * (size_t)S), "hipMalloc");
   // completion clocks per scene, then the start clock
@@ -382,7 +385,6 @@ int edge_prepare(gprm_batch* b, const EdgeSignature& sg) {
     t.rb = b->ctx[s]->rb;
     t.dq = b->ctx[s]->dq;
     t.testnum = b->e_testnum.as<int>() + b->e_base[s];
-    t.stride = b->e_stride.as<int>() + b->e_base[s];
     t.max_testnum = b->e_max.as<int>() + s;
     t.total = b->e_total.as<unsigned long long>() + s;
     t.block0 = blocks;
@@ -410,15 +412,14 @@ int edge_plan(gprm_batch* b, const EdgeSignature& sg, const std::vector<int>& ma
   std::vector<int> budget(S), cap(S, 0);
   for (int s = 0; s < S; ++s)
     budget[s] = std::max(1, std::min(kEdgeStepItems, 0x7fffffff / std::max(1, b->ctx[s]->img.M)));
-  struct Part { int s, e0, e1, lo, hi, cap; };
+  struct Part { int s, e0, e1, l0, l1, cap; };
   std::vector<std::vector<Part>> steps;
   for (const auto& w : edge_windows(gmax)) {
     std::vector<int> per(S, 0), nch(S, 0);
     int nsteps = 0;
     for (int s = 0; s < S; ++s) {
-      if (sg.n[s] == 0 || maxT[s] <= w.first) continue;
-      const int width = std::min(w.second, maxT[s]) - w.first;
-      per[s] = std::max(1, budget[s] / width);
+      if (sg.n[s] == 0 || edge_levels(maxT[s]) <= w.first) continue;
+      per[s] = std::max(1, (budget[s] - 64) / (edge_run_slots(edge_window_most(maxT[s], w.first, w.second)) + 1));
       nch[s] = (sg.n[s] + per[s] - 1) / per[s];
       nsteps = std::max(nsteps, nch[s]);
     }
@@ -426,9 +427,9 @@ int edge_plan(gprm_batch* b, const EdgeSignature& sg, const std::vector<int>& ma
       std::vector<Part> parts;
       for (int s = 0; s < S; ++s) {
         if (j >= nch[s]) continue;
-        const int width = std::min(w.second, maxT[s]) - w.first;
         const int e0 = j * per[s], e1 = std::min(sg.n[s], e0 + per[s]);
-        const long long c = frame_stride((long long)(e1 - e0) * width);
+        const long long c = frame_stride(
+            edge_items_cap(e1 - e0, edge_window_most(maxT[s], w.first, w.second), kCompactBlockMulti));
         parts.push_back({s, e0, e1, w.first, w.second, (int)c});
         cap[s] = std::max(cap[s], (int)c);
       }
@@ -439,6 +440,9 @@ int edge_plan(gprm_batch* b, const EdgeSignature& sg, const std::vector<int>& ma
   // step), control words per task
   std::vector<long long> ibase(S + 1, 0);
   for (int s = 0; s < S; ++s) ibase[s + 1] = ibase[s] + cap[s];
+  std::vector<size_t> mbase(S + 1, 0);  // mask words before each scene's
+  for (int s = 0; s < S; ++s) mbase[s + 1] = mbase[s] + mask_words(b->ctx[s]->img.M) * (size_t)(cap[s] / 64);
+  BHIP(b, b->e_masks.ensure(sizeof(unsigned long long) * std::max<size_t>(mbase[S], 1)), "hipMalloc pair masks");
   int ntasks = 0;
   for (const auto& st : steps) ntasks += (int)st.size();
   BHIP(b, b->e_items.ensure(sizeof(int) * 2 * (size_t)std::max(1LL, ibase[S])), "hipMalloc items");
@@ -477,16 +481,18 @@ int edge_plan(gprm_batch* b, const EdgeSignature& sg, const std::vector<int>& ma
       t.dq = c->dq;
       t.e0 = pt.e0;
       t.e1 = pt.e1;
-      t.lo = pt.lo;
-      t.hi = pt.hi;
+      t.l0 = pt.l0;
+      t.l1 = pt.l1;
       t.item_edge = items + ibase[s];
       t.item_pos = items + icap + ibase[s];
       t.nitems = ctl;
       t.cap = pt.cap;
       t.frames = b->e_frames.as<float>() + (size_t)12 * nd * ibase[s];
+      t.img = c->img;
+      t.mask = scene_masks(b, s) ? b->e_masks.as<unsigned long long>() + mbase[s] : nullptr;
       t.block0 = cb;
       t.fblock0 = fb;
-      cb += (pt.e1 - pt.e0 + 255) / 256;
+      cb += (pt.e1 - pt.e0 + kCompactBlockMulti - 1) / kCompactBlockMulti;
       fb += (pt.cap + kFkBlock - 1) / kFkBlock;
       step->tasks.push_back(t);
       step->scene.push_back(s);
@@ -496,6 +502,7 @@ int edge_plan(gprm_batch* b, const EdgeSignature& sg, const std::vector<int>& ma
       q.a.ndof = nd;
       q.a.frames = t.frames;
       q.a.fstride = pt.cap;
+      q.a.mask = t.mask;
       q.a.hist = b->hist.as<float4>();
       q.a.nitems = -1;
       q.a.nitems_dev = ctl;
@@ -538,7 +545,7 @@ int edge_enqueue(gprm_batch* b) {
   for (const auto& step : b->e_steps) {
     const int nt = (int)step->tasks.size();
     BHIP(b, launch_edge_compact_multi(step->d_tasks.as<EdgeTask>(), nt, step->cblocks, st), "compaction launch");
-    BHIP(b, launch_edge_fk_multi(step->d_tasks.as<EdgeTask>(), nt, step->fblocks, b->ndof, st),
+    BHIP(b, launch_edge_fk_multi(step->d_tasks.as<EdgeTask>(), nt, step->fblocks, b->ndof, b->cull_lds, st),
          "kinematics launch");
     for (int i = 0; i < kBuckets; ++i) {
       if (step->nsva[i] == 0) continue;
@@ -651,6 +658,8 @@ int gprm_batch_create(gprm_ctx* const* ctxs, int nscenes, gprm_batch** out) {
   }
   for (int s = 0; s < nscenes; ++s) {
     const int nv = ctxs[s]->img.sumn;
+    if (scene_masks(b, s))
+      b->cull_lds = std::max(b->cull_lds, cull_lds_bytes(ctxs[s]->img.nworld, ctxs[s]->img.nmov, kFkBlock));
     for (auto& bk : b->buckets)
       if (nv >= bk.lo && nv < bk.hi) {
         bk.scenes.push_back(s);

@@ -16,11 +16,10 @@
 
 namespace gprm {
 
-// Order-position windows of the edge rounds for a largest testnum maxT:
-// [0, 12), then widths growing fourfold, or one window [0, maxT) when
-// pair_tests (a bound on the call's pair tests, -1 if unknown) is small
-// (defined in gprm_api.cpp).
-std::vector<std::pair<int, int>> edge_windows(int maxT, long long pair_tests = -1);
+// Level windows [l0, l1) of the edge rounds for a largest testnum maxT: one
+// per level, or a single one when pair_tests (the call's, or a bound on
+// them, -1 if unknown) is at most one_round (defined in gprm_api.cpp).
+std::vector<std::pair<int, int>> edge_windows(int maxT, long long pair_tests = -1, long long one_round = 0);
 
 struct DevBuf {
   void* p = nullptr;
@@ -59,10 +58,9 @@ struct Slot {
   hipStream_t prep = nullptr;
   hipEvent_t ev_first = nullptr;
   std::vector<hipEvent_t> ev_fk, ev_sva;
-  DevBuf frames, status, item_edge, item_pos, counters, qs, qe, res, testnum, stride, misc, tally, hist;
+  DevBuf frames, status, item_edge, item_pos, mask, counters, qs, qe, res, testnum, misc, tally, hist;
   DevBuf groups;  // point calls: completed units per group of 64 items
-  DevBuf frames_odd, item_edge_odd, item_pos_odd;  // buffer set of the odd edge launches
-  int maxT_hint = 0;  // largest testnum of the slot's earlier edge calls (sizes buffers ahead)
+  DevBuf frames_odd, item_edge_odd, item_pos_odd, mask_odd;  // buffer set of the odd edge launches
   int* small_out = nullptr;  // pinned codes of small point-check calls (kSmallMax ints)
   int* host_res = nullptr;
   int N = 0;

@@ -33,23 +33,6 @@ namespace {
 // benchmark 2^24 runs each window in one launch and measured 5.38 against
 // 5.47 ms per step for 2^23.
 constexpr int kItemBudget = 1 << 24;
-// Sample positions in the first edge round; each later round is kWindowGrowth
-// times wider.  The golden-ratio order spreads the first positions along the
-// edge, so blocked edges are mostly found in the first round.  On the 6-DOF
-// edge benchmark, with doubling windows, a first window of 2/4/8/16/32/64/128
-// gave 6.80/6.70/6.53/6.37-6.42/6.45/6.57/6.72 ms per step; later, (first
-// window, growth) of (16, 2)/(16, 3)/(16, 4)/(16, 5)/(8, 3)/(12, 3)/(24, 3)/
-// (32, 3)/(24, 4) gave 5.76/5.56-5.61/5.61-5.62/5.61/5.77/5.90/5.62/5.69/
-// 5.82 ms.  Once a short remainder joined the last window and the frame
-// planes were 1 KB-aligned, (16, 3)/(16, 4)/(16, 5)/(16, 6)/(8, 4)/(12, 4)/
-// (20, 4)/(24, 3)/(32, 3) gave 5.31/5.20/5.27/5.28/5.45/5.26-5.29/5.28/
-// 5.27-5.29/5.29 ms.  Once the later rounds' kinematics overlapped the
-// previous round, (12, 4)/(16, 4)/(10, 4)/(8, 4)/(16, 3)/(12, 3)/(8, 3)/
-// (16, 5)/(24, 4) gave 4.84-4.88/4.91-4.92/4.93-4.94/5.11/4.89/5.09-5.11/
-// 5.09-5.10/4.93-4.95/5.01 ms: windows [0,12), [12,60), [60,209) for its
-// longest edges.
-constexpr int kFirstWindow = 12;
-constexpr int kWindowGrowth = 4;
 // A call whose whole plan is known (the planner's, bounded by D / dq) and
 // holds at most this many pair tests (edges x largest testnum x pairs) runs
 // as one round.  Each round costs a launch whose end waits for its longest
@@ -59,31 +42,22 @@ constexpr int kWindowGrowth = 4;
 // 2^32 pair tests: config1 at 32 nodes per step 226 / 162 / 163 / 162 ms,
 // 7-DOF 153 / 151 / 140 / 140 ms, 6-DOF at 1,024 nodes 8.1 / 5.7-5.8 /
 // 5.6 / 5.8 ms, with an edge budget at 4,096 nodes 5.7 / 5.8 / 5.1 / 4.9 ms.
-constexpr long long kOneRoundPairTests = 1LL << 32;
+constexpr long long kOneRoundPlanned = 1LL << 32;
+// The same for calls of any edges (samples x pairs), whose largest testnum is
+// at most kOneRoundSamples: those may be mostly blocked, and a single round
+// tests all of a blocked edge's samples.
+constexpr long long kOneRoundAny = 1LL << 28;
+constexpr int kOneRoundSamples = 256;
 
 thread_local std::string g_create_error;
 
 }  // namespace
 
-// Sample-window rounds: positions [0,w0), then widths growing kWindowGrowth-fold;
-// one window when pair_tests (a bound on the call's, or -1) is small.
-std::vector<std::pair<int, int>> edge_windows(int maxT, long long pair_tests) {
+std::vector<std::pair<int, int>> edge_windows(int maxT, long long pair_tests, long long one_round) {
   std::vector<std::pair<int, int>> w;
-  if (pair_tests >= 0 && pair_tests <= kOneRoundPairTests && maxT > 0) {
-    w.push_back({0, maxT});
-    return w;
-  }
-  int lo = 0, width = kFirstWindow;
-  while (lo < maxT) {
-    int hi = (int)std::min<long long>((long long)lo + width, maxT);
-    // A remainder under a quarter of this window joins it: a round of its
-    // own costs about 50 us (four launches and their gaps) however few
-    // samples it holds.
-    if ((long long)maxT - hi < width / 4) hi = maxT;
-    w.push_back({lo, hi});
-    lo = hi;
-    if (width < (1 << 20)) width *= kWindowGrowth;
-  }
+  if (maxT <= 0) return w;
+  const int n = pair_tests >= 0 && pair_tests <= one_round ? 1 : edge_levels(maxT);
+  for (int l = 0; l < n; ++l) w.push_back({l, l + 1 == n ? kLevelAll : l + 1});
   return w;
 }
 
@@ -220,6 +194,8 @@ int build_image(gprm_ctx* c, std::vector<char>* out) {
   off = (off + 63) & ~(size_t)63;
   img.off_polyrecs = (long long)off; off += sizeof(PolyRec) * (size_t)N;
   img.off_pairrecs = (long long)off; off = align16(off + 8 * (size_t)M);
+  img.off_cull = (long long)off; off += 32 * (size_t)N;
+  img.off_cpairs = (long long)off; off = align16(off + 4 * (size_t)M);
   out->assign(off, 0);
   char* b = out->data();
   for (int k = 0; k < N; ++k) {
@@ -289,6 +265,22 @@ int build_image(gprm_ctx* c, std::vector<char>* out) {
     std::memcpy(&hull[1], &cert, 4);
     std::memcpy(b + img.off_hulls + 8 * (size_t)k, hull, 8);
   }
+  // the polytopes at rest, then the moving ones by link, for the pair masks
+  std::vector<int> cull_idx(N);
+  img.nworld = img.nmov = 0;
+  for (int l = 0; l <= s.ndof; ++l) {
+    img.mov_off[l] = img.nmov;
+    for (int k = 0; k < N; ++k) {
+      if (s.sys[k] != l) continue;
+      const int idx = l == 0 ? img.nworld++ : img.nworld + img.nmov++;
+      cull_idx[k] = idx;
+      PolyRec rec;
+      std::memcpy(&rec, b + (size_t)img.off_polyrecs + sizeof(rec) * (size_t)k, sizeof(rec));
+      const float e[8] = {rec.c[0], rec.c[1], rec.c[2], rec.rb, rec.v[0], rec.v[1], rec.v[2], 0.0f};
+      std::memcpy(b + (size_t)img.off_cull + 32 * (size_t)idx, e, 32);
+    }
+  }
+  for (int l = s.ndof + 1; l < kMaxDofDev + 2; ++l) img.mov_off[l] = img.nmov;
   std::vector<int> order(M);
   for (int i = 0; i < M; ++i) order[i] = i;
   std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
@@ -356,6 +348,8 @@ int build_image(gprm_ctx* c, std::vector<char>* out) {
     std::memcpy(b + img.off_pairs + 16 * (size_t)j, pr, 16);
     const int rec[2] = {pr[3], i};
     std::memcpy(b + (size_t)img.off_pairrecs + 8 * (size_t)j, rec, 8);
+    const int cp = cull_idx[s.from[i]] | (cull_idx[s.to[i]] << 16);
+    std::memcpy(b + (size_t)img.off_cpairs + 4 * (size_t)j, &cp, 4);
   }
   return GPRM_OK;
 }
@@ -484,6 +478,34 @@ int item_budget(const gprm_ctx* c) {
   return std::max(1, std::min(kItemBudget, 0x7fffffff / std::max(1, upi)));
 }
 
+// Edge launches of at least this many pair tests (item capacity x pairs) have
+// pair masks.  Below, the launch is bound by its longest full tests, not by
+// the bound tests that masks save, and writing them costs a few
+// microseconds: with / without, edges of up to 0.5 rad on the 7-DOF scene
+// (239 pairs) 128: 156 / 160, 2,048: 376 / 362, 8,192: 468 / 460, 20,011: 650 /
+// 805 us; of up to 1 rad on the 6-DOF scene (106 pairs) 8,192: 484 / 462,
+// 20,011: 745 / 767 us, on the 4-DOF scene (35 pairs) 20,011: 568 / 552 us; the
+// 6-DOF roadmap 2.55 / 3.41 ms.
+constexpr long long kMaskPairTests = 1LL << 27;
+bool use_masks(const gprm_ctx* c, long long cap) {
+  return cap * c->img.M >= kMaskPairTests && cull_fits(c->img, 256);
+}
+// Pair masks of n items (whole groups of 64).
+size_t mask_bytes(const gprm_ctx* c, long long n) {
+  return sizeof(unsigned long long) * (size_t)mask_words(c->img.M) * (size_t)((n + 63) / 64);
+}
+
+// One launch of an edge call: levels [l0, l1) of edges [e0, e1), at most cap
+// items (a multiple of 64, also the frames' plane stride).
+struct EdgeLaunch {
+  int e0, e1, l0, l1, cap;
+};
+
+// The launches of a window over N edges of at most maxT samples, total in
+// all (-1: unknown), each of at most item_budget items unless a single edge
+// has more.
+void plan_window(const gprm_ctx* c, int N, int l0, int l1, int maxT, long long total, std::vector<EdgeLaunch>* plan);
+
 // Point checks of n items on the device (q SoA with offset, res[n]).
 int run_points(gprm_ctx* c, Slot& sl, const float* d_q, long long offset, int n, int* d_res,
                hipStream_t st, const unsigned char* skip = nullptr) {
@@ -531,16 +553,34 @@ int run_points(gprm_ctx* c, Slot& sl, const float* d_q, long long offset, int n,
 }
 
 
-// Edge checks on the device.  testnum/stride/res are computed by the
-// prologue kernel; maxT (host-known or read back) sizes the rounds.
+void plan_window(const gprm_ctx* c, int N, int l0, int l1, int maxT, long long total, std::vector<EdgeLaunch>* plan) {
+  const int most = edge_window_most(maxT, l0, l1);
+  const long long budget = item_budget(c);
+  long long cap = edge_items_cap(N, most, kCompactBlock);
+  if (total >= 0)  // every run padded by at most 15
+    cap = std::min(cap, total + 15LL * N + 16LL * ((N + kCompactBlock - 1) / kCompactBlock));
+  if (cap <= budget) {
+    plan->push_back({0, N, l0, l1, (int)frame_stride(cap)});
+    return;
+  }
+  const int per = (int)std::max(1LL, (budget - 64) / (edge_run_slots(most) + 1));
+  for (int e0 = 0; e0 < N; e0 += per) {
+    const int e1 = std::min(N, e0 + per);
+    plan->push_back({e0, e1, l0, l1, (int)frame_stride(edge_items_cap(e1 - e0, most, kCompactBlock))});
+  }
+}
+
+// Edge checks on the device.  testnum and res are computed by the prologue
+// kernel; the largest testnum and the samples in all (host_maxT, host_total,
+// or read back if host_maxT < 0) size the rounds.  one_round: pair tests up
+// to which a known plan is a single round.
 int run_edges(gprm_ctx* c, Slot& sl, const float* d_qs, const float* d_qe, long long offset, int N,
-              int* d_res, hipStream_t st, int host_maxT, gprm_edge_stats* stats, int maxT_hint = 0,
-              const unsigned char* skip = nullptr) {
+              int* d_res, hipStream_t st, int host_maxT, long long host_total, long long one_round,
+              gprm_edge_stats* stats, const unsigned char* skip = nullptr) {
   if (stats) std::memset(stats, 0, sizeof(*stats));
   if (N <= 0) return GPRM_OK;
   const int nd = c->scene.ndof;
   GPRM_HIP(sl.testnum.ensure(sizeof(int) * (size_t)N), "hipMalloc testnum");
-  GPRM_HIP(sl.stride.ensure(sizeof(int) * (size_t)N), "hipMalloc stride");
   GPRM_HIP(sl.misc.ensure(64), "hipMalloc misc");
   int* d_max = reinterpret_cast<int*>(sl.misc.as<char>() + kMiscMaxT);
   unsigned long long* d_total = reinterpret_cast<unsigned long long*>(sl.misc.as<char>() + kMiscTotal);
@@ -548,13 +588,8 @@ int run_edges(gprm_ctx* c, Slot& sl, const float* d_qs, const float* d_qe, long 
   EdgeArgs ea{};
   ea.qs = d_qs; ea.qe = d_qe; ea.offset = offset; ea.nedges = N;
   ea.skip = skip;
-  ea.testnum = sl.testnum.as<int>(); ea.stride = sl.stride.as<int>(); ea.edge_res = d_res;
-  GPRM_HIP(launch_edge_prologue(c->rb, c->dq, ea, sl.testnum.as<int>(), sl.stride.as<int>(), d_max, d_total, st),
-           "edge prologue launch");
-  // The first window [0, kFirstWindow) needs no largest testnum (edges with
-  // fewer samples emit fewer items), so it is enqueued at once; the largest
-  // testnum, which sizes the later windows, is read back on the side stream
-  // meanwhile.
+  ea.testnum = sl.testnum.as<int>(); ea.edge_res = d_res;
+  GPRM_HIP(launch_edge_prologue(c->rb, c->dq, ea, sl.testnum.as<int>(), d_max, d_total, st), "edge prologue launch");
   const bool need_max = host_maxT < 0 || stats;
   if (need_max) {
     if (!sl.side) GPRM_HIP(hipStreamCreateWithFlags(&sl.side, hipStreamNonBlocking), "hipStreamCreate");
@@ -562,15 +597,8 @@ int run_edges(gprm_ctx* c, Slot& sl, const float* d_qs, const float* d_qe, long 
     if (!sl.pinned) GPRM_HIP(hipHostMalloc(&sl.pinned, 32, hipHostMallocDefault), "hipHostMalloc");
     GPRM_HIP(hipEventRecord(sl.ev_prologue, st), "event");
   }
-  // launches: edges [e0, e1) x order positions [lo, hi), at most item_budget
-  // items each
-  struct Launch { int e0, e1, lo, hi; };
-  std::vector<Launch> plan;
-  std::vector<int> early;  // item counts of launches whose counters were replaced
-  auto add_window = [&](int lo, int hi) {
-    const int per = std::max(1, item_budget(c) / (hi - lo));
-    for (int e0 = 0; e0 < N; e0 += per) plan.push_back({e0, std::min(N, e0 + per), lo, hi});
-  };
+  std::vector<EdgeLaunch> plan;
+  std::vector<int> early;  // counters of launches whose buffer was replaced
   // Launch i uses buffer set i & 1.  Launch 0 runs on the call's stream;
   // launches i >= 1 compact and compute frames on the prep stream (after
   // launch 0's kinematics, and once launch i - 2's separating-vector kernel
@@ -583,34 +611,27 @@ int run_edges(gprm_ctx* c, Slot& sl, const float* d_qs, const float* d_qe, long 
   auto set_frames = [&](size_t i) -> DevBuf& { return (i & 1) ? sl.frames_odd : sl.frames; };
   auto set_edge = [&](size_t i) -> DevBuf& { return (i & 1) ? sl.item_edge_odd : sl.item_edge; };
   auto set_pos = [&](size_t i) -> DevBuf& { return (i & 1) ? sl.item_pos_odd : sl.item_pos; };
-  // Launches expected after the first window when the largest testnum is not
-  // known yet (from the slot's earlier calls or the caller's bound): they only
-  // size the buffer sets, so that the later enqueue does not have to grow
-  // buffers that launches in flight still use.
-  std::vector<Launch> expected;
+  auto set_mask = [&](size_t i) -> DevBuf& { return (i & 1) ? sl.mask_odd : sl.mask; };
+  constexpr int kCnt = 4;  // counters per launch: item slots, work counter, samples, unused
   auto enqueue = [&](size_t from) -> int {
     int cap[2] = {0, 0};
-    auto size_launch = [&](size_t i, const Launch& p) {
-      cap[i & 1] = std::max(cap[i & 1], (int)frame_stride((long long)(p.e1 - p.e0) * (p.hi - p.lo)));
-    };
-    for (size_t i = from; i < plan.size(); ++i) size_launch(i, plan[i]);
-    for (size_t j = 0; j < expected.size(); ++j) size_launch(plan.size() + j, expected[j]);
-    size_t fbytes[2], ibytes[2];
+    for (size_t i = from; i < plan.size(); ++i) cap[i & 1] = std::max(cap[i & 1], plan[i].cap);
+    size_t fbytes[2], ibytes[2], mbytes[2];
     for (int k = 0; k < 2; ++k) {
       fbytes[k] = sizeof(float) * 12 * nd * (size_t)std::max(cap[k], 1);
       ibytes[k] = sizeof(int) * (size_t)std::max(cap[k], 1);
+      mbytes[k] = use_masks(c, cap[k]) ? mask_bytes(c, cap[k]) : 0;
     }
-    // per launch: [0] item count, [1] work counter
-    const size_t cbytes = sizeof(int) * 2 * std::max<size_t>(plan.size() + expected.size(), 32);
-    expected.clear();
+    const size_t cbytes = sizeof(int) * kCnt * std::max<size_t>(plan.size(), 32);
     bool grow = cbytes > sl.counters.bytes;
     for (int k = 0; k < 2; ++k)
-      grow = grow || (cap[k] > 0 && (fbytes[k] > set_frames(k).bytes || ibytes[k] > set_edge(k).bytes));
+      grow = grow || (cap[k] > 0 && (fbytes[k] > set_frames(k).bytes || ibytes[k] > set_edge(k).bytes ||
+                                     mbytes[k] > set_mask(k).bytes));
     if (from > 0 && grow) {
       // earlier launches still use the buffers to be replaced; their item
       // counts are kept on the host
       GPRM_HIP(hipStreamSynchronize(st), "sync");
-      early.resize(2 * from);
+      early.resize(kCnt * from);
       GPRM_HIP(hipMemcpy(early.data(), sl.counters.p, sizeof(int) * early.size(), hipMemcpyDeviceToHost), "copy");
     }
     for (int k = 0; k < 2; ++k) {
@@ -618,6 +639,7 @@ int run_edges(gprm_ctx* c, Slot& sl, const float* d_qs, const float* d_qe, long 
       GPRM_HIP(set_frames(k).ensure(fbytes[k]), "hipMalloc frames");
       GPRM_HIP(set_edge(k).ensure(ibytes[k]), "hipMalloc items");
       GPRM_HIP(set_pos(k).ensure(ibytes[k]), "hipMalloc items");
+      GPRM_HIP(set_mask(k).ensure(mbytes[k]), "hipMalloc pair masks");
     }
     GPRM_HIP(sl.counters.ensure(cbytes), "hipMalloc counters");
     GPRM_HIP(sl.hist.ensure(sizeof(float) * 4 * kMaxIter * (size_t)c->shape.grid * c->shape.block),
@@ -633,17 +655,17 @@ int run_edges(gprm_ctx* c, Slot& sl, const float* d_qs, const float* d_qe, long 
     if (!sl.ev_first) GPRM_HIP(hipEventCreateWithFlags(&sl.ev_first, hipEventDisableTiming), "hipEventCreate");
     bool prep_started = false;
     for (size_t i = from; i < plan.size(); ++i) {
-      const Launch& p = plan[i];
-      int* cnt = sl.counters.as<int>() + 2 * i;
+      const EdgeLaunch& p = plan[i];
+      int* cnt = sl.counters.as<int>() + kCnt * i;
       hipStream_t ps = st;
       if (i == 0) {
-        GPRM_HIP(launch_fill_u32(sl.counters.as<unsigned>(), 0u, 2, st), "fill");
+        GPRM_HIP(launch_fill_u32(sl.counters.as<unsigned>(), 0u, kCnt, st), "fill");
       } else {
         ps = sl.prep;
         if (!prep_started) {
           prep_started = true;
           GPRM_HIP(hipStreamWaitEvent(ps, sl.ev_first, 0), "stream wait");
-          GPRM_HIP(launch_fill_u32(sl.counters.as<unsigned>() + 2 * i, 0u, 2 * (long long)(plan.size() - i), ps),
+          GPRM_HIP(launch_fill_u32(sl.counters.as<unsigned>() + kCnt * i, 0u, kCnt * (long long)(plan.size() - i), ps),
                    "fill");
         }
         if (i >= 2) GPRM_HIP(hipStreamWaitEvent(ps, sl.ev_sva[i - 2], 0), "stream wait");
@@ -651,13 +673,13 @@ int run_edges(gprm_ctx* c, Slot& sl, const float* d_qs, const float* d_qe, long 
       int* items_e = set_edge(i).as<int>();
       int* items_p = set_pos(i).as<int>();
       float* frames = set_frames(i).as<float>();
-      GPRM_HIP(launch_edge_compact(ea, p.e0, p.e1, p.lo, p.hi, items_e, items_p, cnt, ps),
+      unsigned long long* mask = use_masks(c, p.cap) ? set_mask(i).as<unsigned long long>() : nullptr;
+      GPRM_HIP(launch_edge_compact(ea, p.e0, p.e1, p.l0, p.l1, items_e, items_p, p.cap, cnt, cnt + 2, ps),
                "edge compaction launch");
-      // item capacity and frame plane stride
-      const int pcap = (int)frame_stride((long long)(p.e1 - p.e0) * (p.hi - p.lo));
       size_t ev = 0;
       GPRM_HIP(prof_begin(c, sl, 1, ps, &ev), "event");
-      GPRM_HIP(launch_edge_fk(c->rb, ea, items_e, items_p, cnt, pcap, frames, ps), "edge kinematics launch");
+      GPRM_HIP(launch_edge_fk(c->rb, ea, items_e, items_p, cnt, p.cap, frames, c->img, mask, ps),
+               "edge kinematics launch");
       GPRM_HIP(prof_end(c, sl, ev, ps), "event");
       if (i == 0) {
         GPRM_HIP(hipEventRecord(sl.ev_first, st), "event");
@@ -669,19 +691,20 @@ int run_edges(gprm_ctx* c, Slot& sl, const float* d_qs, const float* d_qe, long 
       a.img = c->img;
       a.ndof = nd;
       a.frames = frames;
-      a.fstride = pcap;
+      a.fstride = p.cap;
       a.hist = sl.hist.as<float4>();
       a.nitems = -1;
       a.nitems_dev = cnt;
+      a.mask = mask;
       a.counter = reinterpret_cast<unsigned*>(cnt + 1);
       a.item_edge = items_e;
       a.edge_res = d_res;
-      a.pairs_per_unit = unit_pairs(c, pcap);
+      a.pairs_per_unit = unit_pairs(c, p.cap);
       a.units_per_item = (c->img.M + a.pairs_per_unit - 1) / a.pairs_per_unit;
       a.tally = tally_ptr(c, sl);
       a.static_first = 1;
       GPRM_HIP(prof_begin(c, sl, 0, st, &ev), "event");
-      GPRM_HIP(launch_sva(a, 1, launch_shape(c, (long long)((pcap + 63) / 64) * a.units_per_item), st),
+      GPRM_HIP(launch_sva(a, 1, launch_shape(c, (long long)((p.cap + 63) / 64) * a.units_per_item), st),
                "separating-vector launch");
       GPRM_HIP(prof_end(c, sl, ev, st), "event");
       GPRM_HIP(hipEventRecord(sl.ev_sva[i], st), "event");
@@ -690,45 +713,44 @@ int run_edges(gprm_ctx* c, Slot& sl, const float* d_qs, const float* d_qe, long 
   };
   int rc = GPRM_OK;
   int maxT = host_maxT;
+  long long total = host_total;
+  const long long M = c->img.M;
+  // The first window [0, 1) needs no largest testnum, so in a call that
+  // surely takes several rounds it is enqueued at once, and the largest
+  // testnum is read back on the side stream meanwhile.
+  const bool ahead = host_maxT < 0 && 16LL * N * M > kOneRoundAny;
   if (host_maxT >= 0) {
-    // the whole plan is known: one enqueue sizes and launches it
-    for (const auto& w : edge_windows(host_maxT, (long long)N * host_maxT * c->img.M)) add_window(w.first, w.second);
-  } else {
-    add_window(0, kFirstWindow);
-    const int hint = std::max(sl.maxT_hint, maxT_hint);
-    std::swap(plan, expected);
-    for (const auto& w : edge_windows(hint))
-      if (w.first >= kFirstWindow) add_window(w.first, w.second);
-    std::swap(plan, expected);
+    for (const auto& w : edge_windows(host_maxT, (total >= 0 ? total : (long long)N * host_maxT) * M, one_round))
+      plan_window(c, N, w.first, w.second, host_maxT, total, &plan);
+  } else if (ahead) {
+    plan_window(c, N, 0, 1, 16, -1, &plan);
   }
   if ((rc = enqueue(0)) != GPRM_OK) return rc;
-  unsigned long long total = 0;
   if (need_max) {
-    // issued after the first round so that the device gets that round's
-    // launches first
     GPRM_HIP(hipStreamWaitEvent(sl.side, sl.ev_prologue, 0), "stream wait");
     GPRM_HIP(hipMemcpyAsync(sl.pinned, sl.misc.p, kMiscReadback, hipMemcpyDeviceToHost, sl.side), "copy max");
     GPRM_HIP(hipStreamSynchronize(sl.side), "sync");
+    unsigned long long t = 0;
     std::memcpy(&maxT, static_cast<char*>(sl.pinned) + kMiscMaxT, 4);
-    std::memcpy(&total, static_cast<char*>(sl.pinned) + kMiscTotal, 8);
+    std::memcpy(&t, static_cast<char*>(sl.pinned) + kMiscTotal, 8);
+    total = (long long)t;
   }
-  sl.maxT_hint = std::max(sl.maxT_hint, maxT);
   if (host_maxT < 0) {
     const size_t first = plan.size();
-    for (const auto& w : edge_windows(maxT))
-      if (w.first >= kFirstWindow) add_window(w.first, w.second);
+    for (const auto& w : edge_windows(maxT, ahead || maxT > kOneRoundSamples ? -1 : total * M, one_round))
+      if (!ahead || w.first > 0) plan_window(c, N, w.first, w.second, maxT, total, &plan);
     if ((rc = enqueue(first)) != GPRM_OK) return rc;
   }
   if (stats) {
-    std::vector<int> h(2 * plan.size());
+    std::vector<int> h(kCnt * plan.size());
     if (!plan.empty()) {
       GPRM_HIP(hipMemcpyAsync(h.data(), sl.counters.p, sizeof(int) * h.size(), hipMemcpyDeviceToHost, st), "copy");
       GPRM_HIP(hipStreamSynchronize(st), "sync");
     }
     for (size_t i = 0; i < early.size(); ++i) h[i] = early[i];
     long long sched = 0;
-    for (size_t i = 0; i < plan.size(); ++i) sched += h[2 * i];
-    stats->samples_total = (long long)total;
+    for (size_t i = 0; i < plan.size(); ++i) sched += h[kCnt * i + 2];
+    stats->samples_total = total;
     stats->samples_scheduled = sched;
     stats->max_testnum = maxT;
     stats->rounds = (int)plan.size();
@@ -788,7 +810,7 @@ int enqueue_points(gprm_ctx* c, Slot& sl, const float* d_q, long long offset, in
 }
 int enqueue_edges(gprm_ctx* c, Slot& sl, const float* d_qs, const float* d_qe, long long offset, int N, int* d_res,
                   hipStream_t st, int maxT_bound, const unsigned char* skip) {
-  return run_edges(c, sl, d_qs, d_qe, offset, N, d_res, st, maxT_bound, nullptr, 0, skip);
+  return run_edges(c, sl, d_qs, d_qe, offset, N, d_res, st, maxT_bound, -1, kOneRoundPlanned, nullptr, skip);
 }
 
 // Grow the slot's buffers for point checks of n items and edge checks of N
@@ -809,28 +831,25 @@ int reserve_slot(gprm_ctx* c, Slot& sl, int n_points, int N, int maxT_bound) {
     need.push_back({&sl.groups, sizeof(int) * (size_t)((chunk + 63) / 64)});
   }
   if (N > 0) {
-    // the launches of run_edges's plan: windows split into edge ranges,
-    // buffer set i & 1 for launch i
+    // the launches of run_edges's plan, buffer set i & 1 for launch i
+    std::vector<EdgeLaunch> plan;
+    for (const auto& w : edge_windows(maxT_bound, (long long)N * maxT_bound * c->img.M, kOneRoundPlanned))
+      plan_window(c, N, w.first, w.second, maxT_bound, -1, &plan);
     long long cap[2] = {0, 0};
-    size_t launches = 0;
-    for (const auto& w : edge_windows(maxT_bound, (long long)N * maxT_bound * c->img.M)) {
-      const int per = std::max(1, item_budget(c) / (w.second - w.first));
-      for (int e0 = 0; e0 < N; e0 += per, ++launches)
-        cap[launches & 1] = std::max(cap[launches & 1],
-                                     frame_stride((long long)(std::min(N, e0 + per) - e0) * (w.second - w.first)));
-    }
+    for (size_t i = 0; i < plan.size(); ++i) cap[i & 1] = std::max<long long>(cap[i & 1], plan[i].cap);
     DevBuf* fr[2] = {&sl.frames, &sl.frames_odd};
     DevBuf* ie[2] = {&sl.item_edge, &sl.item_edge_odd};
     DevBuf* ip[2] = {&sl.item_pos, &sl.item_pos_odd};
+    DevBuf* mk[2] = {&sl.mask, &sl.mask_odd};
     for (int k = 0; k < 2; ++k) {
       if (cap[k] == 0) continue;
       need.push_back({fr[k], sizeof(float) * 12 * nd * (size_t)cap[k]});
       need.push_back({ie[k], sizeof(int) * (size_t)cap[k]});
       need.push_back({ip[k], sizeof(int) * (size_t)cap[k]});
+      if (use_masks(c, cap[k])) need.push_back({mk[k], mask_bytes(c, cap[k])});
     }
-    need.push_back({&sl.counters, sizeof(int) * 2 * std::max<size_t>(launches, 32)});
+    need.push_back({&sl.counters, sizeof(int) * 4 * std::max<size_t>(plan.size(), 32)});
     need.push_back({&sl.testnum, sizeof(int) * (size_t)N});
-    need.push_back({&sl.stride, sizeof(int) * (size_t)N});
     need.push_back({&sl.misc, 64});
   }
   bool grow = false;
@@ -1033,7 +1052,9 @@ int gprm_indicator2_async(gprm_ctx* c, const float* qs, const float* qe, int* re
     if (!rc) rc = upload_soa(c, sl.qs, qs, N, offset, st);
     if (!rc) rc = upload_soa(c, sl.qe, qe, N, offset, st);
     if (!rc && sl.res.ensure(sizeof(int) * (size_t)N) != hipSuccess) rc = fail(c, GPRM_E_HIP, "hipMalloc res");
-    if (!rc) rc = run_edges(c, sl, sl.qs.as<float>(), sl.qe.as<float>(), N, N, sl.res.as<int>(), st, maxT, nullptr);
+    if (!rc)
+      rc = run_edges(c, sl, sl.qs.as<float>(), sl.qe.as<float>(), N, N, sl.res.as<int>(), st, maxT, total,
+                     kOneRoundPlanned, nullptr);
     if (rc) {
       sl.busy = false;
       return rc;
@@ -1084,7 +1105,7 @@ int gprm_indicator2_dev(gprm_ctx* c, const float* d_qs, const float* d_qe, int* 
   hipStream_t st = stream ? (hipStream_t)stream : sl.stream;
   gprm_edge_stats local;
   if ((rc = prof_prepare(c, sl, st))) return rc;
-  if ((rc = run_edges(c, sl, d_qs, d_qe, offset, N, d_res, st, -1, &local))) return rc;
+  if ((rc = run_edges(c, sl, d_qs, d_qe, offset, N, d_res, st, -1, -1, kOneRoundAny, &local))) return rc;
   GPRM_HIP(hipStreamSynchronize(st), "sync");
   c->numthreads_all += local.samples_total;
   if (stats) *stats = local;

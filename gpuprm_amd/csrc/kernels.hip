@@ -137,9 +137,10 @@ __device__ __forceinline__ T12 t_base(const DevRobot& rb) {
   return T;
 }
 
-template <int NDOF>
+// each(i, T): called with every link frame i (1..ndof) as it is formed.
+template <int NDOF, class F>
 __device__ __forceinline__ void fk_store(const DevRobot& rb, const float* q, float* __restrict__ out, int item,
-                                         long long stride) {
+                                         long long stride, F each) {
   const int nd = NDOF > 0 ? NDOF : rb.ndof;
   T12 T = t_base(rb);
 #pragma unroll
@@ -156,6 +157,7 @@ __device__ __forceinline__ void fk_store(const DevRobot& rb, const float* q, flo
     o[0] = make_float4(T.m[0], T.m[1], T.m[2], T.m[3]);
     o[stride] = make_float4(T.m[4], T.m[5], T.m[6], T.m[7]);
     o[2 * stride] = make_float4(T.m[8], T.m[9], T.m[10], T.m[11]);
+    each(i + 1, T);
   }
 }
 
@@ -197,6 +199,136 @@ __device__ __forceinline__ float bound_radius(const V3& c, float r) {
   return __builtin_fmaf(r, 1.0f + 0x1p-8f, 0x1p-9f * ((fabsf(c.x) + fabsf(c.y)) + (fabsf(c.z) + r)));
 }
 
+// ---- pair masks ------------------------------------------------------------
+// Which pairs does a group of 64 items (a wave) have to test at all?  For
+// most pairs the bound test of the separating-vector kernel passes with room
+// to spare on every item of the group, above all where the items are adjacent
+// samples of an edge, whose links hardly move: on the 6-DOF roadmap's 64
+// consecutive samples about 9 of 10 pairs.  The kinematics kernel, which has
+// the frames in registers, decides those pairs for the whole group:
+//   - per row of 16 lanes and moving polytope, the centre c and the start
+//     vertex v at the row's middle item, and the largest distances mc, mv of
+//     the other items' from them (row reductions);
+//   - then lane l takes pair l, l + 64, ...: with D0 = vQ - vP, E0 = cQ - cP
+//     of the middle items, every item's D and E lie within mv = mvP + mvQ and
+//     mc = mcP + mcQ of them, so
+//       D.E - (rP + rQ)|D| >= D0.E0 - mv|E0| - mc|D0| - mv mc - R (|D0| + mv),
+//     R the radii with the bound test's margins.  Where that is positive (and
+//     |D0| - mv > 1e-4) on all four rows, the bound test's sphere comparison
+//     would pass for every item, and the pair is left out of the group's mask.
+// It costs a wave about 700 instructions per group where the bound tests it
+// saves are about 100 pairs of 30 to 55 each on that scene.
+// With the windows of adjacent samples: the 6-DOF roadmap's edges 3.16 ->
+// 2.51 ms, 20,011 local 7-DOF edges 782 -> 650 us.
+struct CullTab {
+  f32x4* ab;  // entry e: ab[2 e] = (centre, mc), ab[2 e + 1] = (start vertex, mv)
+  float* r;   // entry e: R
+  int nworld, nmov;
+  int wave0;  // this wave's first entry: row k's moving polytope m at wave0 + k nmov + m
+};
+
+__device__ __forceinline__ const __attribute__((address_space(4))) f32x4* cull_polys(const SceneImg& img) {
+  return (const __attribute__((address_space(4))) f32x4*)(reinterpret_cast<unsigned long long>(img.blob) +
+                                                          (unsigned long long)img.off_cull);
+}
+
+// Tables of a block in its dynamic LDS, the polytopes at rest filled in.
+// Every thread of the block calls it.
+__device__ __forceinline__ CullTab cull_stage(const SceneImg& img, int4* lds) {
+  CullTab t;
+  const int entries = img.nworld + (int)(blockDim.x >> 6) * 4 * img.nmov;
+  t.ab = reinterpret_cast<f32x4*>(lds);
+  t.r = reinterpret_cast<float*>(t.ab + 2 * entries);
+  t.nworld = img.nworld;
+  t.nmov = img.nmov;
+  t.wave0 = img.nworld + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * 4 * img.nmov;
+  const GAS f32x4* src = (const GAS f32x4*)(reinterpret_cast<const char*>(img.blob) + img.off_cull);
+  for (int i = threadIdx.x; i < img.nworld; i += blockDim.x) {
+    f32x4 c = src[2 * i];
+    t.r[i] = c.w;
+    c.w = 0.0f;
+    t.ab[2 * i] = c;
+    t.ab[2 * i + 1] = src[2 * i + 1];
+  }
+  __syncthreads();
+  return t;
+}
+
+// x of the row's lane 8 (DPP row_newbcast), in all 16 lanes of the row.
+__device__ __forceinline__ float row_middle(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x150 + 8, 0xf, 0xf, false));
+}
+// The largest x of the row (x >= 0), in all its lanes (DPP row_ror).
+__device__ __forceinline__ float row_max(float x) {
+  x = fmaxf(x, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x128, 0xf, 0xf, false)));
+  x = fmaxf(x, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x124, 0xf, 0xf, false)));
+  x = fmaxf(x, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x122, 0xf, 0xf, false)));
+  x = fmaxf(x, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x121, 0xf, 0xf, false)));
+  return x;
+}
+// How far the row's items lie from its middle one, at most: a NaN counts as
+// infinitely far; enlarged against the rounding of the positions (2^-16 of
+// their magnitude) and of the distance itself.
+__device__ __forceinline__ float row_reach(const V3& x, const V3& x0, float mag) {
+  const V3 d{x.x - x0.x, x.y - x0.y, x.z - x0.z};
+  float d2 = b_dot(d, d);
+  d2 = d2 < __builtin_inff() ? d2 : __builtin_inff();
+  return __builtin_fmaf(__builtin_amdgcn_sqrtf(row_max(d2)), 1.0f + 0x1p-10f, 0x1p-16f * mag);
+}
+
+// The rows' entries of link l's polytopes; every lane of the wave has a valid
+// item's frame T of that link.
+__device__ __forceinline__ void cull_link(const SceneImg& img, const CullTab& t, int l, const T12& T) {
+  const int lane = threadIdx.x & 63;
+  for (int m = img.mov_off[l]; m < img.mov_off[l + 1]; ++m) {
+    const f32x4 c4 = cull_polys(img)[2 * (img.nworld + m)], v4 = cull_polys(img)[2 * (img.nworld + m) + 1];
+    const V3 c = b_apply(T, v3(c4)), v = b_apply(T, v3(v4));
+    const V3 c0{row_middle(c.x), row_middle(c.y), row_middle(c.z)};
+    const V3 v0{row_middle(v.x), row_middle(v.y), row_middle(v.z)};
+    const float mag = (fabsf(c0.x) + fabsf(c0.y)) + (fabsf(c0.z) + c4.w);
+    const float mc = row_reach(c, c0, mag), mv = row_reach(v, v0, mag);
+    if ((lane & 15) == 0) {
+      const int e = t.wave0 + (lane >> 4) * t.nmov + m;
+      t.ab[2 * e] = f32x4{c0.x, c0.y, c0.z, mc};
+      t.ab[2 * e + 1] = f32x4{v0.x, v0.y, v0.z, mv};
+      t.r[e] = __builtin_fmaf(c4.w, 1.0f + 0x1p-8f, 0x1p-9f * (mag + 2.0f * mc));
+    }
+  }
+}
+
+// The group's mask words, after cull_link of every link.
+__device__ __forceinline__ void cull_pairs(const SceneImg& img, const CullTab& t, unsigned long long* __restrict__ mask,
+                                           int group) {
+  const int lane = threadIdx.x & 63;
+  // the entries were written by other lanes of this wave
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  const GAS int* cpairs = (const GAS int*)(reinterpret_cast<const char*>(img.blob) + img.off_cpairs);
+  const int nw = (img.M + 63) >> 6;
+  for (int w = 0; w < nw; ++w) {
+    const int pair = 64 * w + lane;
+    const int cp = cpairs[pair < img.M ? pair : 0];
+    const int p = cp & 0xffff, q = (int)((unsigned)cp >> 16);
+    const int pe = p < t.nworld ? p : t.wave0 + (p - t.nworld), ps = p < t.nworld ? 0 : t.nmov;
+    const int qe = q < t.nworld ? q : t.wave0 + (q - t.nworld), qs = q < t.nworld ? 0 : t.nmov;
+    bool far = true;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int ip = pe + k * ps, iq = qe + k * qs;
+      const f32x4 pc = t.ab[2 * ip], pv = t.ab[2 * ip + 1], qc = t.ab[2 * iq], qv = t.ab[2 * iq + 1];
+      const V3 E{qc.x - pc.x, qc.y - pc.y, qc.z - pc.z}, D{qv.x - pv.x, qv.y - pv.y, qv.z - pv.z};
+      const float mc = qc.w + pc.w, mv = qv.w + pv.w, R = t.r[ip] + t.r[iq];
+      const float ne = __builtin_amdgcn_sqrtf(b_dot(E, E)), nd = __builtin_amdgcn_sqrtf(b_dot(D, D));
+      float lhs = b_dot(D, E);
+      lhs = __builtin_fmaf(-mv, ne, lhs);
+      lhs = __builtin_fmaf(-mc, nd + mv, lhs);
+      far = far & (lhs > R * (nd + mv)) & (nd - mv > 1e-4f);
+    }
+    const unsigned long long m = __ballot((pair < img.M) & !far);
+    if (lane == 0) mask[(size_t)group * nw + w] = m;
+  }
+}
+
 // ----------------------------------------------------------------------------
 // kinematics kernels
 // ----------------------------------------------------------------------------
@@ -234,7 +366,7 @@ __global__ void __launch_bounds__(kFkBlock)
   } else {
     word[i] = kWordFree;
   }
-  fk_store<NDOF>(rb, qq, frames, i, fstride);
+  fk_store<NDOF>(rb, qq, frames, i, fstride, [](int, const T12&) {});
 }
 
 // The frames of n configurations as Kinematics<ndof>::calculate leaves its
@@ -263,18 +395,17 @@ __global__ void finalize_points_kernel(const int* __restrict__ word, int* __rest
   codes[i] = w == kWordFree ? 0 : (w & 15) - 1;
 }
 
-// Frames of item i of an edge round: sample (pos * stride) mod T of its
+// Frames of item i of an edge round to slot `slot`: sample item_pos[i] of its
 // edge, interpolated as robotconfigspace.cpp:406-420 does (c1 = s/(T-1),
 // c2 = 1 - c1, q = c1 qs + c2 qe), then the kinematics.
-template <int NDOF>
+template <int NDOF, class F>
 __device__ __forceinline__ void fk_edge_item(const DevRobot& rb, const EdgeArgs& ea, const int* __restrict__ item_edge,
-                                             const int* __restrict__ item_pos, int i, float* __restrict__ frames,
-                                             long long fstride) {
+                                             const int* __restrict__ item_pos, int i, int slot,
+                                             float* __restrict__ frames, long long fstride, F each) {
   const int nd = NDOF > 0 ? NDOF : rb.ndof;
-  const int e = item_edge[i];
-  const int pos = item_pos[i];
+  const int e = item_edge[i] & ~kItemPad;
+  const int s = item_pos[i];
   const int T = ea.testnum[e];
-  const int s = (int)(((long long)pos * ea.stride[e]) % T);
   float c1, c2;
   if (T > 0) {
     c1 = (float)s / (float)(T - 1);
@@ -287,42 +418,54 @@ __device__ __forceinline__ void fk_edge_item(const DevRobot& rb, const EdgeArgs&
 #pragma unroll
   for (int j = 0; j < (NDOF > 0 ? NDOF : kMaxDofDev); ++j)
     if (NDOF > 0 || j < nd) qq[j] = c1 * ea.qs[e + ea.offset * j] + c2 * ea.qe[e + ea.offset * j];
-  fk_store<NDOF>(rb, qq, frames, i, fstride);
+  fk_store<NDOF>(rb, qq, frames, slot, fstride, each);
 }
 
-// q of the sample at order position pos of edge e (robotconfigspace.cpp:409-420).
+// Kinematics (and pair masks) of items [0, n), the grid striding over them
+// in whole groups of 64; the last group's lanes past the end take the last
+// item (in bounds: the planes hold whole groups), so that the wave's
+// reductions see valid items only.
+template <int NDOF>
+__device__ __forceinline__ void fk_edge_items(const DevRobot& rb, const EdgeArgs& ea, const int* __restrict__ item_edge,
+                                              const int* __restrict__ item_pos, int n, int first, int step,
+                                              float* __restrict__ frames, long long fstride, const SceneImg& img,
+                                              unsigned long long* __restrict__ mask, int4* smem) {
+  CullTab tab{};
+  if (mask != nullptr) tab = cull_stage(img, smem);
+  for (int slot = first; (slot & ~63) < n; slot += step) {
+    const int i = slot < n ? slot : n - 1;
+    if (mask == nullptr) {
+      fk_edge_item<NDOF>(rb, ea, item_edge, item_pos, i, slot, frames, fstride, [](int, const T12&) {});
+    } else {
+      fk_edge_item<NDOF>(rb, ea, item_edge, item_pos, i, slot, frames, fstride,
+                         [&](int l, const T12& T) { cull_link(img, tab, l, T); });
+      cull_pairs(img, tab, mask, slot >> 6);
+    }
+  }
+}
+
 template <int NDOF>
 __global__ void __launch_bounds__(kFkBlock)
     fk_edges_kernel(DevRobot rb, EdgeArgs ea, const int* __restrict__ item_edge,
                     const int* __restrict__ item_pos, const int* __restrict__ nitems_dev, int cap,
-                    float* __restrict__ frames, long long fstride) {
+                    float* __restrict__ frames, long long fstride, SceneImg img,
+                    unsigned long long* __restrict__ mask) {
+  extern __shared__ int4 smem[];
   int n = *nitems_dev;
   if (n > cap) n = cap;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-    fk_edge_item<NDOF>(rb, ea, item_edge, item_pos, i, frames, fstride);
+  fk_edge_items<NDOF>(rb, ea, item_edge, item_pos, n, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x,
+                      frames, fstride, img, mask, smem);
 }
 
-__device__ int gcd_i(int a, int b) {
-  while (b) {
-    int t = a % b;
-    a = b;
-    b = t;
-  }
-  return a;
-}
-
-// testnum (robotconfigspace.cpp:660-673) and the sample order stride: a
-// golden-ratio step coprime with testnum, so that positions 0,1,2,... visit
-// every sample once, spread along the edge.
+// testnum (robotconfigspace.cpp:660-673).
 template <int BLOCK>
 __device__ __forceinline__ void edge_prologue_one(int ndof, float dq, const EdgeArgs& ea, int k,
-                                                  int* __restrict__ testnum, int* __restrict__ stride,
+                                                  int* __restrict__ testnum,
                                                   int* __restrict__ max_testnum,
                                                   unsigned long long* __restrict__ total) {
   int T = 0;
   if (k < ea.nedges && ea.skip != nullptr && ea.skip[k]) {
     testnum[k] = 0;
-    stride[k] = 1;
     ea.edge_res[k] = kEdgeSkipped;
   } else if (k < ea.nedges) {
     float norm = 0.0f;
@@ -332,14 +475,7 @@ __device__ __forceinline__ void edge_prologue_one(int ndof, float dq, const Edge
     }
     norm = __builtin_sqrtf(norm);
     T = (int)(norm / dq) + 1;
-    int g = 1;
-    if (T > 2) {
-      g = (int)((double)T * 0.6180339887498949);
-      if (g < 1) g = 1;
-      while (gcd_i(g, T) != 1) ++g;
-    }
     testnum[k] = T;
-    stride[k] = g;
     ea.edge_res[k] = 0;
   }
   // One atomic pair per block: same-address atomics from all CUs serialise
@@ -372,69 +508,99 @@ __device__ __forceinline__ void edge_prologue_one(int ndof, float dq, const Edge
 }
 
 __global__ void __launch_bounds__(1024)
-    edge_prologue_kernel(int ndof, float dq, EdgeArgs ea, int* __restrict__ testnum,
-                         int* __restrict__ stride, int* __restrict__ max_testnum,
+    edge_prologue_kernel(int ndof, float dq, EdgeArgs ea, int* __restrict__ testnum, int* __restrict__ max_testnum,
                          unsigned long long* __restrict__ total) {
-  edge_prologue_one<1024>(ndof, dq, ea, blockIdx.x * 1024 + threadIdx.x, testnum, stride, max_testnum, total);
+  edge_prologue_one<1024>(ndof, dq, ea, blockIdx.x * 1024 + threadIdx.x, testnum, max_testnum, total);
 }
 
-// Items for order positions [lo, hi) of every open edge in [e0, e1).
+// Items for levels [l0, l1) of every open edge in [e0, e1), an edge's samples
+// in ascending order on consecutive slots.  Runs of more than kRunShort
+// samples start at a multiple of 16 and are padded to one (edge_run_slots);
+// the block's short runs follow them packed, padded together.  Padding items
+// repeat a sample, so that the rows' pair masks see valid items only, and are
+// marked (kItemPad): the separating-vector kernel leaves them out.
 // One atomic per block reserves the block's slots (same-address atomics
 // serialise at the memory side; one per wave took 23 us for 100k edges);
 // each lane's slots follow by prefix count.  Every thread of the block calls
 // it; threads with e >= e1 contribute nothing.
 template <int BLOCK>
-__device__ __forceinline__ void edge_compact_one(const EdgeArgs& ea, int e, int e1, int lo, int hi,
-                                                 int* __restrict__ item_edge, int* __restrict__ item_pos,
-                                                 int* __restrict__ nitems) {
-  int cnt = 0;
-  if (e < e1) {
-    int T = ea.testnum[e];
-    int open = __hip_atomic_load(&ea.edge_res[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0;
-    if (open && T > lo) cnt = (T < hi ? T : hi) - lo;
-  }
-  // wave-inclusive prefix sum of cnt
+__device__ __forceinline__ void edge_compact_one(const EdgeArgs& ea, int e, int e1, int l0, int l1,
+                                                 int* __restrict__ item_edge, int* __restrict__ item_pos, int cap,
+                                                 int* __restrict__ nitems, int* __restrict__ nsamples) {
+  int a = 1, b = 0, cnt = 0;
+  if (e < e1 && __hip_atomic_load(&ea.edge_res[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
+    edge_window(ea.testnum[e], l0, l1, &a, &b, &cnt);
+  const bool is_short = cnt <= kRunShort;
+  // prefix sums of the long runs' slots, the short runs' and the samples
+  int lng = is_short ? 0 : edge_run_slots(cnt), shr = is_short ? cnt : 0, smp = cnt;
+  const int slots = lng;
   const int lane = threadIdx.x & 63;
-  int incl = cnt;
   for (int d = 1; d < 64; d <<= 1) {
-    int v = __shfl_up(incl, d, 64);
-    if (lane >= d) incl += v;
+    const int u = __shfl_up(lng, d, 64), v = __shfl_up(shr, d, 64), x = __shfl_up(smp, d, 64);
+    if (lane >= d) {
+      lng += u;
+      shr += v;
+      smp += x;
+    }
   }
-  __shared__ int s_wave[BLOCK / 64];
-  __shared__ int s_base;
+  __shared__ int s_long[BLOCK / 64], s_short[BLOCK / 64], s_smp[BLOCK / 64];
+  __shared__ int s_base, s_short0, s_shorts;
   const int w = threadIdx.x >> 6;
-  if (lane == 63) s_wave[w] = incl;
+  if (lane == 63) {
+    s_long[w] = lng;
+    s_short[w] = shr;
+    s_smp[w] = smp;
+  }
   __syncthreads();
   if (threadIdx.x == 0) {
-    int sum = 0;
+    int sl = 0, ss = 0, sn = 0;
     for (int i = 0; i < BLOCK / 64; ++i) {
-      const int v = s_wave[i];
-      s_wave[i] = sum;
-      sum += v;
+      const int u = s_long[i], v = s_short[i];
+      s_long[i] = sl;
+      s_short[i] = ss;
+      sl += u;
+      ss += v;
+      sn += s_smp[i];
     }
-    s_base = sum > 0 ? atomicAdd(nitems, sum) : 0;
+    const int total = sl + (ss + 15) / 16 * 16;
+    s_base = total > 0 ? atomicAdd(nitems, total) : 0;
+    s_short0 = sl;
+    s_shorts = ss;
+    if (nsamples != nullptr && sn > 0) atomicAdd(nsamples, sn);
   }
   __syncthreads();
-  // The wave's runs are consecutive: lane l's items start at the wave's base
-  // + its exclusive prefix.  They are written run by run with all 64 lanes,
-  // so every store instruction covers consecutive slots.
-  const int o = s_base + s_wave[w] + incl - cnt;
+  // first slot of the lane's run, and the end of its padding: the block's
+  // last short run pads for all of them
+  const int o = s_base + (is_short ? s_short0 + s_short[w] + shr - cnt : s_long[w] + lng - slots);
+  int fill = is_short ? cnt : slots;
+  if (is_short && cnt > 0 && s_short[w] + shr == s_shorts) fill += (s_shorts + 15) / 16 * 16 - s_shorts;
+  // Four runs at a time, one to each row of 16 lanes, so that every store
+  // instruction covers four spans of consecutive slots.
   unsigned long long runs = __ballot(cnt > 0);
+  const int row = lane >> 4, col = lane & 15;
   while (runs) {
-    const int src = __builtin_ctzll(runs);
-    runs &= runs - 1;
-    const int c = __shfl(cnt, src, 64), os = __shfl(o, src, 64), es = __shfl(e, src, 64);
-    for (int t = lane; t < c; t += 64) {
-      item_edge[os + t] = es;
-      item_pos[os + t] = lo + t;
+    int src = -1;
+    for (int k = 0; k < 4 && runs; ++k) {
+      const int t = __builtin_ctzll(runs);
+      runs &= runs - 1;
+      if (k == row) src = t;
+    }
+    const int from = src < 0 ? 0 : src;
+    const int c = __shfl(cnt, from, 64), f = __shfl(fill, from, 64), os = __shfl(o, from, 64), es = __shfl(e, from, 64);
+    const int as = __shfl(a, from, 64), bs = __shfl(b, from, 64);
+    if (src < 0) continue;
+    for (int t = col; t < f && os + t < cap; t += 16) {
+      item_edge[os + t] = t < c ? es : es | kItemPad;
+      item_pos[os + t] = edge_window_sample(as, bs, t < c ? t : c - 1);
     }
   }
 }
 
-__global__ void __launch_bounds__(1024)
-    edge_compact_kernel(EdgeArgs ea, int e0, int e1, int lo, int hi, int* __restrict__ item_edge,
-                        int* __restrict__ item_pos, int* __restrict__ nitems) {
-  edge_compact_one<1024>(ea, e0 + blockIdx.x * 1024 + threadIdx.x, e1, lo, hi, item_edge, item_pos, nitems);
+__global__ void __launch_bounds__(kCompactBlock)
+    edge_compact_kernel(EdgeArgs ea, int e0, int e1, int l0, int l1, int* __restrict__ item_edge,
+                        int* __restrict__ item_pos, int cap, int* __restrict__ nitems, int* __restrict__ nsamples) {
+  edge_compact_one<kCompactBlock>(ea, e0 + blockIdx.x * kCompactBlock + threadIdx.x, e1, l0, l1, item_edge, item_pos,
+                                  cap, nitems, nsamples);
 }
 
 // Multi-scene edge calls: one task per scene (prologue) or per scene part of
@@ -455,23 +621,26 @@ __device__ __forceinline__ const EdgeTask& edge_task_of(const EdgeTask* __restri
 
 __global__ void __launch_bounds__(256) edge_prologue_multi_kernel(const EdgeTask* __restrict__ tasks, int ntasks) {
   const EdgeTask& T = edge_task_of<false>(tasks, ntasks);
-  edge_prologue_one<256>(T.rb.ndof, T.dq, T.ea, (blockIdx.x - T.block0) * 256 + threadIdx.x, T.testnum, T.stride,
-                    T.max_testnum, T.total);
+  edge_prologue_one<256>(T.rb.ndof, T.dq, T.ea, (blockIdx.x - T.block0) * 256 + threadIdx.x, T.testnum,
+                         T.max_testnum, T.total);
 }
 
-__global__ void __launch_bounds__(256) edge_compact_multi_kernel(const EdgeTask* __restrict__ tasks, int ntasks) {
+__global__ void __launch_bounds__(kCompactBlockMulti)
+    edge_compact_multi_kernel(const EdgeTask* __restrict__ tasks, int ntasks) {
   const EdgeTask& T = edge_task_of<false>(tasks, ntasks);
-  edge_compact_one<256>(T.ea, T.e0 + (blockIdx.x - T.block0) * 256 + threadIdx.x, T.e1, T.lo, T.hi, T.item_edge,
-                        T.item_pos, T.nitems);
+  edge_compact_one<kCompactBlockMulti>(T.ea, T.e0 + (blockIdx.x - T.block0) * kCompactBlockMulti + threadIdx.x, T.e1,
+                                       T.l0, T.l1, T.item_edge, T.item_pos, T.cap, T.nitems, nullptr);
 }
 
 template <int NDOF>
 __global__ void __launch_bounds__(kFkBlock) fk_edges_multi_kernel(const EdgeTask* __restrict__ tasks, int ntasks) {
+  extern __shared__ int4 smem[];
   const EdgeTask& T = edge_task_of<true>(tasks, ntasks);
-  const int i = (blockIdx.x - T.fblock0) * kFkBlock + threadIdx.x;
   int n = *T.nitems;
   if (n > T.cap) n = T.cap;
-  if (i < n) fk_edge_item<NDOF>(T.rb, T.ea, T.item_edge, T.item_pos, i, T.frames, (long long)T.cap);
+  // one pass: the task's blocks cover its capacity
+  fk_edge_items<NDOF>(T.rb, T.ea, T.item_edge, T.item_pos, n, (blockIdx.x - T.fblock0) * kFkBlock + threadIdx.x,
+                      0x40000000, T.frames, (long long)T.cap, T.img, T.mask, smem);
 }
 
 // ---- cell index for the radius search -------------------------------------
@@ -1018,7 +1187,8 @@ __device__ __forceinline__ void sva_units(const SvaArgs& A, const Lds& L, const 
   // the same in every lane, as are the unit indices derived from it: said by
   // readfirstlane, so that the pair loop and the records stay scalar also
   // where the arguments were loaded from memory
-  const int nitems = __builtin_amdgcn_readfirstlane(A.nitems >= 0 ? A.nitems : *A.nitems_dev);
+  const int nitems =
+      __builtin_amdgcn_readfirstlane(A.nitems >= 0 ? A.nitems : (int)min((long long)*A.nitems_dev, A.fstride));
   const int M = A.img.M;
   const int PC = A.pairs_per_unit;
   const unsigned ngroups = (unsigned)((nitems + 63) >> 6);
@@ -1118,16 +1288,19 @@ __device__ __forceinline__ void sva_units(const SvaArgs& A, const Lds& L, const 
     ++n_claimed;
     const unsigned ch = u / ngroups;
     const int item = (int)((u - ch * ngroups) << 6) + lane;
-    const bool active = item < nitems;
+    bool active = item < nitems;
     const int p0 = (int)ch * PC, p1 = min(M, p0 + PC);
     // early exit: in edge mode once any sample of the edge is blocked; in
     // point mode for pairs after (in CRS order) a pair known to collide,
     // since the reference returns the first colliding pair's code.
     int edge = 0, gate = 0x7fffffff;
     bool open_item = active;
+    if (EDGE && active) {
+      edge = ((const GAS int*)A.item_edge)[item];
+      active = open_item = edge >= 0;  // no padding
+    }
     if (active) {
       if (EDGE) {
-        edge = ((const GAS int*)A.item_edge)[item];
         open_item = __hip_atomic_load((GAS int*)A.edge_res + edge, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0;
       } else {
         gate = __hip_atomic_load((GAS int*)A.word + item, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> 4;
@@ -1135,15 +1308,39 @@ __device__ __forceinline__ void sva_units(const SvaArgs& A, const Lds& L, const 
     }
     // the lanes whose item is in the launch, and those of them that are open
     const unsigned long long act = __ballot(active), opn = EDGE ? __ballot(open_item) : act;
+    // The chunk's pairs in order: all of them in point mode (random
+    // configurations leave few pairs out of a mask; walking the masks' bits
+    // alone cost 3.55 against 3.33 ms for 4M points of the 7-DOF scene), in
+    // edge mode those that the group's mask leaves; the others are decided by
+    // the bounds for every item (cull_pairs).
+    const unsigned long long mrow =
+        reinterpret_cast<unsigned long long>(A.mask) + 8ull * (u - ch * ngroups) * (unsigned)((M + 63) >> 6);
+    const int wl = (p1 - 1) >> 6;
+    int w = (p0 >> 6) - 1;
+    unsigned long long bits = 0ull;
+    auto next_pair = [&]() {
+      while (bits == 0ull) {
+        if (w >= wl) return -1;
+        ++w;
+        // a scalar load: the masks are constant during the launch
+        bits = A.mask == nullptr ? ~0ull : ((const __attribute__((address_space(4))) unsigned long long*)mrow)[w];
+        if (w == p0 >> 6) bits &= ~0ull << (p0 & 63);
+        if (w == wl) bits &= ~0ull >> (63 - ((p1 - 1) & 63));
+      }
+      const int p = 64 * w + __builtin_ctzll(bits);
+      bits &= bits - 1;
+      return p;
+    };
     // The unit's pairs run in segments that end where the ring is drained.
     // The caches are local to a segment, so nothing of them is live across
     // a drain, which has registers of its own.
-    int pair = p0;
-    if (EDGE && opn == 0ull) {
-      s_dropped += (unsigned)__popcll(act) * (unsigned)(p1 - p0);
-      pair = p1;
+    int left = EDGE ? p1 - p0 : 0;  // pairs not walked
+    int cur_pair = EDGE ? -1 : p0, nxt_pair = EDGE ? -1 : p0 + 1;
+    if (EDGE && opn != 0ull) {
+      cur_pair = next_pair();
+      nxt_pair = next_pair();
     }
-    while (pair < p1) {
+    while (EDGE ? cur_pair >= 0 : cur_pair < p1) {
       // wave-uniform cache: Q's world bounds for polytope ckQ and its start
       // vertex
       int ckQ = -1;
@@ -1158,14 +1355,19 @@ __device__ __forceinline__ void sva_units(const SvaArgs& A, const Lds& L, const 
       // pair; now it is about 30, and 25 more where the boxes are needed
       // (4.28 -> 3.57 ms for 4M configurations of the 7-DOF scene, 3.83 ->
       // 3.26 ms for the 6-DOF roadmap's edges).
-      i32x2 pr1 = load_pairrec(A.img, pair), pr2 = load_pairrec(A.img, min(pair + 1, M - 1));
+      i32x2 pr1 = load_pairrec(A.img, cur_pair), pr2 = load_pairrec(A.img, EDGE ? max(nxt_pair, 0) : min(nxt_pair, M - 1));
       i32x16 poly1 = load_polyrec(A.img, pr1[0] & 0xffff);
-      for (; pair < p1; ++pair) {
+      bool full = false;
+      do {
         const i32x2 pr = pr1;
         const i32x16 cur = poly1;
+        const int pair = cur_pair;
+        if (EDGE) --left;
         pr1 = pr2;
         poly1 = load_polyrec(A.img, pr1[0] & 0xffff);
-        pr2 = load_pairrec(A.img, min(pair + 2, M - 1));
+        cur_pair = nxt_pair;
+        nxt_pair = EDGE ? next_pair() : nxt_pair + 1;
+        pr2 = load_pairrec(A.img, EDGE ? max(nxt_pair, 0) : min(nxt_pair, M - 1));
         const int crs = pr[1], kQ = (int)((unsigned)pr[0] >> 16);
         // Frames are loaded by every lane: an inactive lane's item is below
         // the plane stride (the item count rounded up to 64), and what it
@@ -1272,16 +1474,18 @@ __device__ __forceinline__ void sva_units(const SvaArgs& A, const Lds& L, const 
             if (EDGE) R.edge[slot] = edge;
           }
           d_tail += (unsigned)__popcll(dm);
-          if (d_tail - d_head >= CAP - 64) {
-            ++pair;
-            break;
-          }
+          full = d_tail - d_head >= CAP - 64;
         }
-      }
-      if (d_tail - d_head >= CAP - 64) {
+      } while ((EDGE ? cur_pair >= 0 : cur_pair < p1) && !full);
+      if (full) {
         sva_drain<EDGE, CAP>(A, L, R, H, hs, d_head, d_tail, n_sep, n_col, n_dropped, n_iter);
         if (fuse) complete_pending();  // the units before this one
       }
+    }
+    // the pairs the mask left out: separated where the item is open
+    if (EDGE) {
+      s_bound += (unsigned)left * (unsigned)__popcll(opn);
+      s_dropped += (unsigned)left * (unsigned)__popcll(act & ~opn);
     }
     ++n_units;
     if (fuse) {
@@ -1373,7 +1577,7 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVE
   for (int r = 0; r < ntasks; ++r) {
     const int t = (int)((blockIdx.x + (unsigned)r) % (unsigned)ntasks);
     const SvaArgs A = tasks[t].a;
-    const int ni = A.nitems >= 0 ? A.nitems : *A.nitems_dev;
+    const int ni = A.nitems >= 0 ? A.nitems : (int)min((long long)*A.nitems_dev, A.fstride);
     const unsigned nunits = sva_unit_count(A, ni);
     if (threadIdx.x == 0)
       s_live = __hip_atomic_load(A.counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < nunits ? 1 : 0;
@@ -1515,7 +1719,7 @@ __global__ void __launch_bounds__(kFkBlock) fk_points_multi_kernel(const FkTask*
   for (int j = 0; j < nd; ++j)
     if (qq[j] < T.rb.mins[j] || qq[j] > T.rb.maxs[j]) { st = 1; break; }
   T.word[i] = st ? kWordOutOfBounds : kWordFree;
-  fk_store<NDOF>(T.rb, qq, T.frames, i, T.fstride);
+  fk_store<NDOF>(T.rb, qq, T.frames, i, T.fstride, [](int, const T12&) {});
 }
 
 // codes of every task from its result words (same block map).
@@ -1548,16 +1752,16 @@ size_t sva_lds_bytes(const SceneImg& img, int block, int gscene) {
 
 int sva_max_lds_bytes() { return 160 * 1024; }
 
-#define GPRM_FK_DISPATCH(KERNEL, GRID, BLOCK, ST, ...)                                      \
-  switch (rb.ndof) {                                                                        \
-    case 2: hipLaunchKernelGGL(KERNEL<2>, GRID, BLOCK, 0, ST, __VA_ARGS__); break;         \
-    case 3: hipLaunchKernelGGL(KERNEL<3>, GRID, BLOCK, 0, ST, __VA_ARGS__); break;         \
-    case 4: hipLaunchKernelGGL(KERNEL<4>, GRID, BLOCK, 0, ST, __VA_ARGS__); break;         \
-    case 5: hipLaunchKernelGGL(KERNEL<5>, GRID, BLOCK, 0, ST, __VA_ARGS__); break;         \
-    case 6: hipLaunchKernelGGL(KERNEL<6>, GRID, BLOCK, 0, ST, __VA_ARGS__); break;         \
-    case 7: hipLaunchKernelGGL(KERNEL<7>, GRID, BLOCK, 0, ST, __VA_ARGS__); break;         \
-    case 8: hipLaunchKernelGGL(KERNEL<8>, GRID, BLOCK, 0, ST, __VA_ARGS__); break;         \
-    default: hipLaunchKernelGGL(KERNEL<0>, GRID, BLOCK, 0, ST, __VA_ARGS__); break;        \
+#define GPRM_FK_DISPATCH(KERNEL, GRID, BLOCK, LDS, ST, ...)                                   \
+  switch (rb.ndof) {                                                                          \
+    case 2: hipLaunchKernelGGL(KERNEL<2>, GRID, BLOCK, LDS, ST, __VA_ARGS__); break;         \
+    case 3: hipLaunchKernelGGL(KERNEL<3>, GRID, BLOCK, LDS, ST, __VA_ARGS__); break;         \
+    case 4: hipLaunchKernelGGL(KERNEL<4>, GRID, BLOCK, LDS, ST, __VA_ARGS__); break;         \
+    case 5: hipLaunchKernelGGL(KERNEL<5>, GRID, BLOCK, LDS, ST, __VA_ARGS__); break;         \
+    case 6: hipLaunchKernelGGL(KERNEL<6>, GRID, BLOCK, LDS, ST, __VA_ARGS__); break;         \
+    case 7: hipLaunchKernelGGL(KERNEL<7>, GRID, BLOCK, LDS, ST, __VA_ARGS__); break;         \
+    case 8: hipLaunchKernelGGL(KERNEL<8>, GRID, BLOCK, LDS, ST, __VA_ARGS__); break;         \
+    default: hipLaunchKernelGGL(KERNEL<0>, GRID, BLOCK, LDS, ST, __VA_ARGS__); break;        \
   }
 
 // Threads per kinematics block: kFkBlock when that still gives at least two
@@ -1571,7 +1775,7 @@ hipError_t launch_fk_points(const DevRobot& rb, const float* q, long long offset
   if (n <= 0) return hipSuccess;
   const int fb = fk_block(n);
   dim3 grid((n + fb - 1) / fb), block(fb);
-  GPRM_FK_DISPATCH(fk_points_kernel, grid, block, st, rb, q, offset, n, frames, fstride, word,
+  GPRM_FK_DISPATCH(fk_points_kernel, grid, block, 0, st, rb, q, offset, n, frames, fstride, word,
                    check_bounds, zero_counter, skip, group_done);
   return hipGetLastError();
 }
@@ -1590,14 +1794,18 @@ hipError_t launch_finalize_points(const int* word, int* codes, int n, hipStream_
 }
 
 hipError_t launch_edge_fk(const DevRobot& rb, EdgeArgs ea, const int* item_edge, const int* item_pos,
-                          const int* nitems, int cap, float* frames, hipStream_t st) {
+                          const int* nitems, int cap, float* frames, const SceneImg& img, unsigned long long* mask,
+                          hipStream_t st) {
   if (cap <= 0) return hipSuccess;
-  const int fb = fk_block(cap);
+  int fb = fk_block(cap);
+  if (mask != nullptr && !cull_fits(img, fb)) fb = 256;
+  if (mask != nullptr && !cull_fits(img, fb)) return hipErrorInvalidValue;
+  const size_t lds = mask != nullptr ? cull_lds_bytes(img.nworld, img.nmov, fb) : 0;
   int blocks = (cap + fb - 1) / fb;
   if (blocks > 4096) blocks = 4096;
   dim3 grid(blocks), block(fb);
-  GPRM_FK_DISPATCH(fk_edges_kernel, grid, block, st, rb, ea, item_edge, item_pos, nitems, cap, frames,
-                   (long long)cap);
+  GPRM_FK_DISPATCH(fk_edges_kernel, grid, block, lds, st, rb, ea, item_edge, item_pos, nitems, cap, frames,
+                   (long long)cap, img, mask);
   return hipGetLastError();
 }
 
@@ -1767,21 +1975,21 @@ hipError_t launch_finalize_points_multi(const FkTask* d_tasks, int ntasks, int n
   return hipGetLastError();
 }
 
-hipError_t launch_edge_prologue(const DevRobot& rb, float dq, EdgeArgs ea, int* testnum_out,
-                                int* stride_out, int* max_testnum, unsigned long long* total,
-                                hipStream_t st) {
+hipError_t launch_edge_prologue(const DevRobot& rb, float dq, EdgeArgs ea, int* testnum_out, int* max_testnum,
+                                unsigned long long* total, hipStream_t st) {
   if (ea.nedges <= 0) return hipSuccess;
   dim3 grid((ea.nedges + 1023) / 1024), block(1024);
-  hipLaunchKernelGGL(edge_prologue_kernel, grid, block, 0, st, rb.ndof, dq, ea, testnum_out, stride_out,
+  hipLaunchKernelGGL(edge_prologue_kernel, grid, block, 0, st, rb.ndof, dq, ea, testnum_out,
                      max_testnum, total);
   return hipGetLastError();
 }
 
-hipError_t launch_edge_compact(EdgeArgs ea, int e0, int e1, int lo, int hi, int* item_edge,
-                               int* item_pos, int* nitems, hipStream_t st) {
+hipError_t launch_edge_compact(EdgeArgs ea, int e0, int e1, int l0, int l1, int* item_edge,
+                               int* item_pos, int cap, int* nitems, int* nsamples, hipStream_t st) {
   if (e1 <= e0) return hipSuccess;
-  dim3 grid((e1 - e0 + 1023) / 1024), block(1024);
-  hipLaunchKernelGGL(edge_compact_kernel, grid, block, 0, st, ea, e0, e1, lo, hi, item_edge, item_pos, nitems);
+  dim3 grid((e1 - e0 + kCompactBlock - 1) / kCompactBlock), block(kCompactBlock);
+  hipLaunchKernelGGL(edge_compact_kernel, grid, block, 0, st, ea, e0, e1, l0, l1, item_edge, item_pos, cap,
+                     nitems, nsamples);
   return hipGetLastError();
 }
 
@@ -1793,21 +2001,22 @@ hipError_t launch_edge_prologue_multi(const EdgeTask* d_tasks, int ntasks, int n
 
 hipError_t launch_edge_compact_multi(const EdgeTask* d_tasks, int ntasks, int nblocks, hipStream_t st) {
   if (ntasks <= 0 || nblocks <= 0) return hipSuccess;
-  hipLaunchKernelGGL(edge_compact_multi_kernel, dim3(nblocks), dim3(256), 0, st, d_tasks, ntasks);
+  hipLaunchKernelGGL(edge_compact_multi_kernel, dim3(nblocks), dim3(kCompactBlockMulti), 0, st, d_tasks, ntasks);
   return hipGetLastError();
 }
 
-hipError_t launch_edge_fk_multi(const EdgeTask* d_tasks, int ntasks, int nblocks, int ndof, hipStream_t st) {
+hipError_t launch_edge_fk_multi(const EdgeTask* d_tasks, int ntasks, int nblocks, int ndof, size_t cull_lds,
+                                hipStream_t st) {
   if (ntasks <= 0 || nblocks <= 0) return hipSuccess;
   dim3 grid(nblocks), block(kFkBlock);
   switch (ndof) {
-    case 2: hipLaunchKernelGGL(fk_edges_multi_kernel<2>, grid, block, 0, st, d_tasks, ntasks); break;
-    case 3: hipLaunchKernelGGL(fk_edges_multi_kernel<3>, grid, block, 0, st, d_tasks, ntasks); break;
-    case 4: hipLaunchKernelGGL(fk_edges_multi_kernel<4>, grid, block, 0, st, d_tasks, ntasks); break;
-    case 5: hipLaunchKernelGGL(fk_edges_multi_kernel<5>, grid, block, 0, st, d_tasks, ntasks); break;
-    case 6: hipLaunchKernelGGL(fk_edges_multi_kernel<6>, grid, block, 0, st, d_tasks, ntasks); break;
-    case 7: hipLaunchKernelGGL(fk_edges_multi_kernel<7>, grid, block, 0, st, d_tasks, ntasks); break;
-    default: hipLaunchKernelGGL(fk_edges_multi_kernel<0>, grid, block, 0, st, d_tasks, ntasks); break;
+    case 2: hipLaunchKernelGGL(fk_edges_multi_kernel<2>, grid, block, cull_lds, st, d_tasks, ntasks); break;
+    case 3: hipLaunchKernelGGL(fk_edges_multi_kernel<3>, grid, block, cull_lds, st, d_tasks, ntasks); break;
+    case 4: hipLaunchKernelGGL(fk_edges_multi_kernel<4>, grid, block, cull_lds, st, d_tasks, ntasks); break;
+    case 5: hipLaunchKernelGGL(fk_edges_multi_kernel<5>, grid, block, cull_lds, st, d_tasks, ntasks); break;
+    case 6: hipLaunchKernelGGL(fk_edges_multi_kernel<6>, grid, block, cull_lds, st, d_tasks, ntasks); break;
+    case 7: hipLaunchKernelGGL(fk_edges_multi_kernel<7>, grid, block, cull_lds, st, d_tasks, ntasks); break;
+    default: hipLaunchKernelGGL(fk_edges_multi_kernel<0>, grid, block, cull_lds, st, d_tasks, ntasks); break;
   }
   return hipGetLastError();
 }

@@ -45,13 +45,31 @@ struct DevRobot {
 // scenes of up to about 100 polytopes and 900 pairs:
 //   polyrecs PolyRec[N]    the bound test's operands of each polytope
 //   pairrecs int2[M]       (polytope P | polytope Q << 16, CRS index), in pair order
+//   cull     float4[2 N]   for the pair masks, the polytopes at rest then the
+//                          moving ones by link: (centre, PolyRec::rb), (start vertex, 0)
+//   cpairs   int[M]        P | Q << 16, each an index into `cull`
 struct SceneImg {
   const int4* blob;        // device pointer to the image
   int bytes;               // size of the staged part, multiple of 16
   int off_verts, off_pairs, off_adj, off_hulls;
-  long long off_polyrecs, off_pairrecs;
+  long long off_polyrecs, off_pairrecs, off_cull, off_cpairs;
   int sumn, summ, M, N;
+  int nworld, nmov;               // polytopes at rest and on links
+  int mov_off[kMaxDofDev + 2];    // moving polytopes of link l: [mov_off[l], mov_off[l + 1])
 };
+
+// Words of a pair mask (one bit per pair, in the image's pair order).
+inline int mask_words(int M) { return (M + 63) / 64; }
+// Dynamic LDS of a kinematics block that writes pair masks: 36 bytes per
+// polytope at rest and, per wave, for each of its four rows of 16 items one
+// entry per moving polytope.
+inline size_t cull_lds_bytes(int nworld, int nmov, int block) {
+  return 36 * ((size_t)nworld + (size_t)(block / 64) * 4 * nmov);
+}
+constexpr size_t kCullLds = 40 * 1024;  // at most; scenes beyond have no masks
+inline bool cull_fits(const SceneImg& img, int block) {
+  return cull_lds_bytes(img.nworld, img.nmov, block) <= kCullLds;
+}
 
 // Operands of a polytope in the bound test (64 bytes, one scalar load), in
 // its own frame.
@@ -75,6 +93,10 @@ struct SvaArgs {
   float4* hist;            // [kMaxIter][grid*block] per-lane iteration history
   int nitems;              // item count, or -1: read *nitems_dev
   const int* nitems_dev;
+  // edge mode: the pairs that some item of a group of 64 needs tested,
+  // mask_words(M) words per group (written by the kinematics launch); null:
+  // all of them
+  const unsigned long long* mask;
   unsigned int* counter;   // work counter (zero before launch)
   int pairs_per_unit;      // pairs of one work unit (a wave claims one chunk of them
                            // for 64 consecutive items)
@@ -88,7 +110,7 @@ struct SvaArgs {
   int* group_done;
   int* codes;
   // edge mode
-  const int* item_edge;    // [item] owning edge
+  const int* item_edge;    // [item] owning edge, negative: padding (kItemPad)
   int* edge_res;           // [edge] nonzero once any sample collides
   // optional counters (may be null): kTallySlots slots of kTallyCount, block
   // b adds its sums into slot b mod kTallySlots, spreading the atomics; a
@@ -212,36 +234,102 @@ struct EdgeArgs {
   // kEdgeSkipped; the planner's edge budget)
   const unsigned char* skip;
   const int* testnum;      // [edge]
-  const int* stride;       // [edge] sample order: position j -> (j*stride) mod testnum
   int* edge_res;           // [edge]
 };
 
+// Samples of an edge in launch windows.  The testnum samples of an edge
+// belong to levels: level 0 holds at most 16 evenly spaced ones, each next
+// level fills up a spacing four times finer, the last level the rest:
+// edge_levels(T) levels with spacings m_l, the multiples of m_l that are not
+// multiples of m_(l-1).  A window covers levels [l0, l1) of every edge, in
+// ascending sample order: adjacent items are adjacent samples, whose links
+// stay close together, which is what the pair masks live on; and the first
+// window's spread samples find most blocked edges.  The 6-DOF roadmap
+// (longest edge 209 samples) takes two windows, of 15 and about 105 samples
+// per edge.
+constexpr int kLevelAll = 64;  // l1 of a window that takes every remaining sample
+__host__ __device__ inline int edge_levels(int T) {
+  if (T <= 16) return 1;
+  if (T <= 256) return 2;
+  int n = 3;
+  for (long long lim = 512; T > lim; lim *= 4) ++n;
+  return n;
+}
+// Samples of the window: the multiples of a that are not multiples of b (b =
+// 0: every multiple of a).  count: how many.
+__host__ __device__ inline void edge_window(int T, int l0, int l1, int* a, int* b, int* count) {
+  const int n = edge_levels(T);
+  *a = 1;
+  *b = 0;
+  *count = 0;
+  if (T <= 0 || l0 >= n) return;
+  int fine = 1;  // m_(n-2), and from it the coarser spacings
+  if (n > 1) {
+    const long long cnt = 16LL << (2 * (n - 2));
+    fine = (int)((T + cnt - 1) / cnt);
+  }
+  if (l1 < n) *a = fine << (2 * (n - 1 - l1));
+  if (l0 > 0) *b = fine << (2 * (n - 1 - l0));
+  *count = (int)(((long long)T + *a - 1) / *a) - (*b ? (int)(((long long)T + *b - 1) / *b) : 0);
+}
+// Sample r (ascending) of that window.
+__host__ __device__ inline int edge_window_sample(int a, int b, int r) {
+  if (b == 0) return r * a;
+  const int k = b / a - 1;
+  return a * (r / k * (k + 1) + r % k + 1);
+}
+// Most samples an edge of at most maxT samples has in the window.
+inline int edge_window_most(int maxT, int l0, int l1) {
+  (void)l0;
+  long long lim = l1 == 1 ? 16 : 256;
+  for (int l = 3; l <= l1 && lim < maxT; ++l) lim = l == 3 ? 512 : lim * 4;
+  return (int)(lim < maxT ? lim : maxT);
+}
+// Item slots of an edge with count samples in a window: runs of more than
+// kRunShort samples start at and are padded to multiples of 16 (a row of
+// lanes), so that a row's items are one edge's.
+constexpr int kRunShort = 8;
+__host__ __device__ inline int edge_run_slots(int count) {
+  return count > kRunShort ? (count + 15) / 16 * 16 : count;
+}
+// Item capacity for n edges of at most `most` samples each in blocks of
+// `block` edges (the compaction pads each block's short runs to 16, too).
+inline long long edge_items_cap(long long n, int most, int block) {
+  return n * edge_run_slots(most) + 16 * ((n + block - 1) / block);
+}
+// Padding items carry their edge with this bit.
+constexpr int kItemPad = (int)0x80000000;
+
 // One scene's part of a multi-scene edge call (device memory).  Prologue
-// tasks (one per scene) cover edges [0, ea.nedges) and write testnum,
-// stride, the scene's largest testnum and its sample total; launch-step
-// tasks cover edges [e0, e1) and order positions [lo, hi): the compaction
-// appends their items (item_edge, item_pos, *nitems, at most cap) and the
-// kinematics writes their frames (link-major, item stride cap).
+// tasks (one per scene) cover edges [0, ea.nedges) and write testnum, the
+// scene's largest testnum and its sample total; launch-step tasks cover edges
+// [e0, e1) and levels [l0, l1): the compaction appends their items
+// (item_edge, item_pos = sample, *nitems, at most cap) and the kinematics
+// writes their frames (link-major, item stride cap) and pair masks.
 struct EdgeTask {
   EdgeArgs ea;
   DevRobot rb;
   float dq;
   int* testnum;
-  int* stride;
   int* max_testnum;
   unsigned long long* total;
-  int e0, e1, lo, hi;
+  int e0, e1, l0, l1;
   int* item_edge;
   int* item_pos;
   int* nitems;
   int cap;                      // item capacity, a multiple of 64 (also the frame plane stride)
   float* frames;
+  SceneImg img;
+  unsigned long long* mask;     // pair masks per group of 64 items, or null
   int block0;    // first block of the task in the prologue / compaction grid (tasks sorted)
   int fblock0;   // first block of the task in the kinematics grid (tasks sorted)
 };
 hipError_t launch_edge_prologue_multi(const EdgeTask* d_tasks, int ntasks, int nblocks, hipStream_t st);
 hipError_t launch_edge_compact_multi(const EdgeTask* d_tasks, int ntasks, int nblocks, hipStream_t st);
-hipError_t launch_edge_fk_multi(const EdgeTask* d_tasks, int ntasks, int nblocks, int ndof, hipStream_t st);
+// cull_lds: the largest cull_lds_bytes of the tasks with masks at kFkBlock
+// threads, 0 if none has.
+hipError_t launch_edge_fk_multi(const EdgeTask* d_tasks, int ntasks, int nblocks, int ndof, size_t cull_lds,
+                                hipStream_t st);
 
 // Deferral rings of the separating-vector kernel: per wave, a ring of
 // sva_ring_cap(block) entries of 12 bytes (item, pair, edge).  Larger rings
@@ -276,15 +364,20 @@ hipError_t launch_fk_points_multi(const FkTask* d_tasks, int ntasks, int nblocks
 hipError_t launch_finalize_points_multi(const FkTask* d_tasks, int ntasks, int nblocks, hipStream_t st);
 hipError_t launch_sva_multi(const SceneTask* d_tasks, int ntasks, int edge_mode, const SvaShape& sh, size_t img_bytes,
                             unsigned long long* t_start, unsigned long long* tally, hipStream_t st);
-hipError_t launch_edge_prologue(const DevRobot& rb, float dq, EdgeArgs ea, int* testnum_out,
-                                int* stride_out, int* max_testnum, unsigned long long* total,
-                                hipStream_t st);
-hipError_t launch_edge_compact(EdgeArgs ea, int e0, int e1, int lo, int hi, int* item_edge,
-                               int* item_pos, int* nitems, hipStream_t st);
+hipError_t launch_edge_prologue(const DevRobot& rb, float dq, EdgeArgs ea, int* testnum_out, int* max_testnum,
+                                unsigned long long* total, hipStream_t st);
+// Items of levels [l0, l1) of the open edges in [e0, e1): item_edge, item_pos
+// (the sample), *nitems slots of which *nsamples (may be null) are no padding.
+// Slots beyond cap (an edge longer than the plan's bound) are not written.
+constexpr int kCompactBlock = 1024, kCompactBlockMulti = 256;
+hipError_t launch_edge_compact(EdgeArgs ea, int e0, int e1, int l0, int l1, int* item_edge, int* item_pos,
+                               int cap, int* nitems, int* nsamples, hipStream_t st);
 // Kinematics of the *nitems (<= cap) compacted samples; frames link-major
-// with item stride cap.
+// with item stride cap (the plane stride); their pair masks to mask unless
+// it is null.
 hipError_t launch_edge_fk(const DevRobot& rb, EdgeArgs ea, const int* item_edge, const int* item_pos,
-                          const int* nitems, int cap, float* frames, hipStream_t st);  // cap: plane stride
+                          const int* nitems, int cap, float* frames, const SceneImg& img, unsigned long long* mask,
+                          hipStream_t st);
 // Small point-check calls: up to kSmallMax configurations passed by value,
 // one block each, codes written to out (device-visible, e.g. pinned host
 // memory).  point_small_prepare sets the kernels' LDS limit once per scene.
