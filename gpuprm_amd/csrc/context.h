@@ -58,7 +58,7 @@ struct Slot {
   hipStream_t prep = nullptr;
   hipEvent_t ev_first = nullptr;
   std::vector<hipEvent_t> ev_fk, ev_sva;
-  DevBuf frames, status, item_edge, item_pos, mask, counters, qs, qe, res, testnum, misc, tally, hist;
+  DevBuf frames, status, item_edge, item_pos, mask, counters, queues, qs, qe, res, testnum, misc, tally, hist;
   DevBuf groups;  // point calls: completed units per group of 64 items
   DevBuf frames_odd, item_edge_odd, item_pos_odd, mask_odd;  // buffer set of the odd edge launches
   int* small_out = nullptr;  // pinned codes of small point-check calls (kSmallMax ints)

@@ -516,7 +516,7 @@ int run_points(gprm_ctx* c, Slot& sl, const float* d_q, long long offset, int n,
   GPRM_HIP(sl.status.ensure(sizeof(int) * (size_t)chunk), "hipMalloc words");
   const int nchunks = (n + chunk - 1) / chunk;
   GPRM_HIP(sl.hist.ensure(sizeof(float) * 4 * kMaxIter * (size_t)c->shape.grid * c->shape.block), "hipMalloc history");
-  GPRM_HIP(sl.counters.ensure(sizeof(unsigned) * (size_t)nchunks), "hipMalloc counters");
+  GPRM_HIP(sl.queues.ensure(sizeof(unsigned) * kSvaCounters * (size_t)nchunks), "hipMalloc counters");
   GPRM_HIP(sl.groups.ensure(sizeof(int) * (size_t)((chunk + 63) / 64)), "hipMalloc group counters");
   for (int ci = 0; ci < nchunks; ++ci) {
     int c0 = ci * chunk, cn = std::min(chunk, n - c0);
@@ -524,7 +524,7 @@ int run_points(gprm_ctx* c, Slot& sl, const float* d_q, long long offset, int n,
     GPRM_HIP(prof_begin(c, sl, 1, st, &ev), "event");
     GPRM_HIP(launch_fk_points(c->rb, d_q + c0, offset, cn, sl.frames.as<float>(), frame_stride(cn),
                               sl.status.as<int>(), 1,
-                              sl.counters.as<unsigned>() + ci, st, skip ? skip + c0 : nullptr,
+                              sl.queues.as<unsigned>() + (size_t)kSvaCounters * ci, st, skip ? skip + c0 : nullptr,
                               sl.groups.as<int>()),
              "kinematics launch");
     GPRM_HIP(prof_end(c, sl, ev, st), "event");
@@ -535,7 +535,7 @@ int run_points(gprm_ctx* c, Slot& sl, const float* d_q, long long offset, int n,
     a.fstride = frame_stride(cn);
     a.hist = sl.hist.as<float4>();
     a.nitems = cn;
-    a.counter = sl.counters.as<unsigned>() + ci;
+    a.counter = sl.queues.as<unsigned>() + (size_t)kSvaCounters * ci;
     a.pairs_per_unit = unit_pairs(c, cn);
     a.units_per_item = (c->img.M + a.pairs_per_unit - 1) / a.pairs_per_unit;
     a.word = sl.status.as<int>();
@@ -612,7 +612,7 @@ int run_edges(gprm_ctx* c, Slot& sl, const float* d_qs, const float* d_qe, long 
   auto set_edge = [&](size_t i) -> DevBuf& { return (i & 1) ? sl.item_edge_odd : sl.item_edge; };
   auto set_pos = [&](size_t i) -> DevBuf& { return (i & 1) ? sl.item_pos_odd : sl.item_pos; };
   auto set_mask = [&](size_t i) -> DevBuf& { return (i & 1) ? sl.mask_odd : sl.mask; };
-  constexpr int kCnt = 4;  // counters per launch: item slots, work counter, samples, unused
+  constexpr int kCnt = 2;  // counters per launch: item slots, samples
   auto enqueue = [&](size_t from) -> int {
     int cap[2] = {0, 0};
     for (size_t i = from; i < plan.size(); ++i) cap[i & 1] = std::max(cap[i & 1], plan[i].cap);
@@ -623,7 +623,8 @@ int run_edges(gprm_ctx* c, Slot& sl, const float* d_qs, const float* d_qe, long 
       mbytes[k] = use_masks(c, cap[k]) ? mask_bytes(c, cap[k]) : 0;
     }
     const size_t cbytes = sizeof(int) * kCnt * std::max<size_t>(plan.size(), 32);
-    bool grow = cbytes > sl.counters.bytes;
+    const size_t qbytes = sizeof(unsigned) * kSvaCounters * std::max<size_t>(plan.size(), 4);
+    bool grow = cbytes > sl.counters.bytes || qbytes > sl.queues.bytes;
     for (int k = 0; k < 2; ++k)
       grow = grow || (cap[k] > 0 && (fbytes[k] > set_frames(k).bytes || ibytes[k] > set_edge(k).bytes ||
                                      mbytes[k] > set_mask(k).bytes));
@@ -642,6 +643,7 @@ int run_edges(gprm_ctx* c, Slot& sl, const float* d_qs, const float* d_qe, long 
       GPRM_HIP(set_mask(k).ensure(mbytes[k]), "hipMalloc pair masks");
     }
     GPRM_HIP(sl.counters.ensure(cbytes), "hipMalloc counters");
+    GPRM_HIP(sl.queues.ensure(qbytes), "hipMalloc counters");
     GPRM_HIP(sl.hist.ensure(sizeof(float) * 4 * kMaxIter * (size_t)c->shape.grid * c->shape.block),
              "hipMalloc history");
     if (plan.size() > 1 && !sl.prep) GPRM_HIP(hipStreamCreateWithFlags(&sl.prep, hipStreamNonBlocking), "hipStreamCreate");
@@ -673,8 +675,10 @@ int run_edges(gprm_ctx* c, Slot& sl, const float* d_qs, const float* d_qe, long 
       int* items_e = set_edge(i).as<int>();
       int* items_p = set_pos(i).as<int>();
       float* frames = set_frames(i).as<float>();
+      unsigned* queues = sl.queues.as<unsigned>() + (size_t)kSvaCounters * i;  // zeroed by the compaction
       unsigned long long* mask = use_masks(c, p.cap) ? set_mask(i).as<unsigned long long>() : nullptr;
-      GPRM_HIP(launch_edge_compact(ea, p.e0, p.e1, p.l0, p.l1, items_e, items_p, p.cap, cnt, cnt + 2, ps),
+      GPRM_HIP(launch_edge_compact(ea, p.e0, p.e1, p.l0, p.l1, items_e, items_p, p.cap, cnt, cnt + 1,
+                                   queues, ps),
                "edge compaction launch");
       size_t ev = 0;
       GPRM_HIP(prof_begin(c, sl, 1, ps, &ev), "event");
@@ -696,7 +700,7 @@ int run_edges(gprm_ctx* c, Slot& sl, const float* d_qs, const float* d_qe, long 
       a.nitems = -1;
       a.nitems_dev = cnt;
       a.mask = mask;
-      a.counter = reinterpret_cast<unsigned*>(cnt + 1);
+      a.counter = queues;
       a.item_edge = items_e;
       a.edge_res = d_res;
       a.pairs_per_unit = unit_pairs(c, p.cap);
@@ -749,7 +753,7 @@ int run_edges(gprm_ctx* c, Slot& sl, const float* d_qs, const float* d_qe, long 
     }
     for (size_t i = 0; i < early.size(); ++i) h[i] = early[i];
     long long sched = 0;
-    for (size_t i = 0; i < plan.size(); ++i) sched += h[kCnt * i + 2];
+    for (size_t i = 0; i < plan.size(); ++i) sched += h[kCnt * i + 1];
     stats->samples_total = total;
     stats->samples_scheduled = sched;
     stats->max_testnum = maxT;
@@ -827,7 +831,7 @@ int reserve_slot(gprm_ctx* c, Slot& sl, int n_points, int N, int maxT_bound) {
     const int chunk = std::min(n_points, item_budget(c));
     need.push_back({&sl.frames, sizeof(float) * 12 * nd * (size_t)frame_stride(chunk)});
     need.push_back({&sl.status, sizeof(int) * (size_t)chunk});
-    need.push_back({&sl.counters, sizeof(unsigned) * (size_t)((n_points + chunk - 1) / chunk)});
+    need.push_back({&sl.queues, sizeof(unsigned) * kSvaCounters * (size_t)((n_points + chunk - 1) / chunk)});
     need.push_back({&sl.groups, sizeof(int) * (size_t)((chunk + 63) / 64)});
   }
   if (N > 0) {
@@ -848,7 +852,8 @@ int reserve_slot(gprm_ctx* c, Slot& sl, int n_points, int N, int maxT_bound) {
       need.push_back({ip[k], sizeof(int) * (size_t)cap[k]});
       if (use_masks(c, cap[k])) need.push_back({mk[k], mask_bytes(c, cap[k])});
     }
-    need.push_back({&sl.counters, sizeof(int) * 4 * std::max<size_t>(plan.size(), 32)});
+    need.push_back({&sl.counters, sizeof(int) * 2 * std::max<size_t>(plan.size(), 32)});
+    need.push_back({&sl.queues, sizeof(unsigned) * kSvaCounters * std::max<size_t>(plan.size(), 4)});
     need.push_back({&sl.testnum, sizeof(int) * (size_t)N});
     need.push_back({&sl.misc, 64});
   }

@@ -345,9 +345,9 @@ __global__ void __launch_bounds__(kFkBlock)
                      unsigned* __restrict__ zero_counter, const unsigned char* __restrict__ skip,
                      int* __restrict__ group_done) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
-  // the separating-vector launch that follows claims units from this counter
+  // the separating-vector launch that follows claims units from these counters
   // and counts completed units per group of 64 items in group_done
-  if (i == 0 && zero_counter != nullptr) *zero_counter = 0u;
+  if (zero_counter != nullptr && i < kSvaQueues) zero_counter[i * kSvaQueueStride] = 0u;
   if (group_done != nullptr && (i & 63) == 0 && i < n) group_done[i >> 6] = 0;
   if (i >= n) return;
   const int nd = NDOF > 0 ? NDOF : rb.ndof;
@@ -598,7 +598,9 @@ __device__ __forceinline__ void edge_compact_one(const EdgeArgs& ea, int e, int 
 
 __global__ void __launch_bounds__(kCompactBlock)
     edge_compact_kernel(EdgeArgs ea, int e0, int e1, int l0, int l1, int* __restrict__ item_edge,
-                        int* __restrict__ item_pos, int cap, int* __restrict__ nitems, int* __restrict__ nsamples) {
+                        int* __restrict__ item_pos, int cap, int* __restrict__ nitems, int* __restrict__ nsamples,
+                        unsigned* __restrict__ zero_queues) {
+  if (blockIdx.x == 0 && threadIdx.x < kSvaQueues) zero_queues[threadIdx.x * kSvaQueueStride] = 0u;
   edge_compact_one<kCompactBlock>(ea, e0 + blockIdx.x * kCompactBlock + threadIdx.x, e1, l0, l1, item_edge, item_pos,
                                   cap, nitems, nsamples);
 }
@@ -1053,7 +1055,7 @@ __device__ __forceinline__ unsigned sva_unit_count(const SvaArgs& A, int nitems)
 
 // Phase B of sva_units: every lane takes a deferred pair from the wave's
 // ring and runs the full separating-vector test (collision4.h:227-332) until
-// the ring is empty.  The gate is re-read when a pair is taken.
+// the ring is empty.  The gate is re-read when a pair is taken. 
 template <int EDGE, int CAP>
 __device__ __forceinline__ void sva_drain(const SvaArgs& A, const Lds& L, const Ring& R,
                                           GAS f32x4* H, size_t hs, unsigned& d_head, unsigned d_tail,
@@ -1176,9 +1178,9 @@ __device__ __forceinline__ void sva_drain(const SvaArgs& A, const Lds& L, const 
 //      pairs; a pair it does not decide is appended to the wave's ring;
 //   B. once 64 pairs wait (and at the end), every lane takes deferred pairs
 //      and runs the full test until the ring is empty (sva_drain).
-// H: this lane's iteration history (stride hs); dq: the wave's ring.  Waves
-// run independently: there is no block barrier inside.  cnt.claimed counts
-// the wave's units (the same in every lane).
+// H: this lane's iteration history (stride hs); R: the wave's ring.  Waves
+// run independently: there is no block barrier inside.  cnt.claimed counts the wave's units (the
+// same in every lane).
 template <int EDGE, int CAP>
 __device__ __forceinline__ void sva_units(const SvaArgs& A, const Lds& L, const Ring& R,
                                           GAS f32x4* H, size_t hs, SvaCounts& cnt) {
@@ -1238,27 +1240,39 @@ __device__ __forceinline__ void sva_units(const SvaArgs& A, const Lds& L, const 
     __builtin_amdgcn_wave_barrier();
   };
 
-  // Work distribution.  Claims on one shared counter serialise at the
-  // memory side, so most units are assigned statically: with static_first,
-  // wave w takes units w, w + nwaves, ... for three quarters of the full
-  // rounds (at least one round; all units when there are fewer units than
-  // waves).  The rest is claimed from
-  // the counter in guided chunks of max(1, remaining / (2 nwaves)) units; once
-  // fewer units than waves may remain, a wave reads the counter before
-  // claiming, so that waves finding the queue drained leave without an
-  // atomic.
+  // Work distribution.  Claims on one counter serialise at the memory side
+  // (about 15 ns each), so a launch of small units must not claim them one by
+  // one from one counter: with static_first, wave w takes units w, w + nwaves,
+  // ... for three quarters of the full rounds (all of them when there are
+  // less than four rounds), and the rest is dealt out to kSvaQueues queues,
+  // unit k of it to queue k mod kSvaQueues, each with a counter of its own
+  // from which every kSvaQueues-th wave claims guided chunks of max(1, left /
+  // (2 x the queue's waves)).  The queues hold alike work, so no wave steals
+  // from another's.  (One counter for all: 2.51 against 2.11 ms for the 6-DOF
+  // roadmap, 650 against 468 us for 20,011 local 7-DOF edges, 311 against 191 us
+  // for 2,048 local 4-DOF ones; one round of static units, half or all of
+  // them: 2.24, 2.14, 2.31 ms for the roadmap, 3.49, 3.35, 3.68 against 3.32 ms
+  // for 4M points of the 7-DOF scene.)  Without static_first (the multi-scene kernel, where
+  // blocks rotate over the scenes) one queue holds everything.  Once fewer
+  // units than waves may remain, a wave reads the counter before claiming, so
+  // that waves finding the queue drained leave without an atomic.
   const unsigned nwaves = (gridDim.x * blockDim.x) >> 6;
   // wave-uniform values held in scalar registers: the unit index, and from
   // it the pair loop, the pair records and the cache tags below
   const unsigned wave = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-  unsigned nstatic = 0;
+  unsigned nstatic = 0, nq = 1, q = 0;
   if (A.static_first) {
     const unsigned rounds = nunits / nwaves;
-    // fewer units than waves: one each, nothing left to claim
-    nstatic = rounds == 0 ? nunits : (rounds * 3 / 4 > 1 ? rounds * 3 / 4 : 1u) * nwaves;
+    nstatic = rounds < 4 ? nunits : rounds * 3 / 4 * nwaves;
+    nq = kSvaQueues;
+    q = wave % kSvaQueues;
   }
+  // the queue's units and waves, and its counter
+  const unsigned qunits = nunits - nstatic > q ? (nunits - nstatic - q + nq - 1) / nq : 0u;
+  const unsigned qwaves = nwaves / nq > 0 ? nwaves / nq : 1u;
+  GAS unsigned* const counter = (GAS unsigned*)A.counter + q * kSvaQueueStride;
   unsigned su = wave;          // next static unit
-  unsigned cur = 0, cend = 0;  // units [cur, cend) claimed dynamically
+  unsigned cur = 0, cend = 0;  // the queue's units [cur, cend) are claimed
   unsigned seen = 0;           // the counter as last observed by this wave
   for (;;) {
     unsigned u;
@@ -1266,24 +1280,23 @@ __device__ __forceinline__ void sva_units(const SvaArgs& A, const Lds& L, const 
       u = su;
       su += nwaves;
     } else if (cur < cend) {
-      u = cur++;
+      u = nstatic + q + nq * cur++;
     } else {
-      const unsigned left = nunits - nstatic > seen ? nunits - nstatic - seen : 0u;
+      const unsigned left = qunits > seen ? qunits - seen : 0u;
       if (left == 0) break;
-      const unsigned k = left / (2 * nwaves) > 1 ? left / (2 * nwaves) : 1u;
+      const unsigned k = left / (2 * qwaves) > 1 ? left / (2 * qwaves) : 1u;
       unsigned b = 0xffffffffu;
       if (lane == 0) {
         bool go = true;
-        if (left < nwaves) go = __hip_atomic_load((GAS unsigned*)A.counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) <
-                                nunits - nstatic;
-        if (go) b = __hip_atomic_fetch_add((GAS unsigned*)A.counter, k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (left < qwaves) go = __hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < qunits;
+        if (go) b = __hip_atomic_fetch_add(counter, k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
       b = __builtin_amdgcn_readfirstlane(b);
-      if (b == 0xffffffffu || b >= nunits - nstatic) break;
+      if (b == 0xffffffffu || b >= qunits) break;
       seen = b + k;
-      cur = nstatic + b;
-      cend = cur + k < nunits ? cur + k : nunits;
-      u = cur++;
+      cur = b;
+      cend = b + k < qunits ? b + k : qunits;
+      u = nstatic + q + nq * cur++;
     }
     ++n_claimed;
     const unsigned ch = u / ngroups;
@@ -1985,11 +1998,12 @@ hipError_t launch_edge_prologue(const DevRobot& rb, float dq, EdgeArgs ea, int* 
 }
 
 hipError_t launch_edge_compact(EdgeArgs ea, int e0, int e1, int l0, int l1, int* item_edge,
-                               int* item_pos, int cap, int* nitems, int* nsamples, hipStream_t st) {
+                               int* item_pos, int cap, int* nitems, int* nsamples, unsigned* zero_queues,
+                               hipStream_t st) {
   if (e1 <= e0) return hipSuccess;
   dim3 grid((e1 - e0 + kCompactBlock - 1) / kCompactBlock), block(kCompactBlock);
   hipLaunchKernelGGL(edge_compact_kernel, grid, block, 0, st, ea, e0, e1, l0, l1, item_edge, item_pos, cap,
-                     nitems, nsamples);
+                     nitems, nsamples, zero_queues);
   return hipGetLastError();
 }
 

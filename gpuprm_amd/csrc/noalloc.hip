@@ -26,20 +26,21 @@ namespace gprm {
 namespace {
 
 // Layout of the scratch array (byte offsets, 256-aligned):
-//   [0, 256)                        work counter of the separating-vector launch
-//   [256, 256 + 4 kMaxItems)        result words, one per configuration
+//   [0, kCounterBytes)              work counters of the separating-vector launch
+//   words: 4 kMaxItems              result words, one per configuration
 //   frames: kFramesBytes            link frames, 48 bytes per link and configuration
 //   history: kHistBytes             per-lane iteration history, kMaxIter float4 per lane
 constexpr int kMaxItems = 1 << 16;
 constexpr size_t kCounterOff = 0;
-constexpr size_t kWordsOff = 256;
+constexpr size_t kCounterBytes = sizeof(unsigned) * kSvaCounters;
+constexpr size_t kWordsOff = kCounterBytes;
 constexpr size_t kFramesOff = kWordsOff + sizeof(int) * (size_t)kMaxItems;
 constexpr size_t kFramesBytes = 24u << 20;  // 65536 configurations of up to 8 joints
 constexpr size_t kHistOff = kFramesOff + kFramesBytes;
 constexpr size_t kHistLanes = 327680;       // 256 CUs x 5 blocks x 256 threads
 constexpr size_t kHistBytes = sizeof(float4) * kMaxIter * kHistLanes;
 constexpr size_t kScratchBytes = kHistOff + kHistBytes;  // 74.3 MiB
-static_assert(kFramesOff % 256 == 0 && kHistOff % 256 == 0, "scratch regions must stay 256-aligned");
+static_assert(kWordsOff % 256 == 0 && kFramesOff % 256 == 0 && kHistOff % 256 == 0, "scratch regions must stay 256-aligned");
 
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 

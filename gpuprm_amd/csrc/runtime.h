@@ -97,7 +97,8 @@ struct SvaArgs {
   // mask_words(M) words per group (written by the kinematics launch); null:
   // all of them
   const unsigned long long* mask;
-  unsigned int* counter;   // work counter (zero before launch)
+  unsigned int* counter;   // work counters (zero before launch): kSvaQueues of them,
+                           // kSvaQueueStride apart, with static_first, else one
   int pairs_per_unit;      // pairs of one work unit (a wave claims one chunk of them
                            // for 64 consecutive items)
   int units_per_item;      // ceil(M / pairs_per_unit)
@@ -119,10 +120,14 @@ struct SvaArgs {
   // lane), [4] iterations run, [5] pair tests decided separated by the bound
   // test
   unsigned long long* tally;
-  // single-scene launches: wave w of the grid takes unit w without a claim,
-  // and claims from the counter start after the grid's waves
+  // single-scene launches: most units are taken without a claim, the others
+  // from several queues (sva_units)
   int static_first;
 };
+// Work queues of a single-scene launch, their counters on cache lines of
+// their own.
+constexpr int kSvaQueues = 32, kSvaQueueStride = 32;
+constexpr int kSvaCounters = kSvaQueues * kSvaQueueStride;
 constexpr int kTallyCount = 6;
 constexpr int kTallySlots = 64;
 
@@ -344,8 +349,8 @@ size_t sva_lds_bytes(const SceneImg& img, int block, int gscene = 0);
 int sva_max_lds_bytes();
 
 // Kinematics of n configurations; frames link-major with item stride n.
-// zero_counter (may be null) is set to zero by the launch (the work counter
-// of the separating-vector launch that follows).  skip (may be null): items
+// zero_counter (may be null): work counters set to zero by the launch
+// (SvaArgs::counter of the separating-vector launch that follows).  skip (may be null): items
 // with skip[i] != 0 get the out-of-bounds word, so the separating-vector
 // kernel tests none of their pairs (code 1).
 hipError_t launch_fk_points(const DevRobot& rb, const float* q, long long offset, int n, float* frames,
@@ -369,9 +374,11 @@ hipError_t launch_edge_prologue(const DevRobot& rb, float dq, EdgeArgs ea, int* 
 // Items of levels [l0, l1) of the open edges in [e0, e1): item_edge, item_pos
 // (the sample), *nitems slots of which *nsamples (may be null) are no padding.
 // Slots beyond cap (an edge longer than the plan's bound) are not written.
+// zero_queues: the work counters of the separating-vector launch that
+// follows, set to zero.
 constexpr int kCompactBlock = 1024, kCompactBlockMulti = 256;
 hipError_t launch_edge_compact(EdgeArgs ea, int e0, int e1, int l0, int l1, int* item_edge, int* item_pos,
-                               int cap, int* nitems, int* nsamples, hipStream_t st);
+                               int cap, int* nitems, int* nsamples, unsigned* zero_queues, hipStream_t st);
 // Kinematics of the *nitems (<= cap) compacted samples; frames link-major
 // with item stride cap (the plane stride); their pair masks to mask unless
 // it is null.
