@@ -1053,13 +1053,25 @@ __device__ __forceinline__ unsigned sva_unit_count(const SvaArgs& A, int nitems)
   return (unsigned)((nitems + 63) >> 6) * (unsigned)A.units_per_item;
 }
 
+// The rings of a block's waves as one queue (the last drain): wave w's waiting
+// entries, moved to the start of its ring, are numbered from first[w]; next
+// is the first number not taken yet.  It lies in the last 64 slots of the
+// block's first ring, which are free then (a ring with more than CAP - 65
+// entries would have been drained), so it needs no LDS of its own.
+template <int WAVES>
+struct Pool {
+  unsigned first[WAVES + 1], next;
+};
+static_assert(sizeof(Pool<16>) <= 63 * sizeof(int2), "fits the free slots before the last");
+
 // Phase B of sva_units: every lane takes a deferred pair from the wave's
 // ring and runs the full separating-vector test (collision4.h:227-332) until
-// the ring is empty.  The gate is re-read when a pair is taken. 
-template <int EDGE, int CAP>
+// the ring is empty.  The gate is re-read when a pair is taken.  POOLED: the
+// pairs come from the block's pool instead.
+template <int EDGE, int CAP, int WAVES, bool POOLED>
 __device__ __forceinline__ void sva_drain(const SvaArgs& A, const Lds& L, const Ring& R,
                                           GAS f32x4* H, size_t hs, unsigned& d_head, unsigned d_tail,
-                                          unsigned& n_sep, unsigned& n_col, unsigned& n_dropped, unsigned& n_iter) {
+                                          Pool<WAVES>* pool, unsigned& n_sep, unsigned& n_col, unsigned& n_dropped, unsigned& n_iter) {
   const int lane = threadIdx.x & 63;
   const unsigned long long lt_mask = (1ull << lane) - 1ull;
   // the ring's entries were written by other lanes of this wave
@@ -1073,10 +1085,27 @@ __device__ __forceinline__ void sva_drain(const SvaArgs& A, const Lds& L, const 
   V3 S{0, 0, 0}, w{0, 0, 0};
   for (;;) {
     const unsigned long long wm = __ballot(!busy);
+    const unsigned want = (unsigned)__popcll(wm);
+    if (POOLED && d_head != d_tail && wm != 0ull) {
+      // d_head: the first number the wave may take, d_tail: the pool's end
+      unsigned at = 0;
+      if (lane == 0) at = atomicAdd(&pool->next, want);
+      at = __builtin_amdgcn_readfirstlane(at);
+      d_head = at < d_tail ? at : d_tail;
+    }
     const unsigned avail = d_tail - d_head;
-    const unsigned take = (unsigned)__popcll(wm) < avail ? (unsigned)__popcll(wm) : avail;
+    const unsigned take = want < avail ? want : avail;
     if (!busy && (unsigned)__popcll(wm & lt_mask) < take) {
-      const unsigned slot = (d_head + (unsigned)__popcll(wm & lt_mask)) & (CAP - 1);
+      unsigned slot = d_head + (unsigned)__popcll(wm & lt_mask);
+      if (POOLED) {
+        // the ring that holds it (R is the block's first ring)
+        int w = 0;
+        for (int step = WAVES / 2; step > 0; step /= 2)
+          if (pool->first[w + step] <= slot) w += step;
+        slot = w * CAP + (slot - pool->first[w]);
+      } else {
+        slot &= CAP - 1;
+      }
       const int2 e = R.ent[slot];
       bitem = e.x;
       const int4 pd = L.pairs[e.y];
@@ -1117,7 +1146,7 @@ __device__ __forceinline__ void sva_drain(const SvaArgs& A, const Lds& L, const 
         busy = true;
       }
     }
-    d_head += take;
+    if (!POOLED) d_head += take;
     if (__ballot(busy) == 0ull) {
       if (d_head == d_tail) break;
       continue;
@@ -1179,9 +1208,10 @@ __device__ __forceinline__ void sva_drain(const SvaArgs& A, const Lds& L, const 
 //   B. once 64 pairs wait (and at the end), every lane takes deferred pairs
 //      and runs the full test until the ring is empty (sva_drain).
 // H: this lane's iteration history (stride hs); R: the wave's ring.  Waves
-// run independently: there is no block barrier inside.  cnt.claimed counts the wave's units (the
-// same in every lane).
-template <int EDGE, int CAP>
+// run independently until the queue is exhausted; with POOL the last drain is
+// the block's (every thread calls).  cnt.claimed counts the wave's units (the
+// same in every lane), all finished on return.
+template <int EDGE, int CAP, int WAVES, bool POOL>
 __device__ __forceinline__ void sva_units(const SvaArgs& A, const Lds& L, const Ring& R,
                                           GAS f32x4* H, size_t hs, SvaCounts& cnt) {
   const int lane = threadIdx.x & 63;
@@ -1491,7 +1521,7 @@ __device__ __forceinline__ void sva_units(const SvaArgs& A, const Lds& L, const 
         }
       } while ((EDGE ? cur_pair >= 0 : cur_pair < p1) && !full);
       if (full) {
-        sva_drain<EDGE, CAP>(A, L, R, H, hs, d_head, d_tail, n_sep, n_col, n_dropped, n_iter);
+        sva_drain<EDGE, CAP, WAVES, false>(A, L, R, H, hs, d_head, d_tail, nullptr, n_sep, n_col, n_dropped, n_iter);
         if (fuse) complete_pending();  // the units before this one
       }
     }
@@ -1508,12 +1538,62 @@ __device__ __forceinline__ void sva_units(const SvaArgs& A, const Lds& L, const 
       if (d_tail == d_head) {
         complete_pending();
       } else if (n_pend == (unsigned)CAP) {
-        sva_drain<EDGE, CAP>(A, L, R, H, hs, d_head, d_tail, n_sep, n_col, n_dropped, n_iter);
+        sva_drain<EDGE, CAP, WAVES, false>(A, L, R, H, hs, d_head, d_tail, nullptr, n_sep, n_col, n_dropped, n_iter);
         complete_pending();
       }
     }
   }
-  if (d_tail != d_head) sva_drain<EDGE, CAP>(A, L, R, H, hs, d_head, d_tail, n_sep, n_col, n_dropped, n_iter);
+  // The multi-scene kernel's blocks go on to the next scene together: there,
+  // what waits in the block's rings at a scene's end is one queue for all of
+  // its waves (16 scenes of 1k-64k configurations: 1.78-1.82 against 2.00 ms).
+  // A single scene's launch gains nothing from it (65,536 points of the 4-DOF
+  // scene: 72 against 70 us).
+  if (!POOL) {
+    if (d_tail != d_head)
+      sva_drain<EDGE, CAP, WAVES, false>(A, L, R, H, hs, d_head, d_tail, nullptr, n_sep, n_col, n_dropped, n_iter);
+  } else {
+    const int w = threadIdx.x >> 6;
+    const Ring B{R.ent - w * CAP, R.edge - w * CAP};
+    Pool<WAVES>* const pool = reinterpret_cast<Pool<WAVES>*>(B.ent + CAP - 64);
+    const unsigned count = d_tail - d_head;
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    int2 ent[CAP / 64 - 1];
+    int edg[CAP / 64 - 1];
+#pragma unroll
+    for (int k = 0; k < CAP / 64 - 1; ++k) {
+      const unsigned slot = (d_head + 64 * k + lane) & (CAP - 1);
+      ent[k] = R.ent[slot];
+      edg[k] = EDGE ? R.edge[slot] : 0;
+    }
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int k = 0; k < CAP / 64 - 1; ++k)
+      if (64u * k + lane < count) {
+        R.ent[64 * k + lane] = ent[k];
+        if (EDGE) R.edge[64 * k + lane] = edg[k];
+      }
+    // each wave leaves its count in the last slot of its own ring (other
+    // waves may still be using theirs)
+    if (lane == 0) R.ent[CAP - 1].x = (int)count;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      unsigned sum = 0;
+      for (int i = 0; i < WAVES; ++i) {
+        pool->first[i] = sum;
+        sum += (unsigned)B.ent[i * CAP + CAP - 1].x;
+      }
+      pool->first[WAVES] = sum;
+      pool->next = 0;
+    }
+    __syncthreads();
+    unsigned first = 0, end = __builtin_amdgcn_readfirstlane(pool->first[WAVES]);
+    if (end != 0)
+      sva_drain<EDGE, CAP, WAVES, true>(A, L, B, H, hs, first, end, pool, n_sep, n_col, n_dropped, n_iter);
+    // the pool is read no more after this, and the wave's result words have landed
+    // (their groups' counts follow)
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+  }
   if (fuse) complete_pending();
 
   if (lane == 0) {
@@ -1565,7 +1645,7 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVE
   GAS f32x4* const H = global_f4(A.hist) + (size_t)blockIdx.x * BLOCK + threadIdx.x;
   const size_t hs = (size_t)gridDim.x * BLOCK;
   SvaCounts c;
-  sva_units<EDGE, sva_ring_cap(BLOCK)>(A, L, R, H, hs, c);
+  sva_units<EDGE, sva_ring_cap(BLOCK), BLOCK / 64, false>(A, L, R, H, hs, c);
   if (A.tally != nullptr) add_tally<BLOCK>(c, smem, A.tally);
 }
 
@@ -1599,7 +1679,7 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVE
       const Lds L = stage_scene<BLOCK>(A.img, smem + sva_ring_bytes(BLOCK) / 16);
       __syncthreads();
       const unsigned before = c.claimed;
-      sva_units<EDGE, sva_ring_cap(BLOCK)>(A, L, R, H, hs, c);
+      sva_units<EDGE, sva_ring_cap(BLOCK), BLOCK / 64, true>(A, L, R, H, hs, c);
       const unsigned mine = c.claimed - before;  // the wave's units (the same in every lane)
       if ((threadIdx.x & 63) == 0 && mine > 0) {
         const unsigned old = atomicAdd(tasks[t].done, mine);
