@@ -741,21 +741,25 @@ extern "C" int gprm_radius_neighbours(int ndof, const float* d_nodes, int n, lon
   *total = 0;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const CellGrid g = make_cell_grid(ndof, mins, maxs, D);
-  DevArr cell_id, counts, starts, cursor, sorted, sid, cnt;
+  DevArr cell_id, counts, starts, cursor, sorted, sid, qcount, qstart;
+  const size_t Q = (size_t)std::max(nq, 1);
   if (!counts.ensure(sizeof(int) * (size_t)g.ncells) || !starts.ensure(sizeof(int) * (size_t)g.ncells) ||
       !cursor.ensure(sizeof(int) * (size_t)g.ncells) || !cell_id.ensure(sizeof(int) * (size_t)std::max(n, 1)) ||
       !sid.ensure(sizeof(int) * (size_t)std::max(n, 1)) ||
-      !sorted.ensure(sizeof(float) * ndof * (size_t)std::max(n, 1)) || !cnt.ensure(sizeof(int)))
+      !sorted.ensure(sizeof(float) * ndof * (size_t)std::max(n, 1)) || !qcount.ensure(sizeof(int) * Q) ||
+      !qstart.ensure(sizeof(long long) * (Q + 1)))
     return GPRM_E_HIP;
-  int h = 0;
-  if (launch_fill_i32(cnt.as<int>(), 0, 1, st) != hipSuccess ||
-      launch_grid_build(g, ndof, d_nodes, n, noff, cell_id.as<int>(), counts.as<int>(), starts.as<int>(),
-                        cursor.as<int>(), sorted.as<float>(), sid.as<int>(), st) != hipSuccess ||
-      launch_near_grid(ndof, d_queries, nq, qoff, g, starts.as<int>(), counts.as<int>(), sorted.as<float>(),
-                       sid.as<int>(), n, D * D, d_out_q, d_out_node, d_out_d2, cnt.as<int>(), cap, st) != hipSuccess ||
-      hipMemcpyAsync(&h, cnt.p, sizeof(int), hipMemcpyDeviceToHost, st) != hipSuccess ||
-      hipStreamSynchronize(st) != hipSuccess)
+  long long h = 0;
+  if (launch_grid_build(g, ndof, d_nodes, n, noff, cell_id.as<int>(), counts.as<int>(), starts.as<int>(),
+                        cursor.as<int>(), sorted.as<float>(), sid.as<int>(), st) != hipSuccess)
     return GPRM_E_HIP;
+  if (nq > 0 && n > 0 &&
+      (launch_near_grid(ndof, d_queries, nq, qoff, g, starts.as<int>(), counts.as<int>(), sorted.as<float>(),
+                        sid.as<int>(), n, D * D, qcount.as<int>(), qstart.as<long long>(), qstart.as<long long>() + Q,
+                        d_out_q, d_out_node, d_out_d2, cap, st) != hipSuccess ||
+       hipMemcpyAsync(&h, qstart.as<long long>() + Q, sizeof(h), hipMemcpyDeviceToHost, st) != hipSuccess))
+    return GPRM_E_HIP;
+  if (hipStreamSynchronize(st) != hipSuccess) return GPRM_E_HIP;
   *total = h;
   return GPRM_OK;
 }

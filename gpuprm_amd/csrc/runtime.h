@@ -404,11 +404,13 @@ CellGrid make_cell_grid(int ndof, const float* mins, const float* maxs, float D)
 hipError_t launch_grid_build(const CellGrid& g, int ndof, const float* nodes, int n, long long noff, int* cell_id,
                              int* counts, int* starts, int* cursor, float* sorted, int* sid, hipStream_t st);
 // Radius neighbours over the cell index: every (query j, node l) with
-// |node_l - query_j|^2 < D2, appended to (out_q, out_node, out_d2) up to cap
-// entries; *count receives the total number of matches (may exceed cap).
+// |node_l - query_j|^2 < D2, sorted by query (and by node within a query of
+// at most 1,024 matches), up to cap entries; qcount [nq] and qstart [nq]
+// scratch; *total (device) receives the number of matches (may exceed cap).
 hipError_t launch_near_grid(int ndof, const float* queries, int nq, long long qoff, const CellGrid& g,
                             const int* starts, const int* counts, const float* sorted, const int* sid, int n, float D2,
-                            int* out_q, int* out_node, float* out_d2, int* count, int cap, hipStream_t st);
+                            int* qcount, long long* qstart, long long* total, int* out_q, int* out_node,
+                            float* out_d2, int cap, hipStream_t st);
 hipError_t launch_fill_u32(unsigned int* p, unsigned int v, long long n, hipStream_t st);
 
 // Launch shape of the persistent separating-vector kernel: a kernel variant

@@ -231,8 +231,9 @@ int gprm_prm_solve(gprm_ctx* ctx, const float* qstart, const float* qgoal, const
  * sum_i (node_l[i] - query_j[i])^2 < D^2, the sum taken in float over i in
  * order.  Nodes and queries are SoA device arrays (component i of item k at
  * [k + off*i], off >= count); mins/maxs (host, ndof) bound the nodes.  Up to
- * cap pairs go to the device arrays d_out_* in no particular order; *total
- * receives the number of pairs found (may exceed cap).  Through a cell index
+ * cap pairs go to the device arrays d_out_*, sorted by query and, for queries
+ * of at most 1,024 pairs, by node; *total receives the number of pairs found
+ * (may exceed cap).  Through a cell index
  * over the first coordinates (up to five) instead of the reference's q[0]
  * blocks. */
 int gprm_radius_neighbours(int ndof, const float* d_nodes, int n, long long noff, const float* d_queries, int nq,
