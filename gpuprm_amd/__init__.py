@@ -240,21 +240,25 @@ def radius_neighbours(nodes, queries, mins, maxs, D, cap=None):
     nd, n = int(nodes.shape[0]), int(nodes.shape[1])
     nq = int(queries.shape[1])
     cap = int(cap if cap is not None else max(1, n * 8))
-    oq = torch.empty(cap, dtype=torch.int32, device=nodes.device)
-    on = torch.empty(cap, dtype=torch.int32, device=nodes.device)
-    od = torch.empty(cap, dtype=torch.float32, device=nodes.device)
+    out = torch.empty((3, cap), dtype=torch.int32, device=nodes.device)  # query, node, bits of d2
     tot = C.c_longlong(0)
     rc = lib().gprm_radius_neighbours(nd, C.c_void_p(nodes.data_ptr()), n, max(1, n), C.c_void_p(queries.data_ptr()),
                                       nq, max(1, nq), _f32(mins).ctypes.data_as(_FP), _f32(maxs).ctypes.data_as(_FP),
-                                      float(D), C.c_void_p(oq.data_ptr()), C.c_void_p(on.data_ptr()),
-                                      C.c_void_p(od.data_ptr()), cap, C.byref(tot), None)
+                                      float(D), C.c_void_p(out[0].data_ptr()), C.c_void_p(out[1].data_ptr()),
+                                      C.c_void_p(out[2].data_ptr()), cap, C.byref(tot), None)
     _check(rc)
     k = min(cap, tot.value)
     if tot.value > cap:
         raise GprmError(-4, "%d pairs exceed cap %d" % (tot.value, cap))
-    q, nn, d = oq[:k].cpu().numpy(), on[:k].cpu().numpy(), od[:k].cpu().numpy()
-    o = np.lexsort((nn, q))
-    return q[o], nn[o], d[o]
+    q, nn, d = out[:, :k].cpu().numpy()  # one copy
+    d = d.view(np.float32)
+    # the library sorts the pairs of queries with up to 1,024 of them (sorting
+    # here and copying three arrays, 5.25 ms for 20,000 queries with 50,000
+    # pairs; without, 0.34 ms)
+    if k > 1 and not ((q[1:] > q[:-1]) | ((q[1:] == q[:-1]) & (nn[1:] > nn[:-1]))).all():
+        o = np.lexsort((nn, q))
+        q, nn, d = q[o], nn[o], d[o]
+    return q, nn, d
 
 
 def canonical_edges(A, B):

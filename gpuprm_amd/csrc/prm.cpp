@@ -741,23 +741,35 @@ extern "C" int gprm_radius_neighbours(int ndof, const float* d_nodes, int n, lon
   *total = 0;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const CellGrid g = make_cell_grid(ndof, mins, maxs, D);
-  DevArr cell_id, counts, starts, cursor, sorted, sid, qcount, qstart;
-  const size_t Q = (size_t)std::max(nq, 1);
-  if (!counts.ensure(sizeof(int) * (size_t)g.ncells) || !starts.ensure(sizeof(int) * (size_t)g.ncells) ||
-      !cursor.ensure(sizeof(int) * (size_t)g.ncells) || !cell_id.ensure(sizeof(int) * (size_t)std::max(n, 1)) ||
-      !sid.ensure(sizeof(int) * (size_t)std::max(n, 1)) ||
-      !sorted.ensure(sizeof(float) * ndof * (size_t)std::max(n, 1)) || !qcount.ensure(sizeof(int) * Q) ||
-      !qstart.ensure(sizeof(long long) * (Q + 1)))
-    return GPRM_E_HIP;
+  // one allocation for all scratch arrays (each costs a call tens of
+  // microseconds to get and more to give back)
+  const size_t N = (size_t)std::max(n, 1), Q = (size_t)std::max(nq, 1), C = (size_t)g.ncells;
+  size_t off = 0;
+  const auto take = [&off](size_t bytes) {
+    const size_t at = off;
+    off += (bytes + 255) & ~(size_t)255;
+    return at;
+  };
+  const size_t o_counts = take(4 * C), o_starts = take(4 * C), o_cursor = take(4 * C), o_cell = take(4 * N),
+               o_sid = take(4 * N), o_sorted = take(4 * (size_t)ndof * N), o_qcount = take(4 * Q),
+               o_qstart = take(8 * (Q + 1));
+  DevArr scratch;
+  if (!scratch.ensure(off)) return GPRM_E_HIP;
+  char* const base = scratch.as<char>();
+  int* const counts = reinterpret_cast<int*>(base + o_counts);
+  int* const starts = reinterpret_cast<int*>(base + o_starts);
+  int* const sid = reinterpret_cast<int*>(base + o_sid);
+  float* const sorted = reinterpret_cast<float*>(base + o_sorted);
+  long long* const qstart = reinterpret_cast<long long*>(base + o_qstart);
   long long h = 0;
-  if (launch_grid_build(g, ndof, d_nodes, n, noff, cell_id.as<int>(), counts.as<int>(), starts.as<int>(),
-                        cursor.as<int>(), sorted.as<float>(), sid.as<int>(), st) != hipSuccess)
+  if (launch_grid_build(g, ndof, d_nodes, n, noff, reinterpret_cast<int*>(base + o_cell), counts, starts,
+                        reinterpret_cast<int*>(base + o_cursor), sorted, sid, st) != hipSuccess)
     return GPRM_E_HIP;
   if (nq > 0 && n > 0 &&
-      (launch_near_grid(ndof, d_queries, nq, qoff, g, starts.as<int>(), counts.as<int>(), sorted.as<float>(),
-                        sid.as<int>(), n, D * D, qcount.as<int>(), qstart.as<long long>(), qstart.as<long long>() + Q,
-                        d_out_q, d_out_node, d_out_d2, cap, st) != hipSuccess ||
-       hipMemcpyAsync(&h, qstart.as<long long>() + Q, sizeof(h), hipMemcpyDeviceToHost, st) != hipSuccess))
+      (launch_near_grid(ndof, d_queries, nq, qoff, g, starts, counts, sorted, sid, n, D * D,
+                        reinterpret_cast<int*>(base + o_qcount), qstart, qstart + Q, d_out_q, d_out_node, d_out_d2,
+                        cap, st) != hipSuccess ||
+       hipMemcpyAsync(&h, qstart + Q, sizeof(h), hipMemcpyDeviceToHost, st) != hipSuccess))
     return GPRM_E_HIP;
   if (hipStreamSynchronize(st) != hipSuccess) return GPRM_E_HIP;
   *total = h;
