@@ -120,26 +120,22 @@ __device__ __forceinline__ void layer_mfma(const __bf16* __restrict__ in, const 
   for (int i = 0; i < kPJ; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  // fragments one k-step ahead; the scheduling barrier keeps the compiler
-  // from hoisting all eight steps' loads (128 more registers than there are)
+  // fragments kAhead ahead (each feeds kPJ products); the scheduling barriers
+  // keep the compiler from hoisting more of the 32 loads than there are
+  // registers for
+  constexpr int kAhead = 4;
   const __bf16* src = in + li * kHP + 8 * g;
-  bf16x8 a[4], an[4];
+  bf16x8 a[kAhead];
 #pragma unroll
-  for (int ri = 0; ri < 4; ++ri) a[ri] = *reinterpret_cast<const bf16x8*>(src + 16 * ri * kHP);
+  for (int i = 0; i < kAhead; ++i) a[i] = *reinterpret_cast<const bf16x8*>(src + 16 * (i & 3) * kHP + 32 * (i >> 2));
 #pragma unroll
-  for (int s = 0; s < 8; ++s) {
-    if (s < 7) {
-#pragma unroll
-      for (int ri = 0; ri < 4; ++ri) an[ri] = *reinterpret_cast<const bf16x8*>(src + 16 * ri * kHP + 32 * (s + 1));
-    }
+  for (int i = 0; i < 32; ++i) {
+    const int ri = i & 3, s = i >> 2, j = i + kAhead;
 #pragma unroll
     for (int cj = 0; cj < kPJ; ++cj)
-#pragma unroll
-      for (int ri = 0; ri < 4; ++ri)
-        acc[cj][ri] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[cj][s], a[ri], acc[cj][ri], 0, 0, 0);
+      acc[cj][ri] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[cj][s], a[i % kAhead], acc[cj][ri], 0, 0, 0);
+    if (j < 32) a[i % kAhead] = *reinterpret_cast<const bf16x8*>(src + 16 * (j & 3) * kHP + 32 * (j >> 2));
     __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int ri = 0; ri < 4; ++ri) a[ri] = an[ri];
   }
 }
 
@@ -267,6 +263,29 @@ __device__ __forceinline__ void store_transposed(const __bf16* __restrict__ src,
   }
 }
 
+// Inference's inputs in two parts: this wave's joints k = wave, wave + 8 of
+// rows [r0, r0 + 64), a row per lane, loaded; and (later, when they have
+// arrived) their way into xs, whose columns beyond nd stay zero.
+constexpr int kStage = kXP / kPW;
+__device__ __forceinline__ void stage_load(const float* __restrict__ q, long long off, long long r0, int n, int nd,
+                                           float (&v)[kStage], int wave, int lane) {
+  const long long r = r0 + lane;
+#pragma unroll
+  for (int i = 0; i < kStage; ++i) {
+    const int k = wave + kPW * i;
+    v[i] = 0.0f;
+    if (k < nd && r < n) v[i] = q[r + off * k];
+  }
+}
+__device__ __forceinline__ void stage_store(const float (&v)[kStage], int nd, __bf16* __restrict__ xs, int wave,
+                                            int lane) {
+#pragma unroll
+  for (int i = 0; i < kStage; ++i) {
+    const int k = wave + kPW * i;
+    if (k < nd) xs[lane * kXP + k] = (__bf16)(v[i] * 0.3183098861837907f);
+  }
+}
+
 // bf16(q / pi) of rows [r0, r0 + 64) into xs (64 x kXP, zero beyond ndof and
 // n); with xt also to xt[k * ldT + r0 + row].
 __device__ __forceinline__ void stage_inputs(const float* __restrict__ q, long long off, long long r0, int n, int nd,
@@ -283,21 +302,66 @@ __device__ __forceinline__ void stage_inputs(const float* __restrict__ q, long l
 
 // ---- inference ---------------------------------------------------------------
 // Persistent, one block per CU; W1, W2, W3 in registers (136 VGPRs per
-// wave), two waves per SIMD so one wave's epilogue (SiLU costs two
-// quarter-rate transcendentals per value) overlaps the other's products.
-// LDS: two activation tiles, the staged inputs, b1 | b2 | b3 | w4.
-constexpr size_t kPredictLds = 2 * (size_t)kTileElems * 2 + (size_t)kFR * kXP * 2 + 4 * kH * sizeof(float);
+// wave), two waves per SIMD.  A layer is a step of products (M, matrix unit)
+// and a step of SiLU (E, two quarter-rate transcendentals a value: the
+// longer one).  Were all waves in the same step, one of the two units would
+// always be idle, as it was with one tile in flight.  So a block works on two
+// tiles, A and B, in the order
+//   M1A E1A M1B E1B M2A E2A M2B E2B M3A E3A M3B E3B (next pair:) M1A E1A ...
+// with a barrier after every step, and waves 4-7 run one step behind waves
+// 0-3: on each SIMD one wave multiplies while the other evaluates SiLU.  Every
+// step's inputs were written at least two steps earlier by either half, and a
+// buffer (one per tile for layer 1 and for layer 2) is written again only
+// after the late half has read it.
+// Layer 3's activations go nowhere: each lane multiplies its own (rounded to
+// BF16 like the others) with w4, the waves leave their rows' sums in LDS, and
+// one wave adds the eight of a row in the next pair's first steps.  Reading
+// the activations back for that had taken a quarter of the kernel's time.
+// 1M rows: 500 us with one tile in flight, 368 us so; up to 16,384 rows (one
+// tile per block, the steps of B only barriers) 29 us either way.
+// LDS: four activation tiles, the staged inputs of A and B, b1 | b2 | b3 | w4,
+// the head's sums.
+constexpr size_t kPredictLds = 4 * (size_t)kTileElems * 2 + 2 * (size_t)kFR * kXP * 2 + 4 * kH * sizeof(float) +
+                               2 * kPW * kFR * sizeof(float);
+
+// Layer 3's epilogue: sum[row] = this wave's columns' products of
+// bf16(silu(acc + bias)) with w4, for row = 16 ri + li.
+__device__ __forceinline__ void epi_head(const f32x4 (&acc)[kPJ][4], const float* __restrict__ bias,
+                                         const float* __restrict__ w4, float* __restrict__ sum, int wave, int lane) {
+  const int li = lane & 15, g = lane >> 4;
+  float z[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int cj = 0; cj < kPJ; ++cj) {
+    const int col = kPC * wave + 16 * cj + 4 * g;
+    const float4 bb = *reinterpret_cast<const float4*>(bias + col);
+    const float4 ww = *reinterpret_cast<const float4*>(w4 + col);
+#pragma unroll
+    for (int ri = 0; ri < 4; ++ri) {
+      z[ri] += (float)(__bf16)silu_fast(acc[cj][ri][0] + bb.x) * ww.x;
+      z[ri] += (float)(__bf16)silu_fast(acc[cj][ri][1] + bb.y) * ww.y;
+      z[ri] += (float)(__bf16)silu_fast(acc[cj][ri][2] + bb.z) * ww.z;
+      z[ri] += (float)(__bf16)silu_fast(acc[cj][ri][3] + bb.w) * ww.w;
+    }
+  }
+#pragma unroll
+  for (int ri = 0; ri < 4; ++ri) {
+    z[ri] += __shfl_xor(z[ri], 16, 64);
+    z[ri] += __shfl_xor(z[ri], 32, 64);
+  }
+  // lane 16 g + li keeps row 16 g + li
+  sum[lane] = g == 0 ? z[0] : g == 1 ? z[1] : g == 2 ? z[2] : z[3];
+}
 
 __global__ void __launch_bounds__(kPW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
     mlp_predict_kernel(const float* __restrict__ q, long long off, int n, int nd, const unsigned short* __restrict__ W1h,
                        const unsigned short* __restrict__ W2h, const unsigned short* __restrict__ W3h,
                        const float* __restrict__ P, float* __restrict__ prob) {
   extern __shared__ __bf16 hs[];
-  __bf16* const h0 = hs;
-  __bf16* const h1 = hs + kTileElems;
-  __bf16* const xs = hs + 2 * kTileElems;
-  float* const bs = reinterpret_cast<float*>(xs + kFR * kXP);  // b1 | b2 | b3 | w4
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  // activations: layer 1's of A, of B, layer 2's of A, of B
+  __bf16* const xs = hs + 4 * kTileElems;  // inputs of A, of B
+  float* const bs = reinterpret_cast<float*>(xs + 2 * kFR * kXP);  // b1 | b2 | b3 | w4
+  float* const sums = bs + 4 * kH;  // [tile][wave][row]
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   for (int e = tid; e < kH; e += kPW * 64) {
     bs[e] = P[kOffB1 + e];
     bs[kH + e] = P[kOffB2 + e];
@@ -305,45 +369,68 @@ __global__ void __launch_bounds__(kPW * 64) __attribute__((amdgpu_waves_per_eu(2
     bs[3 * kH + e] = P[kOffW4 + e];
   }
   bf16x8 w1[kPJ], w2[kPJ][8], w3[kPJ][8];
+  const long long stride = (long long)gridDim.x * kFR;
+  long long r0 = (long long)blockIdx.x * kFR;  // tile A's first row, tile B's is r0 + stride
+  stage_inputs(q, off, r0, n, nd, xs, nullptr, 0, tid);
+  stage_inputs(q, off, r0 + stride, n, nd, xs + kFR * kXP, nullptr, 0, tid);
+  // the weights last: loads arrive in order, and layer 1 need not wait for
+  // those of layers 2 and 3
+  const float bias4 = P[kOffB4];
   load_w1_frags(W1h, w1, wave, lane);
   load_frags(W2h, w2, wave, lane);
   load_frags(W3h, w3, wave, lane);
-  const float bias4 = P[kOffB4];
-  const long long stride = (long long)gridDim.x * kFR;
-  stage_inputs(q, off, (long long)blockIdx.x * kFR, n, nd, xs, nullptr, 0, tid);
   __syncthreads();
-  for (long long r0 = (long long)blockIdx.x * kFR; r0 < n; r0 += stride) {
-    f32x4 acc[kPJ][4];
-    layer1_mfma(xs, w1, acc, lane);
-    epi_predict(acc, bs, h0, wave, lane);
-    __syncthreads();
-    // xs is free: the next tile's inputs load while the layers run
-    stage_inputs(q, off, r0 + stride, n, nd, xs, nullptr, 0, tid);
-    layer_mfma(h0, w2, acc, lane);
-    epi_predict(acc, bs + kH, h1, wave, lane);
-    __syncthreads();
-    layer_mfma(h1, w3, acc, lane);
-    epi_predict(acc, bs + 2 * kH, h0, wave, lane);
-    __syncthreads();
-    // head: z = h3 . w4 + b4 (eight threads per row, 32 inputs each),
-    // p = sigmoid(z)
-    {
-      const int row = tid >> 3, part = tid & 7;
-      const float* const w4s = bs + 3 * kH;
-      float sacc = 0.0f;
+  const bool late = wave >= kPW / 2;
+  if (late) __syncthreads();
+  long long before = -1;  // the pair whose heads are due (its tile A), none at first
+  for (;; r0 += 2 * stride) {
+    const bool on = r0 < n;  // the same in every thread, as all conditions here
+    const int lane = opaque_tid() & 63;
+    float next[2][kStage];
 #pragma unroll
-      for (int k = 32 * part; k < 32 * part + 32; k += 8) {
-        const bf16x8 hv = *reinterpret_cast<const bf16x8*>(h0 + row * kHP + k);
+    for (int t = 0; t < 2; ++t) {
+      const long long rt = r0 + t * stride;
+      // the previous pair's probabilities, by one of the early waves
+      if (wave == t && before >= 0) {
+        const long long r = before + t * stride + lane;
+        float z = bias4;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) sacc += (float)hv[j] * w4s[k + j];
+        for (int w = 0; w < kPW; ++w) z += sums[(t * kPW + w) * kFR + lane];
+        if (r < n) prob[r] = rcp(1.0f + __expf(-z));
       }
-      sacc += __shfl_xor(sacc, 1, 64);
-      sacc += __shfl_xor(sacc, 2, 64);
-      sacc += __shfl_xor(sacc, 4, 64);
-      if (part == 0 && r0 + row < n) prob[r0 + row] = rcp(1.0f + __expf(-(sacc + bias4)));
+      f32x4 acc[kPJ][4];
+      const bool run = rt < n;
+      if (run) layer1_mfma(xs + t * kFR * kXP, w1, acc, lane);
+      // the next pair's inputs: loaded here, staged four steps on
+      stage_load(q, off, rt + 2 * stride, n, nd, next[t], wave, lane);
+      __syncthreads();
+      if (run) epi_predict(acc, bs, hs + (size_t)t * kTileElems, wave, lane);
+      __syncthreads();
     }
-    __syncthreads();  // h0 is the next tile's layer-1 output
+    if (!on) break;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      f32x4 acc[kPJ][4];
+      const bool run = r0 + t * stride < n;
+      // both halves' layer 1 has read this pair's inputs
+      stage_store(next[t], nd, xs + t * kFR * kXP, wave, lane);
+      if (run) layer_mfma(hs + (size_t)t * kTileElems, w2, acc, lane);
+      __syncthreads();
+      if (run) epi_predict(acc, bs + kH, hs + (size_t)(2 + t) * kTileElems, wave, lane);
+      __syncthreads();
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      f32x4 acc[kPJ][4];
+      const bool run = r0 + t * stride < n;
+      if (run) layer_mfma(hs + (size_t)(2 + t) * kTileElems, w3, acc, lane);
+      __syncthreads();
+      if (run) epi_head(acc, bs + 2 * kH, bs + 3 * kH, sums + (t * kPW + wave) * kFR, wave, lane);
+      __syncthreads();
+    }
+    before = r0;
   }
+  if (!late) __syncthreads();
 }
 
 // ---- training ------------------------------------------------------------------
