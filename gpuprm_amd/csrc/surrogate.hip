@@ -641,38 +641,52 @@ __global__ void __launch_bounds__(256) mlp_wgrad_kernel(WgradArgs a) {
   __shared__ __bf16 As[2][TI * KP];
   __shared__ __bf16 Bs[2][TJ * KP];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, g = lane >> 4;
-  const bool second = (int)blockIdx.x >= a.tiles;
+  // Consecutive blocks go to the eight XCDs in turn.  Where a row of blocks
+  // has eight tiles, eight rows at a time are transposed, so that the tiles
+  // of one split, which read the same rows, share an XCD's L2.
+  int bx = blockIdx.x, split = blockIdx.y;
+  if (gridDim.x == 8 && split < (int)(gridDim.y & ~7u)) {
+    const int low = split & 7;
+    split += bx - low;
+    bx = low;
+  }
+  const bool second = bx >= a.tiles;
   const WgradLayer L = second ? a.L1 : a.L0;
-  const int tile = (int)blockIdx.x - (second ? a.tiles : 0);
+  const int tile = bx - (second ? a.tiles : 0);
   const int tilesJ = L.J / TJ;
   const int i0 = (tile / tilesJ) * TI, j0 = (tile % tilesJ) * TJ;
   const int wi = wave / BJ, wj = wave % BJ;
-  const long long kb = (long long)blockIdx.y * a.kc, ke = min(a.K, kb + a.kc);
+  const long long kb = (long long)split * a.kc, ke = min(a.K, kb + a.kc);
   const bool do_bias = j0 == 0 && wj == 0;
-  bf16x8 ra[NA], rb[NB];
-  auto gload = [&](long long k0) {
+  // Chunk c's loads are issued kAheadK chunks before it is multiplied: with
+  // one ahead an iteration was one round trip to memory, 27 us for 32,768
+  // rows (the two 256 x 256 layers); 23 us so (with the blocks' order above 24).
+  constexpr int kAheadK = 4;
+  bf16x8 ra[kAheadK][NA], rb[kAheadK][NB];
+  auto gload = [&](int c, int slot) {
+    const long long k0 = kb + (long long)KC * c;
 #pragma unroll
     for (int m = 0; m < NA; ++m) {
-      const int c = tid + 256 * m, row = c / (KC / 8), part = c % (KC / 8);
-      ra[m] = *reinterpret_cast<const bf16x8*>(L.A + (size_t)(i0 + row) * a.ldT + k0 + 8 * part);
+      const int e = tid + 256 * m, row = e / (KC / 8), part = e % (KC / 8);
+      ra[slot][m] = *reinterpret_cast<const bf16x8*>(L.A + (size_t)(i0 + row) * a.ldT + k0 + 8 * part);
     }
 #pragma unroll
     for (int m = 0; m < NB; ++m) {
-      const int c = tid + 256 * m, row = c / (KC / 8), part = c % (KC / 8);
-      if (c < TJ * (KC / 8))
-        rb[m] = *reinterpret_cast<const bf16x8*>(L.B + (size_t)(j0 + row) * a.ldT + k0 + 8 * part);
+      const int e = tid + 256 * m, row = e / (KC / 8), part = e % (KC / 8);
+      if (e < TJ * (KC / 8))
+        rb[slot][m] = *reinterpret_cast<const bf16x8*>(L.B + (size_t)(j0 + row) * a.ldT + k0 + 8 * part);
     }
   };
-  auto sstore = [&](int buf) {
+  auto sstore = [&](int slot, int buf) {
 #pragma unroll
     for (int m = 0; m < NA; ++m) {
-      const int c = tid + 256 * m, row = c / (KC / 8), part = c % (KC / 8);
-      *reinterpret_cast<bf16x8*>(&As[buf][row * KP + 8 * part]) = ra[m];
+      const int e = tid + 256 * m, row = e / (KC / 8), part = e % (KC / 8);
+      *reinterpret_cast<bf16x8*>(&As[buf][row * KP + 8 * part]) = ra[slot][m];
     }
 #pragma unroll
     for (int m = 0; m < NB; ++m) {
-      const int c = tid + 256 * m, row = c / (KC / 8), part = c % (KC / 8);
-      if (c < TJ * (KC / 8)) *reinterpret_cast<bf16x8*>(&Bs[buf][row * KP + 8 * part]) = rb[m];
+      const int e = tid + 256 * m, row = e / (KC / 8), part = e % (KC / 8);
+      if (e < TJ * (KC / 8)) *reinterpret_cast<bf16x8*>(&Bs[buf][row * KP + 8 * part]) = rb[slot][m];
     }
   };
   f32x4 acc[4][WN];
@@ -681,15 +695,7 @@ __global__ void __launch_bounds__(256) mlp_wgrad_kernel(WgradArgs a) {
 #pragma unroll
     for (int bj = 0; bj < WN; ++bj) acc[bi][bj] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   float bsum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-  if (kb < ke) {
-    gload(kb);
-    sstore(0);
-  }
-  __syncthreads();
-  int buf = 0;
-  for (long long k0 = kb; k0 < ke; k0 += KC) {
-    const bool more = k0 + KC < ke;
-    if (more) gload(k0 + KC);
+  auto multiply = [&](int buf) {
     bf16x8 af[4], bfr[WN];
 #pragma unroll
     for (int bi = 0; bi < 4; ++bi)
@@ -708,12 +714,38 @@ __global__ void __launch_bounds__(256) mlp_wgrad_kernel(WgradArgs a) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) bsum[bi] += (float)af[bi][e];
     }
-    if (more) sstore(buf ^ 1);
-    __syncthreads();
-    buf ^= 1;
+  };
+  const int nc = kb < ke ? (int)((ke - kb) / KC) : 0;  // both are multiples of KC
+#pragma unroll
+  for (int u = 0; u < kAheadK; ++u)
+    if (u < nc) gload(u, u);
+  if (nc > 0) sstore(0, 0);
+  __syncthreads();
+  // chunk c is in buffer c % 2, was in slot c % kAheadK (even, so c0 is too)
+  int c0 = 0;
+  for (; c0 + 2 * kAheadK <= nc; c0 += kAheadK) {  // every load below exists: no branches between them
+#pragma unroll
+    for (int u = 0; u < kAheadK; ++u) {
+      gload(c0 + u + kAheadK, u);
+      multiply(u & 1);
+      sstore((u + 1) % kAheadK, (u & 1) ^ 1);
+      __syncthreads();
+    }
+  }
+  for (; c0 < nc; c0 += kAheadK) {
+#pragma unroll
+    for (int u = 0; u < kAheadK; ++u) {
+      const int c = c0 + u;
+      if (c < nc) {
+        if (c + kAheadK < nc) gload(c + kAheadK, u);
+        multiply(u & 1);
+        if (c + 1 < nc) sstore((u + 1) % kAheadK, (u & 1) ^ 1);
+        __syncthreads();
+      }
+    }
   }
   // D(i, j) of a 16 x 16 block: lane holds column j = li, rows 4 g + r
-  float* const out = a.ws + (size_t)blockIdx.y * a.row;
+  float* const out = a.ws + (size_t)split * a.row;
 #pragma unroll
   for (int bi = 0; bi < 4; ++bi)
 #pragma unroll
@@ -751,43 +783,54 @@ struct UpdateArgs {
   float lr, b1, b2, eps, c1, c2;
 };
 
-__global__ void mlp_update_kernel(UpdateArgs a) {
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx > kPtot) return;
-  if (idx == kPtot) {
+// Rows [first, last) of partial sums `pitch` apart, added in order, 32 loads
+// in flight at a time.  (The last, short group reads its last row again
+// rather than branch around every load.)
+__device__ __forceinline__ float sum_rows(const float* __restrict__ src, int first, int last, int pitch) {
+  float sum = 0.0f;
+  for (int s0 = first; s0 < last; s0 += 32) {
+    float v[32];
+#pragma unroll
+    for (int j = 0; j < 32; ++j) v[j] = src[(size_t)min(s0 + j, last - 1) * pitch];
+#pragma unroll
+    for (int j = 0; j < 32; ++j) sum += s0 + j < last ? v[j] : 0.0f;
+  }
+  return sum;
+}
+
+// W1 .. b3 have at most 128 splits, one thread per parameter.  w4, b4 and the
+// loss have one partial row per block of F (256): there a block's four waves
+// take a quarter of the rows each, for 64 of these parameters, and the
+// quarters are added in order.  As one thread's chain of loads (the loss's 8
+// at a time) they were the whole launch, 19 us; 6.2 us so.
+constexpr int kUpdTail = (kRowF + 63) / 64;  // blocks of the second kind, after those of the first
+constexpr int kUpdBlocks = (kOffW4 + 255) / 256 + kUpdTail;
+
+__global__ void __launch_bounds__(256) mlp_update_kernel(UpdateArgs a) {
+  __shared__ float quarter[4][64];
+  const int tail = (int)blockIdx.x - (kUpdBlocks - kUpdTail);
+  int idx = blockIdx.x * 256 + threadIdx.x;
+  float gsum = 0.0f;
+  if (tail < 0) {
+    if (idx >= kOffW4) return;
+    if (a.mode != 2)
+      gsum = idx < kOffW2 ? sum_rows(a.wsW1 + idx, 0, a.SW1, kOffW2) : sum_rows(a.wsW + idx, 0, a.SW, kRowW);
+  } else {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = 64 * tail + lane;
+    idx = kOffW4 + c;
     if (a.mode != 2) {
-      float l = 0.0f;
-      for (int s0 = 0; s0 < a.SF; s0 += 8) {
-        float v[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = s0 + j < a.SF ? a.wsF[(size_t)(s0 + j) * kRowF + kH + 1] : 0.0f;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) l += v[j];
-      }
-      a.loss[0] = l;
+      if (c < kH + 2) quarter[wave][lane] = sum_rows(a.wsF + c, a.SF * wave / 4, a.SF * (wave + 1) / 4, kRowF);
+      __syncthreads();
     }
-    return;
+    if (wave > 0 || idx > kPtot) return;
+    if (a.mode != 2) gsum = ((quarter[0][lane] + quarter[1][lane]) + quarter[2][lane]) + quarter[3][lane];
+    if (idx == kPtot) {
+      if (a.mode != 2) a.loss[0] = gsum;
+      return;
+    }
   }
   float w = a.P[idx];
   if (a.mode != 2) {
-    const float* src;
-    int rows, pitch;
-    if (idx < kOffW2) {
-      src = a.wsW1 + idx; rows = a.SW1; pitch = kOffW2;
-    } else if (idx < kRowW) {
-      src = a.wsW + idx; rows = a.SW; pitch = kRowW;
-    } else {
-      src = a.wsF + (idx - kOffW4); rows = a.SF; pitch = kRowF;
-    }
-    // in split order, 32 loads in flight at a time
-    float gsum = 0.0f;
-    for (int s0 = 0; s0 < rows; s0 += 32) {
-      float v[32];
-#pragma unroll
-      for (int j = 0; j < 32; ++j) v[j] = s0 + j < rows ? src[(size_t)(s0 + j) * pitch] : 0.0f;
-#pragma unroll
-      for (int j = 0; j < 32; ++j) gsum += v[j];
-    }
     a.G[idx] = gsum;
     if (a.mode == 1) {
       const float mi = a.b1 * a.M[idx] + (1.0f - a.b1) * gsum;
@@ -888,7 +931,7 @@ hipError_t update(Surrogate* s, int mode, float lr, hipStream_t st) {
   u.lr = lr; u.b1 = 0.9f; u.b2 = 0.999f; u.eps = 1e-8f;
   u.c1 = 1.0f - std::pow(u.b1, (float)s->step);
   u.c2 = 1.0f - std::pow(u.b2, (float)s->step);
-  hipLaunchKernelGGL(mlp_update_kernel, dim3((kPtot + 1 + 255) / 256), dim3(256), 0, st, u);
+  hipLaunchKernelGGL(mlp_update_kernel, dim3(kUpdBlocks), dim3(256), 0, st, u);
   if (mode != 0)
     hipLaunchKernelGGL(mlp_transpose_kernel, dim3(kH / 64, kH / 64, 2), dim3(256), 0, st, s->W2h, s->W3h, s->W2t,
                        s->W3t);
