@@ -109,7 +109,13 @@ size_t align16(size_t x) { return (x + 15) & ~(size_t)15; }
 // each, the scan's too: it suffices that the scan's margin exceeds
 // (2 L + 2) g.  The coefficients are checked here from the stored adjacency,
 // so a row that misses edges has no factor.
+//   Faces of more than three vertices are not quite plane in floats, so a
+// vertex of a face may lie outside the cone by a rounding error.  A negative
+// coefficient -m adds at most m |e_i.d| <= 2 m vmax |d|_1, and counts as
+// m kScanOutside of sum l_i.  (Refusing any negative one left most boxes to the
+// climb: 65,536 points of the 4-DOF scene 66 against 62.5 us so.)
 constexpr int kScanVertices = 32, kScanDegree = 16;
+constexpr double kScanOutside = 5e6;  // 2 vmax |d|_1 over the 2 g (g = 3.41 2^-24 vmax |d|_1) of one l_i, and some
 float support_factor(const Polytope& p) {
   const float none = INFINITY;
   const int n = p.n();
@@ -143,8 +149,9 @@ float support_factor(const Polytope& p) {
                      p0[2] * (p1[0] * p2[1] - p1[1] * p2[0]);
             };
             const double li = det3(x, e[j], f) / det, lj = det3(e[i], x, f) / det, lk = det3(e[i], e[j], x) / det;
-            if (li < -1e-12 || lj < -1e-12 || lk < -1e-12) continue;
-            best = std::min(best, li + lj + lk);
+            double sum = 0.0;
+            for (double v : {li, lj, lk}) sum += v > 0.0 ? v : -kScanOutside * v;
+            best = std::min(best, sum);
           }
         }
       if (best > 1e6) return none;
