@@ -877,10 +877,25 @@ struct Lds {
   const unsigned short* adj;    // rows of 4k neighbour ids, padded with the row's own vertex
 };
 
-// Per-lane iteration history R[k] (x, y, z) and combs[k] (w: p | q << 16) in
-// global memory, entry k of a lane at H[k * hs] (lanes adjacent, so the lanes
-// of a wave at the same k touch one contiguous span); only iterations that do
-// not separate touch it.
+// A lane's iteration history R[k] (x, y, z) and combs[k] (w: p | q << 16);
+// only iterations that do not separate touch it.  The first n entries are in
+// LDS (as many as fit beside the launch's resident blocks, history_entries),
+// the others in global memory, where a wave's entries are one 16 KB block.
+// Lanes are adjacent in both.  Every iteration reads all entries before it,
+// two at a time: in memory, with entry k of all lanes of the launch together,
+// each read was a trip to the L2 and often to another page.  (3,001 points of
+// the 7-DOF scene 76 -> 72 us, of which 1 by the blocks; 16 scenes 1.81 -> 1.73
+// ms, the 6-DOF roadmap's edges 2.11 -> 2.02 ms.)
+constexpr int kHistStride = 64;
+struct History {
+  f32x4* l;  // LDS, entries ls apart
+  int n, ls;
+  GAS f32x4* g;  // global memory, entries kHistStride apart
+};
+__device__ __forceinline__ History lane_history(float4* hist, unsigned thread, f32x4* lds, int n, int ls) {
+  return History{lds, n, ls,
+                 (GAS f32x4*)hist + (size_t)(thread >> 6) * (size_t)(kMaxIter * kHistStride) + (thread & 63)};
+}
 
 __device__ __forceinline__ int info_of(const float4& r) { return __float_as_int(r.w); }
 
@@ -975,10 +990,11 @@ __device__ __forceinline__ V2 mult23(const Orth& o, const V3& x) {
 // repeats, as in the reference, where the repetition test comes first; the
 // scan stops changing ra/rb where find_half_plane returns false.
 constexpr int kHistBatch = 2;  // history loads in flight (four spill registers at five waves per SIMD)
-template <class HP>
-__device__ __forceinline__ int sva_slow(HP H, size_t hs, int& k, int l, int pq, const V3& r,
+__device__ __forceinline__ int sva_slow(const History& H, int& k, int l, int pq, const V3& r,
                                         float dp, V3& S, V3& w) {
-  H[k * hs] = f32x4{r.x, r.y, r.z, __int_as_float(pq)};
+  const f32x4 mine{r.x, r.y, r.z, __int_as_float(pq)};
+  if (k < H.n) H.l[k * H.ls] = mine;
+  else H.g[k * kHistStride] = mine;
   // find_half_plane returns at once (w unchanged) when w.r > 0
   const bool scan = k >= 2 && !(dot3(w, r) > 0);
   Orth o{};
@@ -996,10 +1012,11 @@ __device__ __forceinline__ int sva_slow(HP H, size_t hs, int& k, int l, int pq, 
   for (int j0 = 0; j0 < k; j0 += kHistBatch) {
     f32x4 e[kHistBatch];
 #pragma unroll
-    for (int u = 0; u < kHistBatch; ++u)
-      {
+    for (int u = 0; u < kHistBatch; ++u) {
       e[u] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-      if (j0 + u < k) e[u] = H[(j0 + u) * hs];
+      if (j0 + u >= k) continue;
+      if (j0 + u < H.n) e[u] = H.l[(j0 + u) * H.ls];
+      else e[u] = H.g[(j0 + u) * kHistStride];
     }
 #pragma unroll
     for (int u = 0; u < kHistBatch; ++u) {
@@ -1145,7 +1162,7 @@ static_assert(sizeof(Pool<16>) <= 63 * sizeof(int2), "fits the free slots before
 // pairs come from the block's pool instead.
 template <int EDGE, int CAP, int WAVES, bool POOLED>
 __device__ __forceinline__ void sva_drain(const SvaArgs& A, const Lds& L, const Ring& R,
-                                          GAS f32x4* H, size_t hs, unsigned& d_head, unsigned d_tail,
+                                          const History& H, unsigned& d_head, unsigned d_tail,
                                           Pool<WAVES>* pool, unsigned& n_sep, unsigned& n_col, unsigned& n_dropped, unsigned& n_iter) {
   const int lane = threadIdx.x & 63;
   const unsigned long long lt_mask = (1ull << lane) - 1ull;
@@ -1247,7 +1264,7 @@ __device__ __forceinline__ void sva_drain(const SvaArgs& A, const Lds& L, const 
     if (dp >= -kEpsBelow) {
       fin = true;
     } else {
-      code = sva_slow(H, hs, k, l, (p - vbP) | ((q - vbQ) << 16), r, dp, S, w);
+      code = sva_slow(H, k, l, (p - vbP) | ((q - vbQ) << 16), r, dp, S, w);
       if (code != 0) {
         fin = true;
       } else if (++l >= kMaxIter) {
@@ -1282,13 +1299,13 @@ __device__ __forceinline__ void sva_drain(const SvaArgs& A, const Lds& L, const 
 //      pairs; a pair it does not decide is appended to the wave's ring;
 //   B. once 64 pairs wait (and at the end), every lane takes deferred pairs
 //      and runs the full test until the ring is empty (sva_drain).
-// H: this lane's iteration history (stride hs); R: the wave's ring.  Waves
+// H: this lane's iteration history; R: the wave's ring.  Waves
 // run independently until the queue is exhausted; with POOL the last drain is
 // the block's (every thread calls).  cnt.claimed counts the wave's units (the
 // same in every lane), all finished on return.
 template <int EDGE, int CAP, int WAVES, bool POOL>
 __device__ __forceinline__ void sva_units(const SvaArgs& A, const Lds& L, const Ring& R,
-                                          GAS f32x4* H, size_t hs, SvaCounts& cnt) {
+                                          const History& H, SvaCounts& cnt) {
   const int lane = threadIdx.x & 63;
   const unsigned long long lt_mask = (1ull << lane) - 1ull;
   // the same in every lane, as are the unit indices derived from it: said by
@@ -1596,7 +1613,7 @@ __device__ __forceinline__ void sva_units(const SvaArgs& A, const Lds& L, const 
         }
       } while ((EDGE ? cur_pair >= 0 : cur_pair < p1) && !full);
       if (full) {
-        sva_drain<EDGE, CAP, WAVES, false>(A, L, R, H, hs, d_head, d_tail, nullptr, n_sep, n_col, n_dropped, n_iter);
+        sva_drain<EDGE, CAP, WAVES, false>(A, L, R, H, d_head, d_tail, nullptr, n_sep, n_col, n_dropped, n_iter);
         if (fuse) complete_pending();  // the units before this one
       }
     }
@@ -1613,7 +1630,7 @@ __device__ __forceinline__ void sva_units(const SvaArgs& A, const Lds& L, const 
       if (d_tail == d_head) {
         complete_pending();
       } else if (n_pend == (unsigned)CAP) {
-        sva_drain<EDGE, CAP, WAVES, false>(A, L, R, H, hs, d_head, d_tail, nullptr, n_sep, n_col, n_dropped, n_iter);
+        sva_drain<EDGE, CAP, WAVES, false>(A, L, R, H, d_head, d_tail, nullptr, n_sep, n_col, n_dropped, n_iter);
         complete_pending();
       }
     }
@@ -1625,7 +1642,7 @@ __device__ __forceinline__ void sva_units(const SvaArgs& A, const Lds& L, const 
   // scene: 72 against 70 us).
   if (!POOL) {
     if (d_tail != d_head)
-      sva_drain<EDGE, CAP, WAVES, false>(A, L, R, H, hs, d_head, d_tail, nullptr, n_sep, n_col, n_dropped, n_iter);
+      sva_drain<EDGE, CAP, WAVES, false>(A, L, R, H, d_head, d_tail, nullptr, n_sep, n_col, n_dropped, n_iter);
   } else {
     const int w = threadIdx.x >> 6;
     const Ring B{R.ent - w * CAP, R.edge - w * CAP};
@@ -1663,7 +1680,7 @@ __device__ __forceinline__ void sva_units(const SvaArgs& A, const Lds& L, const 
     __syncthreads();
     unsigned first = 0, end = __builtin_amdgcn_readfirstlane(pool->first[WAVES]);
     if (end != 0)
-      sva_drain<EDGE, CAP, WAVES, true>(A, L, B, H, hs, first, end, pool, n_sep, n_col, n_dropped, n_iter);
+      sva_drain<EDGE, CAP, WAVES, true>(A, L, B, H, first, end, pool, n_sep, n_col, n_dropped, n_iter);
     // the pool is read no more after this, and the wave's result words have landed
     // (their groups' counts follow)
     __builtin_amdgcn_s_waitcnt(0);
@@ -1712,15 +1729,16 @@ __device__ __forceinline__ void add_tally(const SvaCounts& c, int4* smem, unsign
 template <int EDGE, int BLOCK, int WAVES, int GS>
 __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES, 8))) sva_kernel(SvaArgs A) {
   extern __shared__ int4 smem[];
-  // dynamic LDS: the waves' deferral rings (sva_ring_bytes), then the
-  // scene image (unless GS)
-  const Lds L = GS ? scene_global(A.img) : stage_scene<BLOCK>(A.img, smem + sva_ring_bytes(BLOCK) / 16);
+  // dynamic LDS: the waves' deferral rings (sva_ring_bytes), the lanes'
+  // first history entries, then the scene image (unless GS)
+  f32x4* const lh = reinterpret_cast<f32x4*>(smem + sva_ring_bytes(BLOCK) / 16);
+  const Lds L = GS ? scene_global(A.img)
+                   : stage_scene<BLOCK>(A.img, reinterpret_cast<int4*>(lh + (size_t)A.lds_hist * BLOCK));
   const Ring R = wave_ring<BLOCK>(smem);
   __syncthreads();
-  GAS f32x4* const H = global_f4(A.hist) + (size_t)blockIdx.x * BLOCK + threadIdx.x;
-  const size_t hs = (size_t)gridDim.x * BLOCK;
+  const History H = lane_history(A.hist, blockIdx.x * BLOCK + threadIdx.x, lh + threadIdx.x, A.lds_hist, BLOCK);
   SvaCounts c;
-  sva_units<EDGE, sva_ring_cap(BLOCK), BLOCK / 64, false>(A, L, R, H, hs, c);
+  sva_units<EDGE, sva_ring_cap(BLOCK), BLOCK / 64, false>(A, L, R, H, c);
   if (A.tally != nullptr) add_tally<BLOCK>(c, smem, A.tally);
 }
 
@@ -1733,13 +1751,14 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVE
 template <int EDGE, int BLOCK, int WAVES>
 __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES, 8)))
     sva_multi_kernel(const SceneTask* __restrict__ tasks, int ntasks, unsigned long long* t_start,
-                     unsigned long long* tally) {
+                     unsigned long long* tally, int lds_hist) {
   extern __shared__ int4 smem[];
   __shared__ int s_live;
   if (threadIdx.x == 0) atomicMin(t_start, (unsigned long long)wall_clock64());
-  GAS f32x4* const H = global_f4(tasks[0].a.hist) + (size_t)blockIdx.x * BLOCK + threadIdx.x;
-  const size_t hs = (size_t)gridDim.x * BLOCK;
-  // dynamic LDS as in sva_kernel: deferral rings, then the scene image
+  f32x4* const lh = reinterpret_cast<f32x4*>(smem + sva_ring_bytes(BLOCK) / 16);
+  const History H =
+      lane_history(tasks[0].a.hist, blockIdx.x * BLOCK + threadIdx.x, lh + threadIdx.x, lds_hist, BLOCK);
+  // dynamic LDS as in sva_kernel: rings, history, scene image
   const Ring R = wave_ring<BLOCK>(smem);
   SvaCounts c;
   for (int r = 0; r < ntasks; ++r) {
@@ -1751,10 +1770,10 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVE
       s_live = __hip_atomic_load(A.counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < nunits ? 1 : 0;
     __syncthreads();
     if (s_live) {
-      const Lds L = stage_scene<BLOCK>(A.img, smem + sva_ring_bytes(BLOCK) / 16);
+      const Lds L = stage_scene<BLOCK>(A.img, reinterpret_cast<int4*>(lh + (size_t)lds_hist * BLOCK));
       __syncthreads();
       const unsigned before = c.claimed;
-      sva_units<EDGE, sva_ring_cap(BLOCK), BLOCK / 64, true>(A, L, R, H, hs, c);
+      sva_units<EDGE, sva_ring_cap(BLOCK), BLOCK / 64, true>(A, L, R, H, c);
       const unsigned mine = c.claimed - before;  // the wave's units (the same in every lane)
       if ((threadIdx.x & 63) == 0 && mine > 0) {
         const unsigned old = atomicAdd(tasks[t].done, mine);
@@ -1791,10 +1810,9 @@ __device__ void fk_frames(const DevRobot& rb, const float* q, T12* out) {
 }
 
 // The full separating-vector test of one pair (collision4.h:227-332), as
-// sva_drain runs it per lane; H: this lane's iteration history, stride hs.
+// sva_drain runs it per lane; H: this lane's iteration history.
 __device__ int sva_pair_full(const Lds& L, const T12& tp, const T12& tq, bool sysP0, bool sysQ0, int vbP, int vbQ,
-                             int kP, int kQ,
-                             f32x4* H, size_t hs) {
+                             int kP, int kQ, const History& H) {
   const V3 vq0 = v3(L.verts[vbQ]), vp0 = v3(L.verts[vbP]);
   const V3 Pq = sysQ0 ? vq0 : t_apply(tq, vq0);
   const V3 Pp = sysP0 ? vp0 : t_apply(tp, vp0);
@@ -1816,7 +1834,7 @@ __device__ int sva_pair_full(const Lds& L, const T12& tp, const T12& tq, bool sy
     normalize3(r);
     const float dp = dot3(S, r);
     if (dp >= -kEpsBelow) return 0;
-    const int code = sva_slow(H, hs, k, l, (p - vbP) | ((q - vbQ) << 16), r, dp, S, w);
+    const int code = sva_slow(H, k, l, (p - vbP) | ((q - vbQ) << 16), r, dp, S, w);
     if (code != 0) return code;
     if (++l >= kMaxIter) return -1;
   }
@@ -1828,8 +1846,8 @@ __global__ void __launch_bounds__(BLOCK) point_small_kernel(SceneImg img, DevRob
   // dynamic LDS: the scene image, the frames, the lanes' iteration history
   const Lds L = stage_scene<BLOCK>(img, smem);
   T12* frames = reinterpret_cast<T12*>(reinterpret_cast<char*>(smem) + img.bytes);
-  f32x4* H = reinterpret_cast<f32x4*>(reinterpret_cast<char*>(smem) + img.bytes + sizeof(T12) * kMaxDofDev) +
-              threadIdx.x;
+  f32x4* const lh = reinterpret_cast<f32x4*>(reinterpret_cast<char*>(smem) + img.bytes + sizeof(T12) * kMaxDofDev);
+  const History H{lh + threadIdx.x, kMaxIter, BLOCK, nullptr};
   __shared__ int s_word;
   const float* q = qs.q[blockIdx.x];
   if (threadIdx.x == 0) {
@@ -1853,7 +1871,7 @@ __global__ void __launch_bounds__(BLOCK) point_small_kernel(SceneImg img, DevRob
       if (sP != 0) tp = frames[sP - 1];
       if (sQ != 0) tq = frames[sQ - 1];
       const int code = sva_pair_full(L, tp, tq, sP == 0, sQ == 0, pd.x & 0xffff, (int)((unsigned)pd.x >> 16),
-                                     pd.w & 0xffff, (int)((unsigned)pd.w >> 16), H, BLOCK);
+                                     pd.w & 0xffff, (int)((unsigned)pd.w >> 16), H);
       if (code != 0) atomicMin(&s_word, ((crs + 1) << 4) | (code + 1));
     }
   }
@@ -2008,22 +2026,39 @@ static const void* sva_multi_variant(int edge_mode, int block, int waves) {
   return nullptr;
 }
 
+// LDS is handed out in granules; of a block's last one 64 bytes are left for
+// the kernels' static variables.
+constexpr size_t kLdsGranule = 1280, kLdsStatic = 64;
+
+// The history entries per lane that fit into LDS beside `lds` other bytes of
+// each block, with as many blocks per CU as a launch of sh.grid blocks needs
+// at once: none of them waits for another's LDS.
+static int history_entries(const SvaShape& sh, size_t lds) {
+  if (sh.cus < 1 || sh.grid < 1) return 0;
+  const size_t per_cu = (size_t)((sh.grid + sh.cus - 1) / sh.cus);
+  const size_t room = (size_t)sva_max_lds_bytes() / kLdsGranule / per_cu * kLdsGranule;
+  if (room < lds + kLdsStatic) return 0;
+  return (int)std::min<size_t>(kMaxIter, (room - lds - kLdsStatic) / (sizeof(float4) * (size_t)sh.block));
+}
+static size_t history_lds(int entries, int block) { return sizeof(float4) * (size_t)entries * (size_t)block; }
+
 // Resident blocks over all CUs of a kernel variant with lds dynamic bytes.
-static hipError_t resident_grid(const void* const fns[2], int block, size_t lds, int device, int* grid) {
-  int cus = 0, blocks = 0;
-  hipError_t e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device);
+static hipError_t resident_grid(const void* const fns[2], int block, size_t lds, int device, int* grid, int* cus) {
+  int blocks = 0;
+  hipError_t e = hipDeviceGetAttribute(cus, hipDeviceAttributeMultiprocessorCount, device);
   if (e != hipSuccess) return e;
-  // the occupancy query sees the dynamic LDS only once the attribute allows it
+  // the occupancy query sees the dynamic LDS only once the attribute allows
+  // it, and small launches add history entries up to all of a CU's
+  const size_t most = std::max(lds, (size_t)sva_max_lds_bytes() - kLdsStatic);
   for (int em = 0; em < 2; ++em) {
     if (!fns[em]) return hipErrorInvalidValue;
-    if (lds > 64 * 1024 &&
-        (e = hipFuncSetAttribute(fns[em], hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)) != hipSuccess)
+    if ((e = hipFuncSetAttribute(fns[em], hipFuncAttributeMaxDynamicSharedMemorySize, (int)most)) != hipSuccess)
       return e;
   }
   e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, fns[1], block, lds);
   if (e != hipSuccess) return e;
   if (blocks < 1) return hipErrorInvalidConfiguration;
-  *grid = cus * blocks;
+  *grid = *cus * blocks;
   return hipSuccess;
 }
 
@@ -2032,7 +2067,7 @@ hipError_t sva_multi_shape_finish(size_t img_bytes, SvaShape* sh, int device) {
   if (lds > (size_t)sva_max_lds_bytes() - 16) return hipErrorInvalidValue;
   if (sh->ppu < 1 || sh->ppu > 256) return hipErrorInvalidValue;
   const void* fns[2] = {sva_multi_variant(0, sh->block, sh->waves), sva_multi_variant(1, sh->block, sh->waves)};
-  return resident_grid(fns, sh->block, lds, device, &sh->grid);
+  return resident_grid(fns, sh->block, lds, device, &sh->grid, &sh->cus);
 }
 
 hipError_t sva_shape_finish(const SceneImg& img, SvaShape* sh, int device) {
@@ -2042,7 +2077,7 @@ hipError_t sva_shape_finish(const SceneImg& img, SvaShape* sh, int device) {
   if (sh->ppu < 1 || sh->ppu > 256) return hipErrorInvalidValue;
   const void* fns[2] = {sva_variant(0, sh->block, sh->waves, sh->gscene),
                         sva_variant(1, sh->block, sh->waves, sh->gscene)};
-  return resident_grid(fns, sh->block, lds, device, &sh->grid);
+  return resident_grid(fns, sh->block, lds, device, &sh->grid, &sh->cus);
 }
 
 SvaShape sva_default_shape(const SceneImg& img) {
@@ -2072,11 +2107,14 @@ SvaShape sva_default_shape(const SceneImg& img) {
 }
 
 hipError_t launch_sva(const SvaArgs& a, int edge_mode, const SvaShape& sh, hipStream_t st) {
-  const size_t lds = sva_lds_bytes(a.img, sh.block, sh.gscene);
+  size_t lds = sva_lds_bytes(a.img, sh.block, sh.gscene);
   if (lds > (size_t)sva_max_lds_bytes() || a.hist == nullptr || sh.grid < 1) return hipErrorInvalidValue;
   const void* fn = sva_variant(edge_mode, sh.block, sh.waves, sh.gscene);
   if (!fn) return hipErrorInvalidValue;
-  void* args[] = {const_cast<SvaArgs*>(&a)};
+  SvaArgs b = a;
+  b.lds_hist = history_entries(sh, lds);
+  lds += history_lds(b.lds_hist, sh.block);
+  void* args[] = {&b};
   return hipLaunchKernel(fn, dim3(sh.grid), dim3(sh.block), args, lds, st);
 }
 
@@ -2118,7 +2156,9 @@ hipError_t launch_sva_multi(const SceneTask* d_tasks, int ntasks, int edge_mode,
   if (lds > (size_t)sva_max_lds_bytes() - 16 || sh.grid < 1) return hipErrorInvalidValue;
   const void* fn = sva_multi_variant(edge_mode, sh.block, sh.waves);
   if (!fn) return hipErrorInvalidValue;
-  void* args[] = {const_cast<SceneTask**>(&d_tasks), &ntasks, &t_start, &tally};
+  int entries = history_entries(sh, lds);
+  lds += history_lds(entries, sh.block);
+  void* args[] = {const_cast<SceneTask**>(&d_tasks), &ntasks, &t_start, &tally, &entries};
   return hipLaunchKernel(fn, dim3(sh.grid), dim3(sh.block), args, lds, st);
 }
 

@@ -90,7 +90,8 @@ struct SvaArgs {
   const float* frames;     // link frames, link-major and quad-planar: float4 j (0..2) of
                            // link s (1..ndof) of item i at frames4[((s-1) 3 + j) fstride + i]
   long long fstride;       // item stride of frames (n of the kinematics launch, or its cap)
-  float4* hist;            // [kMaxIter][grid*block] per-lane iteration history
+  float4* hist;            // per-lane iteration history, kMaxIter entries for each of grid*block lanes
+  int lds_hist;            // the first entries, which are in LDS instead (set by the launcher)
   int nitems;              // item count, or -1: read *nitems_dev
   const int* nitems_dev;
   // edge mode: the pairs that some item of a group of 64 needs tested,
@@ -423,6 +424,7 @@ struct SvaShape {
   int ppu = 32;
   int grid = 0;
   int gscene = 0;  // 1: the kernel reads the scene from the global image (beyond LDS)
+  int cus = 0;     // the device's compute units
 };
 // Variants: (256, 5), (256, 4), (1024, 4), each with the scene in LDS or,
 // when the image and the block's rings do not fit, read from the global
