@@ -133,6 +133,7 @@ struct gprm_ctx {
   gprm::DevBuf img_buf;
   gprm::SceneImg img{};
   gprm::SvaShape shape;
+  gprm::SvaShape shape_few;  // small point launches' instead (grid 0: none)
   std::vector<std::unique_ptr<gprm::Slot>> slots;
   std::map<int, int> requests;  // request id -> slot index
   int next_request = 0;

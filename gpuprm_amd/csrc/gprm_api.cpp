@@ -456,23 +456,42 @@ int prof_fold_tally(gprm_ctx* c, Slot& sl) {
 }  // namespace
 
 // Pairs per work unit of a launch over about n items: the shape's, or fewer
-// so that there are at least two units (chunk x 64-item group) per resident
-// wave; never below 8.
-int unit_pairs(const gprm_ctx* c, long long n) {
-  const long long waves = (long long)c->shape.grid * (c->shape.block / 64);
+// so that there are at least `per_wave` units (chunk x 64-item group) per
+// resident wave; never below 8.
+static int unit_pairs(const gprm_ctx* c, const SvaShape& sh, long long n, int per_wave) {
+  const long long waves = (long long)sh.grid * (sh.block / 64);
   const long long groups = std::max(1LL, (n + 63) / 64);
-  long long want = groups * c->img.M / std::max(1LL, 2 * waves);
-  want = std::max(8LL, std::min((long long)c->shape.ppu, want));
+  long long want = groups * c->img.M / std::max(1LL, per_wave * waves);
+  want = std::max(8LL, std::min((long long)sh.ppu, want));
   return (int)want;
 }
+int unit_pairs(const gprm_ctx* c, long long n) { return unit_pairs(c, c->shape, n, 2); }
 
-// The context's shape with the grid cut to the blocks a launch of `units`
-// work units can use (small launches then dispatch and stage fewer blocks).
-SvaShape launch_shape(const gprm_ctx* c, long long units) {
-  SvaShape sh = c->shape;
+// The shape with the grid cut to the blocks a launch of `units` work units
+// can use (small launches then dispatch and stage fewer blocks).
+static SvaShape launch_shape(SvaShape sh, long long units) {
   const long long per_block = std::max(1, sh.block / 64);
   const long long need = std::max(1LL, (units + per_block - 1) / per_block);
   if (need < sh.grid) sh.grid = (int)need;
+  return sh;
+}
+SvaShape launch_shape(const gprm_ctx* c, long long units) { return launch_shape(c->shape, units); }
+
+// Point checks of n items: the launch's shape before that cut and the pairs
+// of a unit.  While a wave would walk at most kFewPairs pairs, nearly all of
+// the launch is the waves' last full tests, as many chains of iterations as
+// waves; four waves per SIMD then do with fewer of them, and have more of the
+// history in LDS (65,536 points of the 4-DOF scene 75 -> 70 us, 16,384 of the
+// 7-DOF scene 91 -> 84; beyond, 98,304 of the latter 145 -> 150).  From
+// kManyPairs on the units are dealt out in six rounds instead of two, which
+// could be 3.2 taken as four (524,288 points of the 7-DOF scene 500 -> 460 us,
+// 1M of the 6-DOF scene 704 -> 621; at 170 pairs a wave 331 -> 349).
+static SvaShape point_shape(const gprm_ctx* c, long long n, int* unit) {
+  constexpr long long kFewPairs = 24, kManyPairs = 200;
+  const long long pairs = std::max(1LL, (n + 63) / 64) * c->img.M;
+  const long long waves = (long long)c->shape.grid * (c->shape.block / 64);
+  const SvaShape& sh = c->shape_few.grid > 0 && pairs <= kFewPairs * waves ? c->shape_few : c->shape;
+  *unit = unit_pairs(c, sh, n, pairs >= kManyPairs * waves ? 6 : 2);
   return sh;
 }
 
@@ -543,7 +562,7 @@ int run_points(gprm_ctx* c, Slot& sl, const float* d_q, long long offset, int n,
     a.hist = sl.hist.as<float4>();
     a.nitems = cn;
     a.counter = sl.queues.as<unsigned>() + (size_t)kSvaCounters * ci;
-    a.pairs_per_unit = unit_pairs(c, cn);
+    const SvaShape shape = point_shape(c, cn, &a.pairs_per_unit);
     a.units_per_item = (c->img.M + a.pairs_per_unit - 1) / a.pairs_per_unit;
     a.word = sl.status.as<int>();
     // the separating-vector launch writes the codes (no finalize launch)
@@ -552,7 +571,7 @@ int run_points(gprm_ctx* c, Slot& sl, const float* d_q, long long offset, int n,
     a.tally = tally_ptr(c, sl);
     a.static_first = 1;
     GPRM_HIP(prof_begin(c, sl, 0, st, &ev), "event");
-    GPRM_HIP(launch_sva(a, 0, launch_shape(c, (long long)((cn + 63) / 64) * a.units_per_item), st),
+    GPRM_HIP(launch_sva(a, 0, launch_shape(shape, (long long)((cn + 63) / 64) * a.units_per_item), st),
              "separating-vector launch");
     GPRM_HIP(prof_end(c, sl, ev, st), "event");
   }
@@ -947,6 +966,12 @@ int gprm_init(gprm_ctx* c, int rank, int size) {
   c->img.blob = c->img_buf.as<int4>();
   c->shape = sva_default_shape(c->img);
   GPRM_HIP(sva_shape_finish(c->img, &c->shape, c->device), "separating-vector launch shape");
+  c->shape_few = SvaShape{};
+  if (c->shape.waves == 5 && !c->shape.gscene) {
+    SvaShape few = c->shape;
+    few.waves = 4;
+    if (sva_shape_finish(c->img, &few, c->device) == hipSuccess && few.grid <= c->shape.grid) c->shape_few = few;
+  }
   c->small_calls = point_small_prepare(c->img) == hipSuccess;
   c->inited = true;
   return GPRM_OK;
@@ -1222,6 +1247,7 @@ int gprm_set_launch_shape(gprm_ctx* c, const gprm_launch_shape* in) {
   if (e != hipSuccess) return hip_fail(c, e, "launch shape");
   std::lock_guard<std::mutex> lk(c->mu);
   c->shape = sh;
+  c->shape_few = SvaShape{};  // the caller's shape holds for every launch
   return GPRM_OK;
 }
 
