@@ -1789,23 +1789,33 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVE
 // One block per configuration of a call of at most kSmallMax: the
 // configurations come as kernel arguments and the codes go straight to
 // (pinned host) memory, so a call is one launch and one synchronisation.
-// Thread 0 computes the frames into LDS; the threads then run the full
+// The first wave computes the frames into LDS; the threads then run the full
 // separating-vector test on the pairs t, t + BLOCK, ... (no bound test: it
 // only shortcuts pair tests that end separated), skipping pairs later in
 // CRS order than a collision already found, and the block keeps the first
 // colliding pair's code, as the batched kernels do.
 
 // Frames 1..ndof of one configuration (kinematics.h:27-37), the same
-// operations as fk_store.
+// operations as fk_store, by the block's first wave: lane i the joint's own
+// transformation into out[i] (its sine and cosine are the long part; with one
+// lane computing all in turn a call on the 4-DOF scene took 30.4 us, 29.4 so),
+// then lane 0 the chain.
 __device__ void fk_frames(const DevRobot& rb, const float* q, T12* out) {
-  T12 T = t_base(rb);
-  for (int i = 0; i < rb.ndof; ++i) {
-    float qset = rb.q[i], dset = rb.d[i];
-    if (rb.types[i] == 0) qset = q[i];
-    else dset = q[i];
-    const T12 A = t_set_cs(rb.a[i], rb.ca[i], rb.sa[i], qset, dset);
-    T = t_lapply(A, T);
-    out[i] = T;
+  const int lane = threadIdx.x;
+  if (lane < rb.ndof) {
+    const bool turns = rb.types[lane] == 0;
+    out[lane] = t_set_cs(rb.a[lane], rb.ca[lane], rb.sa[lane], turns ? q[lane] : rb.q[lane],
+                         turns ? rb.d[lane] : q[lane]);
+  }
+  // the entries were written by other lanes of this wave
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  if (lane == 0) {
+    T12 T = t_base(rb);
+    for (int i = 0; i < rb.ndof; ++i) {
+      T = t_lapply(out[i], T);
+      out[i] = T;
+    }
   }
 }
 
@@ -1850,12 +1860,12 @@ __global__ void __launch_bounds__(BLOCK) point_small_kernel(SceneImg img, DevRob
   const History H{lh + threadIdx.x, kMaxIter, BLOCK, nullptr};
   __shared__ int s_word;
   const float* q = qs.q[blockIdx.x];
-  if (threadIdx.x == 0) {
+  if (threadIdx.x < 64) {
     // check_boundaries(q) (robotconfigspace.cpp:795-802)
-    int ob = 0;
-    for (int j = 0; j < rb.ndof; ++j)
-      if (q[j] < rb.mins[j] || q[j] > rb.maxs[j]) { ob = 1; break; }
-    s_word = ob ? kWordOutOfBounds : kWordFree;
+    const int j = threadIdx.x;
+    const bool out_of = j < rb.ndof && (q[j] < rb.mins[j] || q[j] > rb.maxs[j]);
+    const bool ob = __ballot(out_of) != 0ull;
+    if (j == 0) s_word = ob ? kWordOutOfBounds : kWordFree;
     if (!ob) fk_frames(rb, q, frames);
   }
   __syncthreads();
