@@ -5,7 +5,7 @@
 // into a device image that the separating-vector kernel stages in LDS.  Work
 // is split into chunks of at most kItemBudget configurations, each chunk
 // being one kinematics launch and one persistent separating-vector launch.
-// Edge queries run in rounds of growing sample windows; after every round the
+// Edge queries run in rounds of ever finer samples (edge_levels); after every round the
 // samples of edges that are already blocked are no longer scheduled.
 #include <hip/hip_runtime.h>
 

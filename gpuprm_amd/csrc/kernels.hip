@@ -2,13 +2,16 @@
 //
 //   fk_points / fk_edges : forward kinematics, one lane per configuration,
 //                          frames kept in VGPRs and written once to HBM.
-//   sva                  : persistent separating-vector kernel; the scene is
-//                          staged in LDS, every lane is an independent worker
-//                          that steps one iteration of the Chung-Wang test per
-//                          trip and refills itself from a wave-level work queue
-//                          (ballot + one atomic per 64 items).
-//   edge_prologue/compact: edge sample counts, sample order, and per-round
-//                          compaction of the samples of still-open edges.
+//                          fk_edges also marks, per group of 64 samples, the
+//                          pairs that bounds over the group leave open.
+//   sva                  : persistent separating-vector kernel; a wave walks
+//                          pairs over 64 items with a bound test (pair operands
+//                          in scalar registers) and puts what that leaves
+//                          open into a ring in LDS, whose pairs its lanes then
+//                          take one each through the Chung-Wang test (the
+//                          scene's vertices and adjacency in LDS).
+//   edge_prologue/compact: edge sample counts, and per-window compaction of
+//                          the samples of still-open edges.
 //
 // Arithmetic follows the reference's host path operation by operation:
 // the file is compiled with -ffp-contract=off (no FMA contraction), IEEE
@@ -1940,8 +1943,8 @@ __global__ void finalize_points_multi_kernel(const FkTask* __restrict__ tasks, i
 // launchers
 // ----------------------------------------------------------------------------
 
-// Dynamic LDS of a separating-vector block: the deferral rings (16 B per
-// thread) and the scene image.
+// Dynamic LDS of a separating-vector block without its history entries: the
+// deferral rings and the scene image.
 size_t sva_lds_bytes(const SceneImg& img, int block, int gscene) {
   return (gscene ? 0 : (size_t)img.bytes) + sva_ring_bytes(block);
 }
