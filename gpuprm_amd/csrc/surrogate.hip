@@ -317,8 +317,9 @@ __device__ __forceinline__ void stage_inputs(const float* __restrict__ q, long l
 // BF16 like the others) with w4, the waves leave their rows' sums in LDS, and
 // one wave adds the eight of a row in the next pair's first steps.  Reading
 // the activations back for that had taken a quarter of the kernel's time.
-// 1M rows: 500 us with one tile in flight, 368 us so; up to 16,384 rows (one
-// tile per block, the steps of B only barriers) 29 us either way.
+// 1M rows: 500 us with one tile in flight, 368 us so; 49,152 rows 44 and 40 us.
+// Up to 16,384 rows, one tile per block, 27.3 and 25.2 us for 64 rows,
+// 29.1 and 27.7 for 16,384.
 // LDS: four activation tiles, the staged inputs of A and B, b1 | b2 | b3 | w4,
 // the head's sums.
 constexpr size_t kPredictLds = 4 * (size_t)kTileElems * 2 + 2 * (size_t)kFR * kXP * 2 + 4 * kH * sizeof(float) +
@@ -372,7 +373,9 @@ __global__ void __launch_bounds__(kPW * 64) __attribute__((amdgpu_waves_per_eu(2
   const long long stride = (long long)gridDim.x * kFR;
   long long r0 = (long long)blockIdx.x * kFR;  // tile A's first row, tile B's is r0 + stride
   stage_inputs(q, off, r0, n, nd, xs, nullptr, 0, tid);
-  stage_inputs(q, off, r0 + stride, n, nd, xs + kFR * kXP, nullptr, 0, tid);
+  // a block with one tile in all takes tile A's steps alone, all waves in step
+  const bool two = r0 + stride < n;
+  if (two) stage_inputs(q, off, r0 + stride, n, nd, xs + kFR * kXP, nullptr, 0, tid);
   // the weights last: loads arrive in order, and layer 1 need not wait for
   // those of layers 2 and 3
   const float bias4 = P[kOffB4];
@@ -380,7 +383,7 @@ __global__ void __launch_bounds__(kPW * 64) __attribute__((amdgpu_waves_per_eu(2
   load_frags(W2h, w2, wave, lane);
   load_frags(W3h, w3, wave, lane);
   __syncthreads();
-  const bool late = wave >= kPW / 2;
+  const bool late = two && wave >= kPW / 2;
   if (late) __syncthreads();
   long long before = -1;  // the pair whose heads are due (its tile A), none at first
   for (;; r0 += 2 * stride) {
@@ -389,6 +392,7 @@ __global__ void __launch_bounds__(kPW * 64) __attribute__((amdgpu_waves_per_eu(2
     float next[2][kStage];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
+      if (t == 1 && !two) break;
       const long long rt = r0 + t * stride;
       // the previous pair's probabilities, by one of the early waves
       if (wave == t && before >= 0) {
@@ -410,6 +414,7 @@ __global__ void __launch_bounds__(kPW * 64) __attribute__((amdgpu_waves_per_eu(2
     if (!on) break;
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
+      if (t == 1 && !two) break;
       f32x4 acc[kPJ][4];
       const bool run = r0 + t * stride < n;
       // both halves' layer 1 has read this pair's inputs
@@ -421,6 +426,7 @@ __global__ void __launch_bounds__(kPW * 64) __attribute__((amdgpu_waves_per_eu(2
     }
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
+      if (t == 1 && !two) break;
       f32x4 acc[kPJ][4];
       const bool run = r0 + t * stride < n;
       if (run) layer_mfma(hs + (size_t)(2 + t) * kTileElems, w3, acc, lane);
@@ -430,7 +436,7 @@ __global__ void __launch_bounds__(kPW * 64) __attribute__((amdgpu_waves_per_eu(2
     }
     before = r0;
   }
-  if (!late) __syncthreads();
+  if (two && !late) __syncthreads();
 }
 
 // ---- training ------------------------------------------------------------------
