@@ -24,7 +24,7 @@
 // step and one persistent separating-vector launch per bucket.  Steps walk
 // the windows of sample levels (edge_levels), shared by all scenes; a
 // window whose items exceed a scene's per-step budget takes several steps,
-// each over a range of that scene's edges.  The steps after the prologue
+// each over a range of that scene's edges (or of one long edge's samples).  The steps after the prologue
 // are what a hipGraph captures; the graph is kept while the arrays, sizes
 // and the per-scene largest testnums stay the same.
 #include <hip/hip_runtime.h>
@@ -412,26 +412,22 @@ int edge_plan(gprm_batch* b, const EdgeSignature& sg, const std::vector<int>& ma
   std::vector<int> budget(S), cap(S, 0);
   for (int s = 0; s < S; ++s)
     budget[s] = std::max(1, std::min(kEdgeStepItems, 0x7fffffff / std::max(1, b->ctx[s]->img.M)));
-  struct Part { int s, e0, e1, l0, l1, cap; };
+  struct Part { int s; EdgeLaunch l; };
   std::vector<std::vector<Part>> steps;
   for (const auto& w : edge_windows(gmax)) {
-    std::vector<int> per(S, 0), nch(S, 0);
-    int nsteps = 0;
+    std::vector<std::vector<EdgeLaunch>> of(S);
+    size_t nsteps = 0;
     for (int s = 0; s < S; ++s) {
       if (sg.n[s] == 0 || edge_levels(maxT[s]) <= w.first) continue;
-      per[s] = std::max(1, (budget[s] - 64) / (edge_run_slots(edge_window_most(maxT[s], w.first, w.second)) + 1));
-      nch[s] = (sg.n[s] + per[s] - 1) / per[s];
-      nsteps = std::max(nsteps, nch[s]);
+      edge_plan_window(budget[s], kCompactBlockMulti, sg.n[s], w.first, w.second, maxT[s], -1, &of[s]);
+      nsteps = std::max(nsteps, of[s].size());
     }
-    for (int j = 0; j < nsteps; ++j) {
+    for (size_t j = 0; j < nsteps; ++j) {
       std::vector<Part> parts;
       for (int s = 0; s < S; ++s) {
-        if (j >= nch[s]) continue;
-        const int e0 = j * per[s], e1 = std::min(sg.n[s], e0 + per[s]);
-        const long long c = frame_stride(
-            edge_items_cap(e1 - e0, edge_window_most(maxT[s], w.first, w.second), kCompactBlockMulti));
-        parts.push_back({s, e0, e1, w.first, w.second, (int)c});
-        cap[s] = std::max(cap[s], (int)c);
+        if (j >= of[s].size()) continue;
+        parts.push_back({s, of[s][j]});
+        cap[s] = std::max(cap[s], of[s][j].cap);
       }
       steps.push_back(std::move(parts));
     }
@@ -479,21 +475,23 @@ int edge_plan(gprm_batch* b, const EdgeSignature& sg, const std::vector<int>& ma
       t.ea = edge_args(b, sg, s);
       t.rb = c->rb;
       t.dq = c->dq;
-      t.e0 = pt.e0;
-      t.e1 = pt.e1;
-      t.l0 = pt.l0;
-      t.l1 = pt.l1;
+      t.e0 = pt.l.e0;
+      t.e1 = pt.l.e1;
+      t.l0 = pt.l.l0;
+      t.l1 = pt.l.l1;
+      t.r0 = pt.l.r0;
+      t.r1 = pt.l.r1;
       t.item_edge = items + ibase[s];
       t.item_pos = items + icap + ibase[s];
       t.nitems = ctl;
-      t.cap = pt.cap;
+      t.cap = pt.l.cap;
       t.frames = b->e_frames.as<float>() + (size_t)12 * nd * ibase[s];
       t.img = c->img;
       t.mask = scene_masks(b, s) ? b->e_masks.as<unsigned long long>() + mbase[s] : nullptr;
       t.block0 = cb;
       t.fblock0 = fb;
-      cb += (pt.e1 - pt.e0 + kCompactBlockMulti - 1) / kCompactBlockMulti;
-      fb += (pt.cap + kFkBlock - 1) / kFkBlock;
+      cb += (pt.l.e1 - pt.l.e0 + kCompactBlockMulti - 1) / kCompactBlockMulti;
+      fb += (pt.l.cap + kFkBlock - 1) / kFkBlock;
       step->tasks.push_back(t);
       step->scene.push_back(s);
       const Bucket& bk = b->buckets[bucket_of[s]];
@@ -501,7 +499,7 @@ int edge_plan(gprm_batch* b, const EdgeSignature& sg, const std::vector<int>& ma
       q.a.img = c->img;
       q.a.ndof = nd;
       q.a.frames = t.frames;
-      q.a.fstride = pt.cap;
+      q.a.fstride = pt.l.cap;
       q.a.mask = t.mask;
       q.a.hist = b->hist.as<float4>();
       q.a.nitems = -1;

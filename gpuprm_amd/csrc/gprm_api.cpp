@@ -521,16 +521,10 @@ size_t mask_bytes(const gprm_ctx* c, long long n) {
   return sizeof(unsigned long long) * (size_t)mask_words(c->img.M) * (size_t)((n + 63) / 64);
 }
 
-// One launch of an edge call: levels [l0, l1) of edges [e0, e1), at most cap
-// items (a multiple of 64, also the frames' plane stride).
-struct EdgeLaunch {
-  int e0, e1, l0, l1, cap;
-};
-
-// The launches of a window over N edges of at most maxT samples, total in
-// all (-1: unknown), each of at most item_budget items unless a single edge
-// has more.
-void plan_window(const gprm_ctx* c, int N, int l0, int l1, int maxT, long long total, std::vector<EdgeLaunch>* plan);
+// The launches of a window (edge_plan_window) with the context's item budget.
+void plan_window(const gprm_ctx* c, int N, int l0, int l1, int maxT, long long total, std::vector<EdgeLaunch>* plan) {
+  edge_plan_window(item_budget(c), kCompactBlock, N, l0, l1, maxT, total, plan);
+}
 
 // Point checks of n items on the device (q SoA with offset, res[n]).
 int run_points(gprm_ctx* c, Slot& sl, const float* d_q, long long offset, int n, int* d_res,
@@ -578,23 +572,6 @@ int run_points(gprm_ctx* c, Slot& sl, const float* d_q, long long offset, int n,
   return GPRM_OK;
 }
 
-
-void plan_window(const gprm_ctx* c, int N, int l0, int l1, int maxT, long long total, std::vector<EdgeLaunch>* plan) {
-  const int most = edge_window_most(maxT, l0, l1);
-  const long long budget = item_budget(c);
-  long long cap = edge_items_cap(N, most, kCompactBlock);
-  if (total >= 0)  // every run padded by at most 15
-    cap = std::min(cap, total + 15LL * N + 16LL * ((N + kCompactBlock - 1) / kCompactBlock));
-  if (cap <= budget) {
-    plan->push_back({0, N, l0, l1, (int)frame_stride(cap)});
-    return;
-  }
-  const int per = (int)std::max(1LL, (budget - 64) / (edge_run_slots(most) + 1));
-  for (int e0 = 0; e0 < N; e0 += per) {
-    const int e1 = std::min(N, e0 + per);
-    plan->push_back({e0, e1, l0, l1, (int)frame_stride(edge_items_cap(e1 - e0, most, kCompactBlock))});
-  }
-}
 
 // Edge checks on the device.  testnum and res are computed by the prologue
 // kernel; the largest testnum and the samples in all (host_maxT, host_total,
@@ -703,8 +680,7 @@ int run_edges(gprm_ctx* c, Slot& sl, const float* d_qs, const float* d_qe, long 
       float* frames = set_frames(i).as<float>();
       unsigned* queues = sl.queues.as<unsigned>() + (size_t)kSvaCounters * i;  // zeroed by the compaction
       unsigned long long* mask = use_masks(c, p.cap) ? set_mask(i).as<unsigned long long>() : nullptr;
-      GPRM_HIP(launch_edge_compact(ea, p.e0, p.e1, p.l0, p.l1, items_e, items_p, p.cap, cnt, cnt + 1,
-                                   queues, ps),
+      GPRM_HIP(launch_edge_compact(ea, p, items_e, items_p, cnt, cnt + 1, queues, ps),
                "edge compaction launch");
       size_t ev = 0;
       GPRM_HIP(prof_begin(c, sl, 1, ps, &ev), "event");

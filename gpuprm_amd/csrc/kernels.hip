@@ -516,7 +516,7 @@ __global__ void __launch_bounds__(1024)
   edge_prologue_one<1024>(ndof, dq, ea, blockIdx.x * 1024 + threadIdx.x, testnum, max_testnum, total);
 }
 
-// Items for levels [l0, l1) of every open edge in [e0, e1), an edge's samples
+// Items for ranks [r0, r1) in the window [l0, l1) of every open edge, an edge's samples
 // in ascending order on consecutive slots.  Runs of more than kRunShort
 // samples start at a multiple of 16 and are padded to one (edge_run_slots);
 // the block's short runs follow them packed, padded together.  Padding items
@@ -527,15 +527,16 @@ __global__ void __launch_bounds__(1024)
 // each lane's slots follow by prefix count.  Every thread of the block calls
 // it; threads with e >= e1 contribute nothing.
 template <int BLOCK>
-__device__ __forceinline__ void edge_compact_one(const EdgeArgs& ea, int e, int e1, int l0, int l1,
+__device__ __forceinline__ void edge_compact_one(const EdgeArgs& ea, int e, int e1, int l0, int l1, int r0, int r1,
                                                  int* __restrict__ item_edge, int* __restrict__ item_pos, int cap,
                                                  int* __restrict__ nitems, int* __restrict__ nsamples) {
   int a = 1, b = 0, cnt = 0;
   if (e < e1 && __hip_atomic_load(&ea.edge_res[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
     edge_window(ea.testnum[e], l0, l1, &a, &b, &cnt);
+  cnt = max(min(cnt, r1) - r0, 0);
   const bool is_short = cnt <= kRunShort;
   // prefix sums of the long runs' slots, the short runs' and the samples
-  int lng = is_short ? 0 : edge_run_slots(cnt), shr = is_short ? cnt : 0, smp = cnt;
+  int lng = is_short ? 0 : (int)edge_run_slots(cnt), shr = is_short ? cnt : 0, smp = cnt;
   const int slots = lng;
   const int lane = threadIdx.x & 63;
   for (int d = 1; d < 64; d <<= 1) {
@@ -594,18 +595,17 @@ __device__ __forceinline__ void edge_compact_one(const EdgeArgs& ea, int e, int 
     if (src < 0) continue;
     for (int t = col; t < f && os + t < cap; t += 16) {
       item_edge[os + t] = t < c ? es : es | kItemPad;
-      item_pos[os + t] = edge_window_sample(as, bs, t < c ? t : c - 1);
+      item_pos[os + t] = edge_window_sample(as, bs, r0 + (t < c ? t : c - 1));
     }
   }
 }
 
 __global__ void __launch_bounds__(kCompactBlock)
-    edge_compact_kernel(EdgeArgs ea, int e0, int e1, int l0, int l1, int* __restrict__ item_edge,
-                        int* __restrict__ item_pos, int cap, int* __restrict__ nitems, int* __restrict__ nsamples,
-                        unsigned* __restrict__ zero_queues) {
+    edge_compact_kernel(EdgeArgs ea, EdgeLaunch p, int* __restrict__ item_edge, int* __restrict__ item_pos,
+                        int* __restrict__ nitems, int* __restrict__ nsamples, unsigned* __restrict__ zero_queues) {
   if (blockIdx.x == 0 && threadIdx.x < kSvaQueues) zero_queues[threadIdx.x * kSvaQueueStride] = 0u;
-  edge_compact_one<kCompactBlock>(ea, e0 + blockIdx.x * kCompactBlock + threadIdx.x, e1, l0, l1, item_edge, item_pos,
-                                  cap, nitems, nsamples);
+  edge_compact_one<kCompactBlock>(ea, p.e0 + blockIdx.x * kCompactBlock + threadIdx.x, p.e1, p.l0, p.l1, p.r0, p.r1,
+                                  item_edge, item_pos, p.cap, nitems, nsamples);
 }
 
 // Multi-scene edge calls: one task per scene (prologue) or per scene part of
@@ -634,7 +634,7 @@ __global__ void __launch_bounds__(kCompactBlockMulti)
     edge_compact_multi_kernel(const EdgeTask* __restrict__ tasks, int ntasks) {
   const EdgeTask& T = edge_task_of<false>(tasks, ntasks);
   edge_compact_one<kCompactBlockMulti>(T.ea, T.e0 + (blockIdx.x - T.block0) * kCompactBlockMulti + threadIdx.x, T.e1,
-                                       T.l0, T.l1, T.item_edge, T.item_pos, T.cap, T.nitems, nullptr);
+                                       T.l0, T.l1, T.r0, T.r1, T.item_edge, T.item_pos, T.cap, T.nitems, nullptr);
 }
 
 template <int NDOF>
@@ -2205,13 +2205,12 @@ hipError_t launch_edge_prologue(const DevRobot& rb, float dq, EdgeArgs ea, int* 
   return hipGetLastError();
 }
 
-hipError_t launch_edge_compact(EdgeArgs ea, int e0, int e1, int l0, int l1, int* item_edge,
-                               int* item_pos, int cap, int* nitems, int* nsamples, unsigned* zero_queues,
-                               hipStream_t st) {
-  if (e1 <= e0) return hipSuccess;
-  dim3 grid((e1 - e0 + kCompactBlock - 1) / kCompactBlock), block(kCompactBlock);
-  hipLaunchKernelGGL(edge_compact_kernel, grid, block, 0, st, ea, e0, e1, l0, l1, item_edge, item_pos, cap,
-                     nitems, nsamples, zero_queues);
+hipError_t launch_edge_compact(EdgeArgs ea, const EdgeLaunch& p, int* item_edge, int* item_pos, int* nitems,
+                               int* nsamples, unsigned* zero_queues, hipStream_t st) {
+  if (p.e1 <= p.e0) return hipSuccess;
+  dim3 grid((p.e1 - p.e0 + kCompactBlock - 1) / kCompactBlock), block(kCompactBlock);
+  hipLaunchKernelGGL(edge_compact_kernel, grid, block, 0, st, ea, p, item_edge, item_pos, nitems, nsamples,
+                     zero_queues);
   return hipGetLastError();
 }
 

@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "edge_plan.h"
+
 namespace gprm {
 
 // Threads per block of the kinematics kernels.  An edge launch's kinematics
@@ -243,73 +245,13 @@ struct EdgeArgs {
   int* edge_res;           // [edge]
 };
 
-// Samples of an edge in launch windows.  The testnum samples of an edge
-// belong to levels: level 0 holds at most 16 evenly spaced ones, each next
-// level fills up a spacing four times finer, the last level the rest:
-// edge_levels(T) levels with spacings m_l, the multiples of m_l that are not
-// multiples of m_(l-1).  A window covers levels [l0, l1) of every edge, in
-// ascending sample order: adjacent items are adjacent samples, whose links
-// stay close together, which is what the pair masks live on; and the first
-// window's spread samples find most blocked edges.  The 6-DOF roadmap
-// (longest edge 209 samples) takes two windows, of 15 and about 105 samples
-// per edge.
-constexpr int kLevelAll = 64;  // l1 of a window that takes every remaining sample
-__host__ __device__ inline int edge_levels(int T) {
-  if (T <= 16) return 1;
-  if (T <= 256) return 2;
-  int n = 3;
-  for (long long lim = 512; T > lim; lim *= 4) ++n;
-  return n;
-}
-// Samples of the window: the multiples of a that are not multiples of b (b =
-// 0: every multiple of a).  count: how many.
-__host__ __device__ inline void edge_window(int T, int l0, int l1, int* a, int* b, int* count) {
-  const int n = edge_levels(T);
-  *a = 1;
-  *b = 0;
-  *count = 0;
-  if (T <= 0 || l0 >= n) return;
-  int fine = 1;  // m_(n-2), and from it the coarser spacings
-  if (n > 1) {
-    const long long cnt = 16LL << (2 * (n - 2));
-    fine = (int)((T + cnt - 1) / cnt);
-  }
-  if (l1 < n) *a = fine << (2 * (n - 1 - l1));
-  if (l0 > 0) *b = fine << (2 * (n - 1 - l0));
-  *count = (int)(((long long)T + *a - 1) / *a) - (*b ? (int)(((long long)T + *b - 1) / *b) : 0);
-}
-// Sample r (ascending) of that window.
-__host__ __device__ inline int edge_window_sample(int a, int b, int r) {
-  if (b == 0) return r * a;
-  const int k = b / a - 1;
-  return a * (r / k * (k + 1) + r % k + 1);
-}
-// Most samples an edge of at most maxT samples has in the window.
-inline int edge_window_most(int maxT, int l0, int l1) {
-  (void)l0;
-  long long lim = l1 == 1 ? 16 : 256;
-  for (int l = 3; l <= l1 && lim < maxT; ++l) lim = l == 3 ? 512 : lim * 4;
-  return (int)(lim < maxT ? lim : maxT);
-}
-// Item slots of an edge with count samples in a window: runs of more than
-// kRunShort samples start at and are padded to multiples of 16 (a row of
-// lanes), so that a row's items are one edge's.
-constexpr int kRunShort = 8;
-__host__ __device__ inline int edge_run_slots(int count) {
-  return count > kRunShort ? (count + 15) / 16 * 16 : count;
-}
-// Item capacity for n edges of at most `most` samples each in blocks of
-// `block` edges (the compaction pads each block's short runs to 16, too).
-inline long long edge_items_cap(long long n, int most, int block) {
-  return n * edge_run_slots(most) + 16 * ((n + block - 1) / block);
-}
 // Padding items carry their edge with this bit.
 constexpr int kItemPad = (int)0x80000000;
 
 // One scene's part of a multi-scene edge call (device memory).  Prologue
 // tasks (one per scene) cover edges [0, ea.nedges) and write testnum, the
 // scene's largest testnum and its sample total; launch-step tasks cover edges
-// [e0, e1) and levels [l0, l1): the compaction appends their items
+// [e0, e1) and ranks [r0, r1) of levels [l0, l1): the compaction appends their items
 // (item_edge, item_pos = sample, *nitems, at most cap) and the kinematics
 // writes their frames (link-major, item stride cap) and pair masks.
 struct EdgeTask {
@@ -319,7 +261,7 @@ struct EdgeTask {
   int* testnum;
   int* max_testnum;
   unsigned long long* total;
-  int e0, e1, l0, l1;
+  int e0, e1, l0, l1, r0, r1;
   int* item_edge;
   int* item_pos;
   int* nitems;
@@ -372,14 +314,15 @@ hipError_t launch_sva_multi(const SceneTask* d_tasks, int ntasks, int edge_mode,
                             unsigned long long* t_start, unsigned long long* tally, hipStream_t st);
 hipError_t launch_edge_prologue(const DevRobot& rb, float dq, EdgeArgs ea, int* testnum_out, int* max_testnum,
                                 unsigned long long* total, hipStream_t st);
-// Items of levels [l0, l1) of the open edges in [e0, e1): item_edge, item_pos
+// Items of ranks [p.r0, p.r1) in the window [p.l0, p.l1) of the open edges in
+// [p.e0, p.e1): item_edge, item_pos
 // (the sample), *nitems slots of which *nsamples (may be null) are no padding.
-// Slots beyond cap (an edge longer than the plan's bound) are not written.
+// Slots beyond p.cap (an edge longer than the plan's bound) are not written.
 // zero_queues: the work counters of the separating-vector launch that
 // follows, set to zero.
 constexpr int kCompactBlock = 1024, kCompactBlockMulti = 256;
-hipError_t launch_edge_compact(EdgeArgs ea, int e0, int e1, int l0, int l1, int* item_edge, int* item_pos,
-                               int cap, int* nitems, int* nsamples, unsigned* zero_queues, hipStream_t st);
+hipError_t launch_edge_compact(EdgeArgs ea, const EdgeLaunch& p, int* item_edge, int* item_pos, int* nitems,
+                               int* nsamples, unsigned* zero_queues, hipStream_t st);
 // Kinematics of the *nitems (<= cap) compacted samples; frames link-major
 // with item stride cap (the plane stride); their pair masks to mask unless
 // it is null.
