@@ -481,6 +481,8 @@ int edge_plan(gprm_batch* b, const EdgeSignature& sg, const std::vector<int>& ma
       t.l1 = pt.l.l1;
       t.r0 = pt.l.r0;
       t.r1 = pt.l.r1;
+      const int xb = (t.e1 - t.e0 + kCompactBlockMulti - 1) / kCompactBlockMulti;
+      t.slice = edge_slice(t.r1 - t.r0, xb);
       t.item_edge = items + ibase[s];
       t.item_pos = items + icap + ibase[s];
       t.nitems = ctl;
@@ -490,7 +492,7 @@ int edge_plan(gprm_batch* b, const EdgeSignature& sg, const std::vector<int>& ma
       t.mask = scene_masks(b, s) ? b->e_masks.as<unsigned long long>() + mbase[s] : nullptr;
       t.block0 = cb;
       t.fblock0 = fb;
-      cb += (pt.l.e1 - pt.l.e0 + kCompactBlockMulti - 1) / kCompactBlockMulti;
+      cb += xb * edge_slices(t.r1 - t.r0, xb);
       fb += (pt.l.cap + kFkBlock - 1) / kFkBlock;
       step->tasks.push_back(t);
       step->scene.push_back(s);

@@ -53,7 +53,7 @@ GPRM_EDGE_HD void edge_window(int T, int l0, int l1, int* a, int* b, int* count)
 GPRM_EDGE_HD int edge_window_sample(int a, int b, int r) {
   if (b == 0) return r * a;
   const int k = b / a - 1;
-  return a * (r / k * (k + 1) + r % k + 1);
+  return a * (r + r / k + 1);
 }
 // Most samples an edge of at most maxT samples has in the window.
 inline int edge_window_most(int maxT, int l1) {
@@ -68,10 +68,34 @@ constexpr int kRunShort = 8;
 GPRM_EDGE_HD long long edge_run_slots(int count) {
   return count > kRunShort ? (count + 15LL) / 16 * 16 : count;
 }
-// Item capacity for n edges of at most `most` samples each in blocks of
-// `block` edges (the compaction pads each block's short runs to 16, too).
-inline long long edge_items_cap(long long n, int most, int block) {
-  return n * edge_run_slots(most) + 16 * ((n + block - 1) / block);
+// A compaction block takes at most edge_slice ranks of each of its edges,
+// further blocks the next slices, because a run is written by 16 lanes: one
+// edge's million samples by one block's row took milliseconds, several times
+// their checks.  A slice is a multiple of 16, so that only an edge's last one
+// is padded.  There are at most kSliceBlocks blocks, or 16 slices where the
+// edges alone are many blocks: those of edges that are blocked or short find
+// nothing to do, but 16,384 of them cost about 15 us.
+constexpr int kSliceLeast = 1024;
+constexpr long long kSliceBlocks = 2048;
+inline int edge_slice(int ranks, long long xblocks) {
+  const long long most = std::max(kSliceBlocks / std::max(xblocks, 1LL), 16LL);
+  const long long s = std::max<long long>(kSliceLeast, (ranks + most - 1) / most);
+  return ((int)std::min<long long>(s, std::max(ranks, 1)) + 15) & ~15;
+}
+inline int edge_slices(int ranks, long long xblocks) {
+  const int s = edge_slice(ranks, xblocks);
+  return ranks > s ? (int)(((long long)ranks + s - 1) / s) : 1;
+}
+// What the blocks of n edges with at most `ranks` ranks each pad their packed
+// short runs by, at most.
+inline long long edge_block_pads(long long n, int ranks, int block) {
+  const long long x = (n + block - 1) / block;
+  return 16 * x * edge_slices(ranks, x);
+}
+// Item capacity for n edges of at most `ranks` ranks each in blocks of
+// `block` edges.
+inline long long edge_items_cap(long long n, int ranks, int block) {
+  return n * edge_run_slots(ranks) + edge_block_pads(n, ranks, block);
 }
 
 // One launch of an edge call: of the window [l0, l1) of edges [e0, e1), the
@@ -92,13 +116,15 @@ inline void edge_plan_window(long long budget, int block, int N, int l0, int l1,
   const auto groups = [](long long items) { return (int)((items + 63) / 64 * 64); };
   long long cap = edge_items_cap(N, most, block);
   if (total >= 0)  // every run padded by at most 15
-    cap = std::min(cap, total + 15LL * N + 16LL * ((N + block - 1) / block));
+    cap = std::min(cap, total + 15LL * N + edge_block_pads(N, most, block));
   if (cap <= budget) {
     plan->push_back({0, N, l0, l1, 0, most, groups(cap)});
     return;
   }
-  const int ranks = (int)std::min<long long>(most, std::max(16LL, (budget - 64) / 16 * 16));
-  const int per = (int)std::max(1LL, (budget - 64) / (edge_run_slots(ranks) + 1));
+  // (the blocks' padding is at most 1/64 of an edge of several slices, and 16)
+  const int ranks = (int)std::min<long long>(most, std::max(16LL, (budget - 64) * 64 / 65 / 16 * 16));
+  const int per =
+      (int)std::max(1LL, (budget - 64) / (edge_run_slots(ranks) + 1 + (ranks > kSliceLeast ? ranks / 64 + 1 : 0)));
   for (int e0 = 0, e1; e0 < N; e0 = e1) {
     e1 = N - e0 < per ? N : e0 + per;
     for (long long r0 = 0; r0 < most; r0 += ranks) {

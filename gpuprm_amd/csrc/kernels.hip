@@ -516,8 +516,8 @@ __global__ void __launch_bounds__(1024)
   edge_prologue_one<1024>(ndof, dq, ea, blockIdx.x * 1024 + threadIdx.x, testnum, max_testnum, total);
 }
 
-// Items for ranks [r0, r1) in the window [l0, l1) of every open edge, an edge's samples
-// in ascending order on consecutive slots.  Runs of more than kRunShort
+// Items for ranks [r0, r1) in the window [l0, l1) of every open edge, an edge's
+// samples in ascending order on consecutive slots.  Runs of more than kRunShort
 // samples start at a multiple of 16 and are padded to one (edge_run_slots);
 // the block's short runs follow them packed, padded together.  Padding items
 // repeat a sample, so that the rows' pair masks see valid items only, and are
@@ -602,10 +602,12 @@ __device__ __forceinline__ void edge_compact_one(const EdgeArgs& ea, int e, int 
 
 __global__ void __launch_bounds__(kCompactBlock)
     edge_compact_kernel(EdgeArgs ea, EdgeLaunch p, int* __restrict__ item_edge, int* __restrict__ item_pos,
-                        int* __restrict__ nitems, int* __restrict__ nsamples, unsigned* __restrict__ zero_queues) {
-  if (blockIdx.x == 0 && threadIdx.x < kSvaQueues) zero_queues[threadIdx.x * kSvaQueueStride] = 0u;
-  edge_compact_one<kCompactBlock>(ea, p.e0 + blockIdx.x * kCompactBlock + threadIdx.x, p.e1, p.l0, p.l1, p.r0, p.r1,
-                                  item_edge, item_pos, p.cap, nitems, nsamples);
+                        int* __restrict__ nitems, int* __restrict__ nsamples, unsigned* __restrict__ zero_queues,
+                        int slice) {
+  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < kSvaQueues) zero_queues[threadIdx.x * kSvaQueueStride] = 0u;
+  const int r0 = p.r0 + (int)blockIdx.y * slice;
+  edge_compact_one<kCompactBlock>(ea, p.e0 + blockIdx.x * kCompactBlock + threadIdx.x, p.e1, p.l0, p.l1, r0,
+                                  r0 + min(slice, p.r1 - r0), item_edge, item_pos, p.cap, nitems, nsamples);
 }
 
 // Multi-scene edge calls: one task per scene (prologue) or per scene part of
@@ -633,8 +635,12 @@ __global__ void __launch_bounds__(256) edge_prologue_multi_kernel(const EdgeTask
 __global__ void __launch_bounds__(kCompactBlockMulti)
     edge_compact_multi_kernel(const EdgeTask* __restrict__ tasks, int ntasks) {
   const EdgeTask& T = edge_task_of<false>(tasks, ntasks);
-  edge_compact_one<kCompactBlockMulti>(T.ea, T.e0 + (blockIdx.x - T.block0) * kCompactBlockMulti + threadIdx.x, T.e1,
-                                       T.l0, T.l1, T.r0, T.r1, T.item_edge, T.item_pos, T.cap, T.nitems, nullptr);
+  const int xblocks = (T.e1 - T.e0 + kCompactBlockMulti - 1) / kCompactBlockMulti;
+  const int y = (int)(blockIdx.x - T.block0) / xblocks, x = (int)(blockIdx.x - T.block0) - y * xblocks;
+  const int r0 = T.r0 + y * T.slice;
+  edge_compact_one<kCompactBlockMulti>(T.ea, T.e0 + x * kCompactBlockMulti + threadIdx.x, T.e1, T.l0, T.l1, r0,
+                                       r0 + min(T.slice, T.r1 - r0), T.item_edge, T.item_pos, T.cap, T.nitems,
+                                       nullptr);
 }
 
 template <int NDOF>
@@ -2208,9 +2214,10 @@ hipError_t launch_edge_prologue(const DevRobot& rb, float dq, EdgeArgs ea, int* 
 hipError_t launch_edge_compact(EdgeArgs ea, const EdgeLaunch& p, int* item_edge, int* item_pos, int* nitems,
                                int* nsamples, unsigned* zero_queues, hipStream_t st) {
   if (p.e1 <= p.e0) return hipSuccess;
-  dim3 grid((p.e1 - p.e0 + kCompactBlock - 1) / kCompactBlock), block(kCompactBlock);
+  const int x = (p.e1 - p.e0 + kCompactBlock - 1) / kCompactBlock, ranks = p.r1 - p.r0;
+  dim3 grid(x, edge_slices(ranks, x)), block(kCompactBlock);
   hipLaunchKernelGGL(edge_compact_kernel, grid, block, 0, st, ea, p, item_edge, item_pos, nitems, nsamples,
-                     zero_queues);
+                     zero_queues, edge_slice(ranks, x));
   return hipGetLastError();
 }
 

@@ -262,6 +262,7 @@ struct EdgeTask {
   int* max_testnum;
   unsigned long long* total;
   int e0, e1, l0, l1, r0, r1;
+  int slice;                    // ranks of one compaction block (edge_slice)
   int* item_edge;
   int* item_pos;
   int* nitems;

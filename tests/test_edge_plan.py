@@ -64,19 +64,28 @@ SRC = textwrap.dedent(r'''
           if (x.l0 != l || x.l1 != l1 || x.e0 >= x.e1 || x.r0 >= x.r1) return fail("launch", budget, N, maxT);
           if (x.cap <= 0 || x.cap % 64 || x.cap > std::max(budget + 63, 128LL)) return fail("cap", budget, maxT, x.cap);
           long long slots = 0;
-          for (int b0 = x.e0; b0 < x.e1; b0 += block) {  // as the compaction packs a block's runs
-            long long packed = 0;
-            for (int e = b0; e < std::min(b0 + block, x.e1); ++e) {
-              int a, b, cnt;
-              edge_window(T[e], l, l1, &a, &b, &cnt);
-              const int mine = std::max(std::min(cnt, x.r1) - x.r0, 0);
-              if (mine > 0 && next[e] != x.r0) return fail("ranks", e, x.r0, next[e]);
-              if (mine > 0) next[e] = x.r1;
-              got[e] += mine;
-              (mine <= kRunShort ? packed : slots) += edge_run_slots(mine);
+          const long long xb = (x.e1 - x.e0 + block - 1) / block;
+          const int slice = edge_slice(x.r1 - x.r0, xb), ny = edge_slices(x.r1 - x.r0, xb);
+          if (slice < 16 || slice % 16 || xb * ny > std::max(kSliceBlocks, 16 * xb) || ny > 65535) return fail("slice", slice, ny, xb);
+          std::vector<long long> packed(xb * ny, 0);  // as the compaction packs a block's runs
+          for (int e = x.e0; e < x.e1; ++e) {
+            int a, b, cnt;
+            edge_window(T[e], l, l1, &a, &b, &cnt);
+            long long mine = 0;
+            for (int y = 0; y < ny; ++y) {
+              const int r0 = x.r0 + y * slice, r1 = r0 + std::min(slice, x.r1 - r0);
+              const int run = std::max(std::min(cnt, r1) - r0, 0);
+              if (r1 <= r0) return fail("empty slice", y, ny, slice);
+              if (run == 0) break;
+              mine += run;
+              if (run <= kRunShort) packed[y * xb + (e - x.e0) / block] += run;
+              else slots += edge_run_slots(run);
             }
-            slots += (packed + 15) / 16 * 16;
+            if (mine > 0 && next[e] != x.r0) return fail("ranks", e, x.r0, next[e]);
+            if (mine > 0) next[e] = x.r1;
+            got[e] += mine;
           }
+          for (long long n : packed) slots += (n + 15) / 16 * 16;
           if (slots > x.cap) return fail("slots", slots, x.cap, maxT);
         }
         for (int e = 0; e < N; ++e) {
@@ -100,7 +109,7 @@ SRC = textwrap.dedent(r'''
         for (int block : {256, 1024})
           for (int N : {1, 2, 255, 1024, 3001}) {
             const long long parts = (long long)maxT / budget * N;
-            if (parts > 2000000) continue;  // as many launches
+            if (parts > 3000) continue;  // as many launches
             for (int known = 0; known < 2; ++known)
               if (plan(budget, block, N, maxT, known != 0, 77u + N)) return 1;
           }

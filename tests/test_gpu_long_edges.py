@@ -90,6 +90,38 @@ def test_edge_longer_than_a_launch(workload_dir, T, batch):
     assert np.array_equal(got[2:] != 0, want != 0)
 
 
+def test_edges_of_several_slices(workload_dir):
+    """Windows of about 1,024 ranks (a compaction block's slice) and of many
+    slices, short edges between them: the oracle's decisions, and every sample
+    of the free edges scheduled."""
+    import torch
+
+    import gpuprm_amd
+    d = workload_dir(1)
+    dq = 2e-5
+    sp = gpu_space(d, dq)
+    rng = np.random.default_rng(8)
+    T = np.array([1364, 1365, 1366, 1367, 1381, 2731, 4095, 4097, 30000, 100003] * 6 + [3, 17, 200] * 40)
+    rng.shuffle(T)
+    QS = rng.uniform(-3.0, 3.0, size=(4, len(T)))
+    u = rng.normal(size=QS.shape)
+    QE = QS + u / np.linalg.norm(u, axis=0) * (T - 0.5) * dq
+    QS, QE = QS.astype(np.float32), QE.astype(np.float32)
+    want, total = OracleScene(d, dq).indicator2(QS, QE, nthreads=8)
+    assert 0 < (want != 0).sum() < len(want)
+    qs, qe = torch.from_numpy(QS).cuda(), torch.from_numpy(QE).cuda()
+    res = torch.full((len(T),), 7, dtype=torch.int32, device="cuda")
+    print("slices: %d edges" % len(T), flush=True)
+    st = sp.indicator2_dev(qs, qe, res)
+    assert st.samples_total == total and np.array_equal(res.cpu().numpy() != 0, want != 0)
+    free = torch.from_numpy(np.flatnonzero(want == 0)).cuda()
+    st = sp.indicator2_dev(qs[:, free].contiguous(), qe[:, free].contiguous(), res[:len(free)])
+    assert st.samples_scheduled == st.samples_total and not res[:len(free)].any()
+    res.fill_(7)
+    gpuprm_amd.SceneBatch([sp]).indicator2_dev([qs], [qe], [res])
+    assert np.array_equal(res.cpu().numpy() != 0, want != 0)
+
+
 def gpu_space(d, dq):
     import gpuprm_amd
     sp = gpuprm_amd.RobotConfigspace(d, dq, 1 << 16)
