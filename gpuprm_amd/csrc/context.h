@@ -49,7 +49,7 @@ struct Slot {
   // (into pinned memory) while the first round runs on the call's stream
   hipStream_t side = nullptr;
   hipEvent_t ev_prologue = nullptr;
-  void* pinned = nullptr;  // 32 bytes: copy of misc[0, kMiscReadback)
+  void* pinned = nullptr;  // 32 bytes: copy of misc[0, kMiscReadback), then a flag the compaction may set
   // Edge launches after the first compact their items and compute their
   // frames on the prep stream, into the buffer set of the launch's parity,
   // while the previous launch's separating-vector kernel runs: ev_first

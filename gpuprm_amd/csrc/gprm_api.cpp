@@ -594,10 +594,18 @@ int run_edges(gprm_ctx* c, Slot& sl, const float* d_qs, const float* d_qe, long 
   ea.testnum = sl.testnum.as<int>(); ea.edge_res = d_res;
   GPRM_HIP(launch_edge_prologue(c->rb, c->dq, ea, sl.testnum.as<int>(), d_max, d_total, st), "edge prologue launch");
   const bool need_max = host_maxT < 0 || stats;
+  // Set by a compaction whose items exceed the plan's capacity (edges_complete).
+  // The planner, which enqueues without waiting, compares the largest testnum
+  // with its bound instead.
+  int* overflow = nullptr;
+  if (host_total >= 0 || stats) {
+    if (!sl.pinned) GPRM_HIP(hipHostMalloc(&sl.pinned, 32, hipHostMallocDefault), "hipHostMalloc");
+    overflow = reinterpret_cast<int*>(static_cast<char*>(sl.pinned) + kMiscReadback);
+    *overflow = 0;
+  }
   if (need_max) {
     if (!sl.side) GPRM_HIP(hipStreamCreateWithFlags(&sl.side, hipStreamNonBlocking), "hipStreamCreate");
     if (!sl.ev_prologue) GPRM_HIP(hipEventCreateWithFlags(&sl.ev_prologue, hipEventDisableTiming), "hipEventCreate");
-    if (!sl.pinned) GPRM_HIP(hipHostMalloc(&sl.pinned, 32, hipHostMallocDefault), "hipHostMalloc");
     GPRM_HIP(hipEventRecord(sl.ev_prologue, st), "event");
   }
   std::vector<EdgeLaunch> plan;
@@ -680,7 +688,7 @@ int run_edges(gprm_ctx* c, Slot& sl, const float* d_qs, const float* d_qe, long 
       float* frames = set_frames(i).as<float>();
       unsigned* queues = sl.queues.as<unsigned>() + (size_t)kSvaCounters * i;  // zeroed by the compaction
       unsigned long long* mask = use_masks(c, p.cap) ? set_mask(i).as<unsigned long long>() : nullptr;
-      GPRM_HIP(launch_edge_compact(ea, p, items_e, items_p, cnt, cnt + 1, queues, ps),
+      GPRM_HIP(launch_edge_compact(ea, p, items_e, items_p, cnt, cnt + 1, overflow, queues, ps),
                "edge compaction launch");
       size_t ev = 0;
       GPRM_HIP(prof_begin(c, sl, 1, ps, &ev), "event");
@@ -764,8 +772,16 @@ int run_edges(gprm_ctx* c, Slot& sl, const float* d_qs, const float* d_qe, long 
   return GPRM_OK;
 }
 
+// After an edge call's last launch has finished: an item that found no slot is
+// a sample that was not tested, so the results do not stand.
+int edges_complete(gprm_ctx* c, const Slot& sl) {
+  const volatile int* overflow = reinterpret_cast<const int*>(static_cast<const char*>(sl.pinned) + kMiscReadback);
+  return sl.pinned && *overflow ? fail(c, GPRM_E_CAPACITY, "more edge samples than the plan holds") : GPRM_OK;
+}
+
 // Host-side testnum (robotconfigspace.cpp:660-673), same float operations as
 // the prologue kernel; gives the round plan without a device round trip.
+// Edges of undefined or infinite length count no samples.
 long long host_testnum(const gprm_ctx* c, const float* qs, const float* qe, int N, int offset, int* maxT) {
   long long tot = 0;
   int mx = 0;
@@ -776,7 +792,8 @@ long long host_testnum(const gprm_ctx* c, const float* qs, const float* qe, int 
       norm += diff * diff;
     }
     norm = std::sqrt(norm);
-    int T = (int)(norm / c->dq) + 1;
+    const float steps = norm / c->dq;
+    const int T = steps < 0x1p31f ? (int)steps + 1 : 0;
     tot += T;
     mx = std::max(mx, T);
   }
@@ -1095,6 +1112,7 @@ int gprm_indicator2_wait(gprm_ctx* c, int request) {
     GPRM_HIP(hipMemcpyAsync(sl.host_res, sl.res.p, sizeof(int) * sl.N, hipMemcpyDeviceToHost, sl.stream),
              "copy D2H");
   GPRM_HIP(hipStreamSynchronize(sl.stream), "sync");
+  if (sl.N > 0 && (rc = edges_complete(c, sl))) return rc;
   return prof_harvest(c, sl);
 }
 
@@ -1120,6 +1138,7 @@ int gprm_indicator2_dev(gprm_ctx* c, const float* d_qs, const float* d_qe, int* 
   if ((rc = prof_prepare(c, sl, st))) return rc;
   if ((rc = run_edges(c, sl, d_qs, d_qe, offset, N, d_res, st, -1, -1, kOneRoundAny, &local))) return rc;
   GPRM_HIP(hipStreamSynchronize(st), "sync");
+  if (N > 0 && (rc = edges_complete(c, sl))) return rc;
   c->numthreads_all += local.samples_total;
   if (stats) *stats = local;
   return prof_harvest(c, sl);

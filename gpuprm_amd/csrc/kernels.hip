@@ -477,7 +477,9 @@ __device__ __forceinline__ void edge_prologue_one(int ndof, float dq, const Edge
       norm += diff * diff;
     }
     norm = __builtin_sqrtf(norm);
-    T = (int)(norm / dq) + 1;
+    // an undefined length (NaN) is one sample, an infinite one none
+    const float steps = norm / dq;
+    T = steps >= 0x1p31f ? 0 : steps == steps ? (int)steps + 1 : 1;
     testnum[k] = T;
     ea.edge_res[k] = 0;
   }
@@ -529,7 +531,8 @@ __global__ void __launch_bounds__(1024)
 template <int BLOCK>
 __device__ __forceinline__ void edge_compact_one(const EdgeArgs& ea, int e, int e1, int l0, int l1, int r0, int r1,
                                                  int* __restrict__ item_edge, int* __restrict__ item_pos, int cap,
-                                                 int* __restrict__ nitems, int* __restrict__ nsamples) {
+                                                 int* __restrict__ nitems, int* __restrict__ nsamples,
+                                                 int* __restrict__ overflow) {
   int a = 1, b = 0, cnt = 0;
   if (e < e1 && __hip_atomic_load(&ea.edge_res[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
     edge_window(ea.testnum[e], l0, l1, &a, &b, &cnt);
@@ -571,6 +574,7 @@ __device__ __forceinline__ void edge_compact_one(const EdgeArgs& ea, int e, int 
     s_short0 = sl;
     s_shorts = ss;
     if (nsamples != nullptr && sn > 0) atomicAdd(nsamples, sn);
+    if (overflow != nullptr && s_base > cap - total) *overflow = 1;
   }
   __syncthreads();
   // first slot of the lane's run, and the end of its padding: the block's
@@ -603,11 +607,12 @@ __device__ __forceinline__ void edge_compact_one(const EdgeArgs& ea, int e, int 
 __global__ void __launch_bounds__(kCompactBlock)
     edge_compact_kernel(EdgeArgs ea, EdgeLaunch p, int* __restrict__ item_edge, int* __restrict__ item_pos,
                         int* __restrict__ nitems, int* __restrict__ nsamples, unsigned* __restrict__ zero_queues,
-                        int slice) {
+                        int slice, int* __restrict__ overflow) {
   if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < kSvaQueues) zero_queues[threadIdx.x * kSvaQueueStride] = 0u;
   const int r0 = p.r0 + (int)blockIdx.y * slice;
   edge_compact_one<kCompactBlock>(ea, p.e0 + blockIdx.x * kCompactBlock + threadIdx.x, p.e1, p.l0, p.l1, r0,
-                                  r0 + min(slice, p.r1 - r0), item_edge, item_pos, p.cap, nitems, nsamples);
+                                  r0 + min(slice, p.r1 - r0), item_edge, item_pos, p.cap, nitems, nsamples,
+                                  overflow);
 }
 
 // Multi-scene edge calls: one task per scene (prologue) or per scene part of
@@ -640,7 +645,7 @@ __global__ void __launch_bounds__(kCompactBlockMulti)
   const int r0 = T.r0 + y * T.slice;
   edge_compact_one<kCompactBlockMulti>(T.ea, T.e0 + x * kCompactBlockMulti + threadIdx.x, T.e1, T.l0, T.l1, r0,
                                        r0 + min(T.slice, T.r1 - r0), T.item_edge, T.item_pos, T.cap, T.nitems,
-                                       nullptr);
+                                       nullptr, nullptr);
 }
 
 template <int NDOF>
@@ -2212,12 +2217,12 @@ hipError_t launch_edge_prologue(const DevRobot& rb, float dq, EdgeArgs ea, int* 
 }
 
 hipError_t launch_edge_compact(EdgeArgs ea, const EdgeLaunch& p, int* item_edge, int* item_pos, int* nitems,
-                               int* nsamples, unsigned* zero_queues, hipStream_t st) {
+                               int* nsamples, int* overflow, unsigned* zero_queues, hipStream_t st) {
   if (p.e1 <= p.e0) return hipSuccess;
   const int x = (p.e1 - p.e0 + kCompactBlock - 1) / kCompactBlock, ranks = p.r1 - p.r0;
   dim3 grid(x, edge_slices(ranks, x)), block(kCompactBlock);
   hipLaunchKernelGGL(edge_compact_kernel, grid, block, 0, st, ea, p, item_edge, item_pos, nitems, nsamples,
-                     zero_queues, edge_slice(ranks, x));
+                     zero_queues, edge_slice(ranks, x), overflow);
   return hipGetLastError();
 }
 

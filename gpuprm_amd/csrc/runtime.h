@@ -318,12 +318,13 @@ hipError_t launch_edge_prologue(const DevRobot& rb, float dq, EdgeArgs ea, int* 
 // Items of ranks [p.r0, p.r1) in the window [p.l0, p.l1) of the open edges in
 // [p.e0, p.e1): item_edge, item_pos
 // (the sample), *nitems slots of which *nsamples (may be null) are no padding.
-// Slots beyond p.cap (an edge longer than the plan's bound) are not written.
+// Slots beyond p.cap (an edge longer than the plan's bound) are not written;
+// *overflow (device-visible, may be null) becomes 1 then.
 // zero_queues: the work counters of the separating-vector launch that
 // follows, set to zero.
 constexpr int kCompactBlock = 1024, kCompactBlockMulti = 256;
 hipError_t launch_edge_compact(EdgeArgs ea, const EdgeLaunch& p, int* item_edge, int* item_pos, int* nitems,
-                               int* nsamples, unsigned* zero_queues, hipStream_t st);
+                               int* nsamples, int* overflow, unsigned* zero_queues, hipStream_t st);
 // Kinematics of the *nitems (<= cap) compacted samples; frames link-major
 // with item stride cap (the plane stride); their pair masks to mask unless
 // it is null.
