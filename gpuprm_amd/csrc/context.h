@@ -35,21 +35,20 @@ struct DevBuf {
   template <class T> T* as() const { return static_cast<T*>(p); }
 };
 
-// Layout of a slot's `misc` words written by the edge prologue and read back
-// into `pinned`: the largest testnum (int) and the sample total (u64).
+// Layout of a slot's `misc` words written by the edge prologue: the largest
+// testnum (int), the sample total (u64), and a count of its finished blocks
+// (u32).  Of `pinned` (EdgePinned): the same two, written there by the
+// prologue's last block, and the compaction's flag.
 constexpr size_t kMiscMaxT = 0;
 constexpr size_t kMiscTotal = 16;
-constexpr size_t kMiscReadback = 24;
+constexpr size_t kMiscBlocks = 32;
 
 // Buffers of one in-flight request (the reference keeps one buffer set and
 // one stream per outstanding request, robotconfigspace.cpp:627-650).
 struct Slot {
   hipStream_t stream = nullptr;
-  // edge calls read the prologue's largest testnum back on a side stream
-  // (into pinned memory) while the first round runs on the call's stream
-  hipStream_t side = nullptr;
-  hipEvent_t ev_prologue = nullptr;
-  void* pinned = nullptr;  // 32 bytes: copy of misc[0, kMiscReadback), then a flag the compaction may set
+  hipEvent_t ev_prologue = nullptr;  // an edge call's prologue has finished
+  EdgePinned* pinned = nullptr;      // pinned memory, what the host reads of an edge call
   // Edge launches after the first compact their items and compute their
   // frames on the prep stream, into the buffer set of the launch's parity,
   // while the previous launch's separating-vector kernel runs: ev_first
@@ -73,7 +72,6 @@ struct Slot {
   ~Slot() {
     for (auto e : ev_start) (void)hipEventDestroy(e);
     for (auto e : ev_end) (void)hipEventDestroy(e);
-    if (side) (void)hipStreamSynchronize(side);
     if (prep) (void)hipStreamSynchronize(prep);
     for (auto e : ev_fk) (void)hipEventDestroy(e);
     for (auto e : ev_sva) (void)hipEventDestroy(e);
@@ -85,7 +83,6 @@ struct Slot {
       if (stream) (void)hipStreamSynchronize(stream);
       (void)hipHostFree(small_out);
     }
-    if (side) (void)hipStreamDestroy(side);
     if (stream) (void)hipStreamDestroy(stream);
   }
 };

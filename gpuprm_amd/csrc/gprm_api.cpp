@@ -587,24 +587,32 @@ int run_edges(gprm_ctx* c, Slot& sl, const float* d_qs, const float* d_qe, long 
   GPRM_HIP(sl.misc.ensure(64), "hipMalloc misc");
   int* d_max = reinterpret_cast<int*>(sl.misc.as<char>() + kMiscMaxT);
   unsigned long long* d_total = reinterpret_cast<unsigned long long*>(sl.misc.as<char>() + kMiscTotal);
-  GPRM_HIP(launch_fill_u32(sl.misc.as<unsigned>(), 0u, 16, st), "fill");
+  if (N > kPrologueBlock) GPRM_HIP(launch_fill_u32(sl.misc.as<unsigned>(), 0u, 16, st), "fill");
   EdgeArgs ea{};
   ea.qs = d_qs; ea.qe = d_qe; ea.offset = offset; ea.nedges = N;
   ea.skip = skip;
   ea.testnum = sl.testnum.as<int>(); ea.edge_res = d_res;
-  GPRM_HIP(launch_edge_prologue(c->rb, c->dq, ea, sl.testnum.as<int>(), d_max, d_total, st), "edge prologue launch");
-  const bool need_max = host_maxT < 0 || stats;
   // Set by a compaction whose items exceed the plan's capacity (edges_complete).
   // The planner, which enqueues without waiting, compares the largest testnum
   // with its bound instead.
   int* overflow = nullptr;
-  if (host_total >= 0 || stats) {
-    if (!sl.pinned) GPRM_HIP(hipHostMalloc(&sl.pinned, 32, hipHostMallocDefault), "hipHostMalloc");
-    overflow = reinterpret_cast<int*>(static_cast<char*>(sl.pinned) + kMiscReadback);
+  if (host_total >= 0 || host_maxT < 0) {
+    if (!sl.pinned)
+      GPRM_HIP(hipHostMalloc(reinterpret_cast<void**>(&sl.pinned), sizeof(EdgePinned), hipHostMallocDefault),
+               "hipHostMalloc");
+    overflow = &sl.pinned->overflow;
     *overflow = 0;
   }
-  if (need_max) {
-    if (!sl.side) GPRM_HIP(hipStreamCreateWithFlags(&sl.side, hipStreamNonBlocking), "hipStreamCreate");
+  const bool need_max = host_maxT < 0;
+  GPRM_HIP(launch_edge_prologue(c->rb, c->dq, ea, sl.testnum.as<int>(), d_max, d_total,
+                                reinterpret_cast<unsigned*>(sl.misc.as<char>() + kMiscBlocks),
+                                need_max ? sl.pinned : nullptr, st),
+           "edge prologue launch");
+  // The first window [0, 1) needs no largest testnum, so in a call that
+  // surely takes several rounds it is enqueued at once, before the wait for
+  // the prologue.
+  const bool ahead = need_max && 16LL * N * c->img.M > kOneRoundAny;
+  if (ahead) {
     if (!sl.ev_prologue) GPRM_HIP(hipEventCreateWithFlags(&sl.ev_prologue, hipEventDisableTiming), "hipEventCreate");
     GPRM_HIP(hipEventRecord(sl.ev_prologue, st), "event");
   }
@@ -729,10 +737,6 @@ int run_edges(gprm_ctx* c, Slot& sl, const float* d_qs, const float* d_qe, long 
   int maxT = host_maxT;
   long long total = host_total;
   const long long M = c->img.M;
-  // The first window [0, 1) needs no largest testnum, so in a call that
-  // surely takes several rounds it is enqueued at once, and the largest
-  // testnum is read back on the side stream meanwhile.
-  const bool ahead = host_maxT < 0 && 16LL * N * M > kOneRoundAny;
   if (host_maxT >= 0) {
     for (const auto& w : edge_windows(host_maxT, (total >= 0 ? total : (long long)N * host_maxT) * M, one_round))
       plan_window(c, N, w.first, w.second, host_maxT, total, &plan);
@@ -741,13 +745,9 @@ int run_edges(gprm_ctx* c, Slot& sl, const float* d_qs, const float* d_qe, long 
   }
   if ((rc = enqueue(0)) != GPRM_OK) return rc;
   if (need_max) {
-    GPRM_HIP(hipStreamWaitEvent(sl.side, sl.ev_prologue, 0), "stream wait");
-    GPRM_HIP(hipMemcpyAsync(sl.pinned, sl.misc.p, kMiscReadback, hipMemcpyDeviceToHost, sl.side), "copy max");
-    GPRM_HIP(hipStreamSynchronize(sl.side), "sync");
-    unsigned long long t = 0;
-    std::memcpy(&maxT, static_cast<char*>(sl.pinned) + kMiscMaxT, 4);
-    std::memcpy(&t, static_cast<char*>(sl.pinned) + kMiscTotal, 8);
-    total = (long long)t;
+    GPRM_HIP(ahead ? hipEventSynchronize(sl.ev_prologue) : hipStreamSynchronize(st), "sync");
+    maxT = sl.pinned->maxT;
+    total = (long long)sl.pinned->total;
   }
   if (host_maxT < 0) {
     const size_t first = plan.size();
@@ -775,8 +775,7 @@ int run_edges(gprm_ctx* c, Slot& sl, const float* d_qs, const float* d_qe, long 
 // After an edge call's last launch has finished: an item that found no slot is
 // a sample that was not tested, so the results do not stand.
 int edges_complete(gprm_ctx* c, const Slot& sl) {
-  const volatile int* overflow = reinterpret_cast<const int*>(static_cast<const char*>(sl.pinned) + kMiscReadback);
-  return sl.pinned && *overflow ? fail(c, GPRM_E_CAPACITY, "more edge samples than the plan holds") : GPRM_OK;
+  return sl.pinned && sl.pinned->overflow ? fail(c, GPRM_E_CAPACITY, "more edge samples than the plan holds") : GPRM_OK;
 }
 
 // Host-side testnum (robotconfigspace.cpp:660-673), same float operations as

@@ -465,7 +465,7 @@ template <int BLOCK>
 __device__ __forceinline__ void edge_prologue_one(int ndof, float dq, const EdgeArgs& ea, int k,
                                                   int* __restrict__ testnum,
                                                   int* __restrict__ max_testnum,
-                                                  unsigned long long* __restrict__ total) {
+                                                  unsigned long long* __restrict__ total, bool only = false) {
   int T = 0;
   if (k < ea.nedges && ea.skip != nullptr && ea.skip[k]) {
     testnum[k] = 0;
@@ -505,17 +505,35 @@ __device__ __forceinline__ void edge_prologue_one(int ndof, float dq, const Edge
       tmax = max(tmax, s_max[w]);
       tsum += s_sum[w];
     }
-    if (tmax > 0) {
+    if (only) {
+      *max_testnum = tmax;
+      *total = tsum;
+    } else if (tmax > 0) {
       atomicMax(max_testnum, tmax);
       atomicAdd(total, tsum);
     }
   }
 }
 
-__global__ void __launch_bounds__(1024)
-    edge_prologue_kernel(int ndof, float dq, EdgeArgs ea, int* __restrict__ testnum, int* __restrict__ max_testnum,
-                         unsigned long long* __restrict__ total) {
-  edge_prologue_one<1024>(ndof, dq, ea, blockIdx.x * 1024 + threadIdx.x, testnum, max_testnum, total);
+// The block that finishes last leaves the totals in pinned memory, so that the
+// host waits for this launch and nothing more.  (With an event, a copy on a
+// second stream and a wait for that, calls of short edges, which are one round,
+// took 108-138 us where 75-105 are enough: 32 edges of 0.08 rad on the 4-DOF
+// scene 113 and 81 us.)
+__global__ void __launch_bounds__(kPrologueBlock)
+    edge_prologue_kernel(int ndof, float dq, EdgeArgs ea, int* __restrict__ testnum, int* max_testnum,
+                         unsigned long long* total, unsigned* blocks, EdgePinned* host) {
+  const bool only = gridDim.x == 1;
+  edge_prologue_one<kPrologueBlock>(ndof, dq, ea, blockIdx.x * kPrologueBlock + threadIdx.x, testnum, max_testnum,
+                                    total, only);
+  if (host == nullptr || threadIdx.x != 0) return;
+  if (!only) {
+    __threadfence();
+    if (atomicAdd(blocks, 1u) != gridDim.x - 1) return;
+    __threadfence();
+  }
+  host->maxT = only ? *max_testnum : atomicMax(max_testnum, 0);
+  host->total = only ? *total : atomicAdd(total, 0ull);
 }
 
 // Items for ranks [r0, r1) in the window [l0, l1) of every open edge, an edge's
@@ -2208,11 +2226,11 @@ hipError_t launch_finalize_points_multi(const FkTask* d_tasks, int ntasks, int n
 }
 
 hipError_t launch_edge_prologue(const DevRobot& rb, float dq, EdgeArgs ea, int* testnum_out, int* max_testnum,
-                                unsigned long long* total, hipStream_t st) {
+                                unsigned long long* total, unsigned* blocks, EdgePinned* host, hipStream_t st) {
   if (ea.nedges <= 0) return hipSuccess;
-  dim3 grid((ea.nedges + 1023) / 1024), block(1024);
+  dim3 grid((ea.nedges + kPrologueBlock - 1) / kPrologueBlock), block(kPrologueBlock);
   hipLaunchKernelGGL(edge_prologue_kernel, grid, block, 0, st, rb.ndof, dq, ea, testnum_out,
-                     max_testnum, total);
+                     max_testnum, total, blocks, host);
   return hipGetLastError();
 }
 

@@ -234,6 +234,13 @@ __device__ __forceinline__ void node_dist2(const float* __restrict__ coords, siz
 // as free).
 constexpr int kEdgeSkipped = 0x40000000;
 
+// What the kernels of an edge call leave in pinned memory for the host.
+struct EdgePinned {
+  unsigned long long total;  // samples of all edges
+  int maxT;                  // the largest testnum
+  int overflow;              // nonzero: a launch's items exceeded its capacity
+};
+
 // Edge work description.
 struct EdgeArgs {
   const float* qs; const float* qe; long long offset;  // SoA, component i of edge k at [k + offset*i]
@@ -313,8 +320,12 @@ hipError_t launch_fk_points_multi(const FkTask* d_tasks, int ntasks, int nblocks
 hipError_t launch_finalize_points_multi(const FkTask* d_tasks, int ntasks, int nblocks, hipStream_t st);
 hipError_t launch_sva_multi(const SceneTask* d_tasks, int ntasks, int edge_mode, const SvaShape& sh, size_t img_bytes,
                             unsigned long long* t_start, unsigned long long* tally, hipStream_t st);
+// testnum and edge results; the largest testnum to *max_testnum and the sum to
+// *total, which with *blocks are zeroed before where the edges are more than
+// one block's (kPrologueBlock), and both to *host (pinned memory, may be null).
+constexpr int kPrologueBlock = 1024;
 hipError_t launch_edge_prologue(const DevRobot& rb, float dq, EdgeArgs ea, int* testnum_out, int* max_testnum,
-                                unsigned long long* total, hipStream_t st);
+                                unsigned long long* total, unsigned* blocks, EdgePinned* host, hipStream_t st);
 // Items of ranks [p.r0, p.r1) in the window [p.l0, p.l1) of the open edges in
 // [p.e0, p.e1): item_edge, item_pos
 // (the sample), *nitems slots of which *nsamples (may be null) are no padding.
