@@ -97,73 +97,6 @@ void fill_robot(const Scene& s, DevRobot* rb) {
 
 size_t align16(size_t x) { return (x + 15) & ~(size_t)15; }
 
-// Certificate factor of a polytope's support scan (support in kernels.hip):
-// with w the vertex whose product with a direction d is largest, by more than
-// factor |d|_1 above every other vertex's, the hill climb in floats ends at w
-// from any start; inf if that cannot be promised, or if the climb is the
-// cheaper way (more vertices than kScanVertices).
-//   The polytope lies in the cone of the stored neighbours' edges e_i at each
-// vertex u: w - u = sum l_i e_i, l_i >= 0.  So (w - u).d <= (sum l_i) max e_i.d,
-// and u has a neighbour better by (w - u).d / L, L the largest sum l_i over
-// all u and w.  The climb's products err by at most g = 3.1 2^-24 vmax |d|_1
-// each, the scan's too: it suffices that the scan's margin exceeds
-// (2 L + 2) g.  The coefficients are checked here from the stored adjacency,
-// so a row that misses edges has no factor.
-//   Faces of more than three vertices are not quite plane in floats, so a
-// vertex of a face may lie outside the cone by a rounding error.  A negative
-// coefficient -m adds at most m |e_i.d| <= 2 m vmax |d|_1, and counts as
-// m kScanOutside of sum l_i.  (Refusing any negative one left most boxes to the
-// climb: 65,536 points of the 4-DOF scene 66 against 62.5 us so.)
-constexpr int kScanVertices = 32, kScanDegree = 16;
-constexpr double kScanOutside = 5e6;  // 2 vmax |d|_1 over the 2 g (g = 3.41 2^-24 vmax |d|_1) of one l_i, and some
-float support_factor(const Polytope& p) {
-  const float none = INFINITY;
-  const int n = p.n();
-  if (n > kScanVertices) return none;
-  auto at = [&](int v, int a) { return (double)p.verts[3 * v + a]; };
-  double vmax = 0.0, L = 0.0;
-  for (float x : p.verts) vmax = std::max(vmax, std::fabs((double)x));
-  for (int u = 0; u < n; ++u) {
-    const int deg = p.cnt[u];
-    if (deg > kScanDegree) return none;
-    double e[kScanDegree][3];
-    for (int i = 0; i < deg; ++i)
-      for (int a = 0; a < 3; ++a) e[i][a] = at(p.dest[p.dsp[u] + i], a) - at(u, a);
-    for (int w = 0; w < n; ++w) {
-      if (w == u) continue;
-      const double x[3] = {at(w, 0) - at(u, 0), at(w, 1) - at(u, 1), at(w, 2) - at(u, 2)};
-      double best = 1e300;
-      for (int i = 0; i < deg && best > 1.0; ++i)  // a neighbour: its own edge
-        if (p.dest[p.dsp[u] + i] == w) best = 1.0;
-      for (int i = 0; i < deg && best > 4.0; ++i)
-        for (int j = i + 1; j < deg && best > 4.0; ++j) {
-          const double c[3] = {e[i][1] * e[j][2] - e[i][2] * e[j][1], e[i][2] * e[j][0] - e[i][0] * e[j][2],
-                               e[i][0] * e[j][1] - e[i][1] * e[j][0]};
-          for (int k = j + 1; k < deg && best > 4.0; ++k) {
-            const double* f = e[k];
-            const double det = c[0] * f[0] + c[1] * f[1] + c[2] * f[2];
-            auto len = [](const double* v) { return std::sqrt(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]); };
-            if (!(std::fabs(det) > 1e-5 * len(e[i]) * len(e[j]) * len(f))) continue;
-            auto det3 = [](const double* p0, const double* p1, const double* p2) {
-              return p0[0] * (p1[1] * p2[2] - p1[2] * p2[1]) - p0[1] * (p1[0] * p2[2] - p1[2] * p2[0]) +
-                     p0[2] * (p1[0] * p2[1] - p1[1] * p2[0]);
-            };
-            const double li = det3(x, e[j], f) / det, lj = det3(e[i], x, f) / det, lk = det3(e[i], e[j], x) / det;
-            double sum = 0.0;
-            for (double v : {li, lj, lk}) sum += v > 0.0 ? v : -kScanOutside * v;
-            best = std::min(best, sum);
-          }
-        }
-      if (best > 1e6) return none;
-      L = std::max(L, best);
-    }
-  }
-  // the products' errors, and 1e-8 vmax for the coefficients' own
-  const double f = ((2.0 * L + 2.0) * 3.41 * 0x1p-24 + 1e-8) * vmax;
-  const float r = (float)(f * (1.0 + 1e-6));
-  return std::isfinite(r) ? r : none;
-}
-
 // Pack the scene image (layout documented at SceneImg).  The kernel visits
 // pairs grouped by the frames they need; each pair keeps its index in the
 // reference's CRS order (polytope4data.h:343-357: by `from`, then as given),
@@ -267,9 +200,7 @@ int build_image(gprm_ctx* c, std::vector<char>* out) {
     rec.rb = s.sys[k] == 0 ? rb : rf;
     rec.frame = s.sys[k];
     std::memcpy(b + (size_t)img.off_polyrecs + sizeof(rec) * (size_t)k, &rec, sizeof(rec));
-    const float cert = support_factor(p);
-    int hull[2] = {std::isfinite(cert) ? p.n() : 0, 0};
-    std::memcpy(&hull[1], &cert, 4);
+    const int hull[2] = {p.n(), vbase[k]};  // launch_support_factors' input
     std::memcpy(b + img.off_hulls + 8 * (size_t)k, hull, 8);
   }
   // the polytopes at rest, then the moving ones by link, for the pair masks
@@ -954,8 +885,11 @@ int gprm_init(gprm_ctx* c, int rank, int size) {
   int rc = build_image(c, &image);
   if (rc != GPRM_OK) return rc;
   GPRM_HIP(c->img_buf.ensure(image.size()), "hipMalloc scene");
-  GPRM_HIP(hipMemcpy(c->img_buf.p, image.data(), image.size(), hipMemcpyHostToDevice), "copy scene");
+  // (waited for at the end, with the launch)
+  struct Wait { ~Wait() { (void)hipStreamSynchronize(nullptr); } } wait;
+  GPRM_HIP(hipMemcpyAsync(c->img_buf.p, image.data(), image.size(), hipMemcpyHostToDevice, nullptr), "copy scene");
   c->img.blob = c->img_buf.as<int4>();
+  GPRM_HIP(launch_support_factors(c->img, c->img_buf.as<char>(), nullptr), "support certificates");
   c->shape = sva_default_shape(c->img);
   GPRM_HIP(sva_shape_finish(c->img, &c->shape, c->device), "separating-vector launch shape");
   c->shape_few = SvaShape{};
@@ -965,6 +899,7 @@ int gprm_init(gprm_ctx* c, int rank, int size) {
     if (sva_shape_finish(c->img, &few, c->device) == hipSuccess && few.grid <= c->shape.grid) c->shape_few = few;
   }
   c->small_calls = point_small_prepare(c->img) == hipSuccess;
+  GPRM_HIP(hipStreamSynchronize(nullptr), "support certificates");
   c->inited = true;
   return GPRM_OK;
 }

@@ -973,7 +973,7 @@ __device__ __forceinline__ int climb(const Lds& L, int p, const V3& dir) {
 // steps as the wave's slowest lane; instead the lanes read all vertices of
 // their polytope, which depend on nothing, and keep the largest product and
 // the next one.  Where they are further apart than the certificate asks
-// (support_factor in the host runtime: then the climb, from any start and in
+// (support_factor_kernel: then the climb, from any start and in
 // its own rounding, ends at the largest), that vertex is the answer; else the
 // climb runs.  The scan's products only have to stay inside the certificate.
 // 9 vector instructions a vertex against about 65 a climb step (4M points of
@@ -1002,6 +1002,131 @@ __device__ __forceinline__ int support(const Lds& L, int k, int v0, int p, const
   // (false for a NaN, too; need < 1e20 keeps the products far from overflow)
   if ((best - second > need) & (need < 1e20f)) return v0 + at;
   return climb(L, p, dir);
+}
+
+// Certificate factors of the polytopes' support scans (support):
+// with w the vertex whose product with a direction d is largest, by more than
+// factor |d|_1 above every other vertex's, the hill climb in floats ends at w
+// from any start; inf if that cannot be promised, or if the climb is the
+// cheaper way (more vertices than kScanVertices).
+//   The polytope lies in the cone of the stored neighbours' edges e_i at each
+// vertex u: w - u = sum l_i e_i, l_i >= 0.  So (w - u).d <= (sum l_i) max e_i.d,
+// and u has a neighbour better by (w - u).d / L, L the largest sum l_i over
+// all u and w.  The climb's products err by at most g = 3.1 2^-24 vmax |d|_1
+// each, the scan's too: it suffices that the scan's margin exceeds
+// (2 L + 2) g.  The coefficients are checked here from the stored adjacency,
+// so a row that misses edges has no factor.
+//   Faces of more than three vertices are not quite plane in floats, so a
+// vertex of a face may lie outside the cone by a rounding error.  A negative
+// coefficient -m adds at most m |e_i.d| <= 2 m vmax |d|_1, and counts as
+// m kScanOutside of sum l_i.  (Refusing any negative one left most boxes to the
+// climb: 65,536 points of the 4-DOF scene 66 against 62.5 us so.)
+//   A block computes one polytope's factor, 32 lanes a vertex u's part of it:
+// each lane inverts one cone (e_i, e_j, e_k) at a time, kCertCones of them go
+// to LDS, and every lane tries them for its own vertex w, until all w have a
+// sum of at most 4, which need not be bettered.  On the host, pair after pair,
+// the 256 polytopes of 32 vertices of a large scene took 21 ms of its set-up,
+// 0.04 so (set-up in all 21.2 -> 0.25 ms; 0.13 -> 0.06 for the 7-DOF scene's 39
+// polytopes; 23 -> 29 us for the 4-DOF scene's 12, of which 10 are the launch).
+constexpr int kScanVertices = 32, kScanDegree = 16, kCertCones = 16, kCertBlock = 32 * kScanVertices;
+constexpr double kScanOutside = 5e6;  // 2 vmax |d|_1 over the 2 g (g = 3.41 2^-24 vmax |d|_1) of one l_i, and some
+__global__ void __launch_bounds__(kCertBlock) support_factor_kernel(SceneImg img, char* __restrict__ blob) {
+  __shared__ double s_v[kScanVertices][3], s_e[kScanVertices][kScanDegree][3], s_len[kScanVertices][kScanDegree];
+  __shared__ double s_cone[kScanVertices][kCertCones][9];
+  __shared__ int s_nb[kScanVertices][kScanDegree], s_deg[kScanVertices];
+  __shared__ unsigned long long s_L;  // the bits of L >= 0, which order as the values do
+  __shared__ int s_none;
+  int2* const hull = reinterpret_cast<int2*>(blob + img.off_hulls) + blockIdx.x;
+  const float4* const verts = reinterpret_cast<const float4*>(blob + img.off_verts);
+  const unsigned short* const adj = reinterpret_cast<const unsigned short*>(blob + img.off_adj);
+  const int n = hull->x, v0 = hull->y;
+  const int u = threadIdx.x >> 5, w = threadIdx.x & 31;
+  if (threadIdx.x == 0) {
+    s_L = 0ull;
+    s_none = n > kScanVertices ? 1 : 0;
+  }
+  __syncthreads();
+  if (u == 0 && n <= kScanVertices && w < n) {
+    const float4 r = verts[v0 + w];
+    s_v[w][0] = r.x;
+    s_v[w][1] = r.y;
+    s_v[w][2] = r.z;
+    s_deg[w] = info_of(r) & 255;
+    if (s_deg[w] > kScanDegree) s_none = 1;
+  }
+  __syncthreads();
+  const int count = s_none ? 0 : n;
+  const int deg = u < count ? s_deg[u] : 0;
+  if (w < deg) {
+    const int to = adj[(info_of(verts[v0 + u]) >> 8) + w] - v0;
+    s_nb[u][w] = to;
+    double* const e = s_e[u][w];
+    for (int a = 0; a < 3; ++a) e[a] = s_v[to][a] - s_v[u][a];
+    s_len[u][w] = __builtin_sqrt(e[0] * e[0] + e[1] * e[1] + e[2] * e[2]);
+  }
+  __syncthreads();
+  if (u < count) {
+    const bool asked = w < count && w != u;
+    double x[3] = {0.0, 0.0, 0.0}, best = asked ? 1e300 : 0.0;
+    if (asked)
+      for (int a = 0; a < 3; ++a) x[a] = s_v[w][a] - s_v[u][a];
+    for (int i = 0; i < deg; ++i)  // a neighbour: its own edge
+      if (asked && s_nb[u][i] == w) best = 1.0;
+    const int triples = deg * (deg - 1) * (deg - 2) / 6;
+    const unsigned long long half = 0xffffffffull << (threadIdx.x & 32);
+    for (int t0 = 0; t0 < triples && (__ballot(best > 4.0) & half) != 0ull; t0 += kCertCones) {
+      const int t = t0 + w;
+      if (w < kCertCones) {
+        double* const m = s_cone[u][w];
+        m[0] = __builtin_nan("");  // no cone: every comparison with it is false
+        if (t < triples) {
+          int i = 0, j, k = t;  // triple t: i < j < k
+          for (int c; k >= (c = (deg - 1 - i) * (deg - 2 - i) / 2); ++i) k -= c;
+          for (j = i + 1; k >= deg - 1 - j; ++j) k -= deg - 1 - j;
+          k += j + 1;
+          const double *ei = s_e[u][i], *ej = s_e[u][j], *f = s_e[u][k];
+          const double c[3] = {ei[1] * ej[2] - ei[2] * ej[1], ei[2] * ej[0] - ei[0] * ej[2],
+                               ei[0] * ej[1] - ei[1] * ej[0]};
+          const double det = c[0] * f[0] + c[1] * f[1] + c[2] * f[2];
+          if (fabs(det) > 1e-5 * s_len[u][i] * s_len[u][j] * s_len[u][k]) {
+            const double inv = 1.0 / det;
+            m[0] = (ej[1] * f[2] - ej[2] * f[1]) * inv;
+            m[1] = (ej[2] * f[0] - ej[0] * f[2]) * inv;
+            m[2] = (ej[0] * f[1] - ej[1] * f[0]) * inv;
+            m[3] = (f[1] * ei[2] - f[2] * ei[1]) * inv;
+            m[4] = (f[2] * ei[0] - f[0] * ei[2]) * inv;
+            m[5] = (f[0] * ei[1] - f[1] * ei[0]) * inv;
+            for (int a = 0; a < 3; ++a) m[6 + a] = c[a] * inv;
+          }
+        }
+      }
+      // the cones were written by other lanes of this wave
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      for (int s = 0; s < kCertCones; ++s) {
+        const double* const m = s_cone[u][s];
+        double sum = 0.0;
+        for (int r = 0; r < 9; r += 3) {
+          const double l = m[r] * x[0] + m[r + 1] * x[1] + m[r + 2] * x[2];
+          sum += l > 0.0 ? l : -kScanOutside * l;
+        }
+        if (sum < best) best = sum;
+      }
+      __builtin_amdgcn_wave_barrier();  // before the next cones
+    }
+    if (best > 1e6) s_none = 1;
+    else atomicMax(&s_L, (unsigned long long)__double_as_longlong(best));
+  }
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  double vmax = 0.0;
+  for (int i = 0; i < count; ++i)
+    for (int a = 0; a < 3; ++a) vmax = fmax(vmax, fabs(s_v[i][a]));
+  // the products' errors, and 1e-8 vmax for the coefficients' own
+  const double L = __longlong_as_double((long long)s_L);
+  const float f = (float)(((2.0 * L + 2.0) * 3.41 * 0x1p-24 + 1e-8) * vmax * (1.0 + 1e-6));
+  const bool ok = s_none == 0 && f < __builtin_inff();
+  *hull = make_int2(ok ? n : 0, __float_as_int(ok ? f : __builtin_inff()));
 }
 
 // orthtrafo23 (collision4.h:111-134)
@@ -2164,6 +2289,12 @@ hipError_t launch_sva(const SvaArgs& a, int edge_mode, const SvaShape& sh, hipSt
 // iteration history.
 static size_t point_small_lds(const SceneImg& img, int block) {
   return (size_t)img.bytes + sizeof(T12) * kMaxDofDev + sizeof(float4) * kMaxIter * (size_t)block;
+}
+
+hipError_t launch_support_factors(const SceneImg& img, char* blob, hipStream_t st) {
+  if (img.N <= 0) return hipSuccess;
+  hipLaunchKernelGGL(support_factor_kernel, dim3(img.N), dim3(kCertBlock), 0, st, img, blob);
+  return hipGetLastError();
 }
 
 hipError_t point_small_prepare(const SceneImg& img) {

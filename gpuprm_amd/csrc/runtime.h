@@ -41,7 +41,8 @@ struct DevRobot {
 //                          each padded to a multiple of 4 with the row's vertex
 //   hulls    int2[N]       per polytope: (its vertex count, the bits of the
 //                          support scan's certificate factor; see support in
-//                          kernels.hip), (0, inf): no scan
+//                          kernels.hip), (0, inf): no scan; written by
+//                          launch_support_factors
 // Behind the staged image lie tables that are read through the scalar cache
 // (byte offsets, 64-byte aligned), small enough to stay in its 16 KB for
 // scenes of up to about 100 polytopes and 900 pairs:
@@ -351,6 +352,10 @@ struct SmallPoints {
   float q[kSmallMax][kMaxDofDev];
 };
 hipError_t point_small_prepare(const SceneImg& img);
+// The support scan's certificate factors into the image's hulls, in the
+// device image `blob` (img.blob, writable); the hulls hold (vertex count,
+// first vertex) before.
+hipError_t launch_support_factors(const SceneImg& img, char* blob, hipStream_t st);
 hipError_t launch_point_small(const SceneImg& img, const DevRobot& rb, const SmallPoints& qs, int* out,
                               hipStream_t st);
 hipError_t launch_fill_i32(int* p, int v, long long n, hipStream_t st);
