@@ -408,6 +408,17 @@ static SvaShape launch_shape(SvaShape sh, long long units) {
 }
 SvaShape launch_shape(const gprm_ctx* c, long long units) { return launch_shape(c->shape, units); }
 
+// What small point launches take beside `shape` (point_shape): its four-wave
+// variant, or none (grid 0).
+static SvaShape few_shape(const gprm_ctx* c, const SvaShape& shape) {
+  SvaShape few = shape;
+  few.waves = 4;
+  if (shape.waves == 5 && !shape.gscene && sva_shape_finish(c->img, &few, c->device) == hipSuccess &&
+      few.grid <= shape.grid)
+    return few;
+  return SvaShape{};
+}
+
 // Point checks of n items: the launch's shape before that cut and the pairs
 // of a unit.  While a wave would walk at most kFewPairs pairs, nearly all of
 // the launch is the waves' last full tests, as many chains of iterations as
@@ -892,12 +903,7 @@ int gprm_init(gprm_ctx* c, int rank, int size) {
   GPRM_HIP(launch_support_factors(c->img, c->img_buf.as<char>(), nullptr), "support certificates");
   c->shape = sva_default_shape(c->img);
   GPRM_HIP(sva_shape_finish(c->img, &c->shape, c->device), "separating-vector launch shape");
-  c->shape_few = SvaShape{};
-  if (c->shape.waves == 5 && !c->shape.gscene) {
-    SvaShape few = c->shape;
-    few.waves = 4;
-    if (sva_shape_finish(c->img, &few, c->device) == hipSuccess && few.grid <= c->shape.grid) c->shape_few = few;
-  }
+  c->shape_few = few_shape(c, c->shape);
   c->small_calls = point_small_prepare(c->img) == hipSuccess;
   GPRM_HIP(hipStreamSynchronize(nullptr), "support certificates");
   c->inited = true;
@@ -1162,10 +1168,8 @@ int gprm_get_launch_shape(gprm_ctx* c, gprm_launch_shape* out) {
   return GPRM_OK;
 }
 
-int gprm_set_launch_shape(gprm_ctx* c, const gprm_launch_shape* in) {
-  int rc = check_ready(c);
-  if (rc) return rc;
-  if (!in) return fail(c, GPRM_E_INVALID, "null argument");
+// few: small point launches take the shape's four-wave variant, as by default.
+static int set_shape(gprm_ctx* c, const gprm_launch_shape* in, bool few) {
   SvaShape sh;
   sh.block = in->block;
   sh.waves = in->waves;
@@ -1176,8 +1180,15 @@ int gprm_set_launch_shape(gprm_ctx* c, const gprm_launch_shape* in) {
   if (e != hipSuccess) return hip_fail(c, e, "launch shape");
   std::lock_guard<std::mutex> lk(c->mu);
   c->shape = sh;
-  c->shape_few = SvaShape{};  // the caller's shape holds for every launch
+  c->shape_few = few ? few_shape(c, sh) : SvaShape{};
   return GPRM_OK;
+}
+
+int gprm_set_launch_shape(gprm_ctx* c, const gprm_launch_shape* in) {
+  int rc = check_ready(c);
+  if (rc) return rc;
+  if (!in) return fail(c, GPRM_E_INVALID, "null argument");
+  return set_shape(c, in, false);  // the caller's shape holds for every launch
 }
 
 int gprm_autotune(gprm_ctx* c, const float* d_q, const float* d_qe, int n, long long offset, int reps,
@@ -1190,15 +1201,15 @@ int gprm_autotune(gprm_ctx* c, const float* d_q, const float* d_qe, int n, long 
   struct Free { int* p; ~Free() { (void)hipFree(p); } } fr{d_res};
   const gprm_launch_shape variants[] = {{256, 5, 0, 0}, {256, 4, 0, 0}, {1024, 4, 0, 0}};
   const int ppus[] = {32, 64, 128, 256};
-  gprm_launch_shape keep{};
-  if ((rc = gprm_get_launch_shape(c, &keep)) != GPRM_OK) return rc;
+  gprm_launch_shape found{};
+  if ((rc = gprm_get_launch_shape(c, &found)) != GPRM_OK) return rc;
+  const SvaShape keep = c->shape, keep_few = c->shape_few;
   double best_ms = 1e300;
-  gprm_launch_shape found = keep;
   for (const auto& v : variants)
     for (int ppu : ppus) {
       gprm_launch_shape sh = v;
       sh.pairs_per_unit = ppu;
-      if (gprm_set_launch_shape(c, &sh) != GPRM_OK) continue;  // not available for this scene
+      if (set_shape(c, &sh, true) != GPRM_OK) continue;  // not available for this scene
       // the median of reps timed runs after one warm-up
       std::vector<double> ts;
       for (int r = 0; r <= reps; ++r) {
@@ -1207,7 +1218,9 @@ int gprm_autotune(gprm_ctx* c, const float* d_q, const float* d_qe, int n, long 
                   : gprm_indicator_dev(c, d_q, d_res, n, offset, nullptr);
         const double t = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
         if (rc != GPRM_OK) {
-          (void)gprm_set_launch_shape(c, &keep);
+          std::lock_guard<std::mutex> lk(c->mu);
+          c->shape = keep;
+          c->shape_few = keep_few;
           return rc;
         }
         if (r > 0) ts.push_back(t);
@@ -1219,7 +1232,7 @@ int gprm_autotune(gprm_ctx* c, const float* d_q, const float* d_qe, int n, long 
         (void)gprm_get_launch_shape(c, &found);
       }
     }
-  if ((rc = gprm_set_launch_shape(c, &found)) != GPRM_OK) return rc;
+  if ((rc = set_shape(c, &found, true)) != GPRM_OK) return rc;
   *best = found;
   if (ms_best) *ms_best = (float)best_ms;
   return GPRM_OK;
