@@ -47,6 +47,12 @@ constexpr size_t kMiscBlocks = 32;
 // one stream per outstanding request, robotconfigspace.cpp:627-650).
 struct Slot {
   hipStream_t stream = nullptr;
+  // Never used, but created between the call's stream and the prep stream: the
+  // runtime deals streams to four hardware queues by their number, and without
+  // it the prep stream of a program's third scene got the queue of the call's
+  // stream, so that a round's preparation ran after the round before it instead
+  // of beside it (the 6-DOF roadmap's edges 2,009 -> 2,075 us).
+  hipStream_t spare = nullptr;
   hipEvent_t ev_prologue = nullptr;  // an edge call's prologue has finished
   EdgePinned* pinned = nullptr;      // pinned memory, what the host reads of an edge call
   // Edge launches after the first compact their items and compute their
@@ -83,6 +89,7 @@ struct Slot {
       if (stream) (void)hipStreamSynchronize(stream);
       (void)hipHostFree(small_out);
     }
+    if (spare) (void)hipStreamDestroy(spare);
     if (stream) (void)hipStreamDestroy(stream);
   }
 };

@@ -546,6 +546,7 @@ int run_edges(gprm_ctx* c, Slot& sl, const float* d_qs, const float* d_qe, long 
     *overflow = 0;
   }
   const bool need_max = host_maxT < 0;
+  if (need_max && !sl.spare) GPRM_HIP(hipStreamCreateWithFlags(&sl.spare, hipStreamNonBlocking), "hipStreamCreate");
   GPRM_HIP(launch_edge_prologue(c->rb, c->dq, ea, sl.testnum.as<int>(), d_max, d_total,
                                 reinterpret_cast<unsigned*>(sl.misc.as<char>() + kMiscBlocks),
                                 need_max ? sl.pinned : nullptr, st),
