@@ -45,7 +45,15 @@ constexpr int kItemBudget = 1 << 24;
 constexpr long long kOneRoundPlanned = 1LL << 32;
 // The same for calls of any edges (samples x pairs), whose largest testnum is
 // at most kOneRoundSamples: those may be mostly blocked, and a single round
-// tests all of a blocked edge's samples.
+// tests all of a blocked edge's samples.  One round / rounds by level, edges of
+// one length: 0.2 rad (a tenth to a fifth blocked) at 2^27 pair tests on the 4-,
+// 6- and 7-DOF scenes 922 / 994, 561 / 628, 384 / 447 us, 7-DOF at 2^28 616 / 699;
+// 0.6 rad (a third) 722 / 653, 456 / 460, 335 / 350 and at 2^28 1,262 / 1,122,
+// 732 / 687, 466 / 484; 1.5 rad (half) at 2^26 425 / 337, 299 / 275, 243 / 276 and
+// at 2^28 1,180 / 792, 692 / 506, 459 / 387.  So the line is right for short
+// edges; longer ones would want it nearer to 2^26.  Of more samples than that,
+// 3 rad: 100 edges 142 / 161, 154 / 163, 174 / 198 us, 1,600 224 / 231, 260 / 240,
+// 286 / 317, 6,400 425 / 284, 570 / 344, 593 / 377.
 constexpr long long kOneRoundAny = 1LL << 28;
 constexpr int kOneRoundSamples = 256;
 
@@ -449,12 +457,12 @@ int item_budget(const gprm_ctx* c) {
 // Edge launches of at least this many pair tests (item capacity x pairs) have
 // pair masks.  Below, the launch is bound by its longest full tests, not by
 // the bound tests that masks save, and writing them costs a few
-// microseconds: with / without, edges of up to 0.5 rad on the 7-DOF scene
-// (239 pairs) 128: 156 / 160, 2,048: 376 / 362, 8,192: 468 / 460, 20,011: 650 /
-// 805 us; of up to 1 rad on the 6-DOF scene (106 pairs) 8,192: 484 / 462,
-// 20,011: 745 / 767 us, on the 4-DOF scene (35 pairs) 20,011: 568 / 552 us; the
-// 6-DOF roadmap 2.55 / 3.41 ms.
-constexpr long long kMaskPairTests = 1LL << 27;
+// microseconds.  With / without, edges of 1 rad: 100 on the 7-DOF scene (239
+// pairs, 2^21.4) 123 / 121 us, 400 (2^23.4) 149 / 159, 1,600 201 / 244, 25,600
+// 694 / 1,072; on the 6-DOF scene (106 pairs) 100 (2^20.2) 112 / 111, 400
+// (2^22.2) 141 / 144, 6,400 314 / 382; on the 4-DOF scene (35 pairs) 400
+// (2^20.7) 121 / 120, 1,600 (2^22.6) 161 / 167, 25,600 524 / 576.
+constexpr long long kMaskPairTests = 1LL << 22;
 bool use_masks(const gprm_ctx* c, long long cap) {
   return cap * c->img.M >= kMaskPairTests && cull_fits(c->img, 256);
 }
