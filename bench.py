@@ -51,7 +51,8 @@ M_PAIRS = 0
 # instruction counts), measured by rocprofv3 on a build of the sources whose
 # hash the file records; see profiles/sva_kernel_edges_wl2_traffic.md.
 PROFILE_SIDECAR = os.path.join(ROOT, "profiles", "sva_kernel_edges_wl2.json")
-PROFILED_SOURCES = ("gpuprm_amd/csrc/kernels.hip", "gpuprm_amd/csrc/gprm_api.cpp", "gpuprm_amd/csrc/runtime.h")
+PROFILED_SOURCES = ("gpuprm_amd/csrc/kernels.hip", "gpuprm_amd/csrc/gprm_api.cpp", "gpuprm_amd/csrc/runtime.h",
+                    "gpuprm_amd/csrc/edge_plan.h")
 
 
 def sources_sha16():

@@ -5,8 +5,8 @@
 // into a device image that the separating-vector kernel stages in LDS.  Work
 // is split into chunks of at most kItemBudget configurations, each chunk
 // being one kinematics launch and one persistent separating-vector launch.
-// Edge queries run in rounds of ever finer samples (edge_levels); after every round the
-// samples of edges that are already blocked are no longer scheduled.
+// Edge queries run in rounds of ever finer samples (edge_plan.h); after every
+// round the samples of edges that are already blocked are no longer scheduled.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -1212,7 +1212,12 @@ int gprm_autotune(gprm_ctx* c, const float* d_q, const float* d_qe, int n, long 
   const int ppus[] = {32, 64, 128, 256};
   gprm_launch_shape found{};
   if ((rc = gprm_get_launch_shape(c, &found)) != GPRM_OK) return rc;
-  const SvaShape keep = c->shape, keep_few = c->shape_few;
+  SvaShape keep, keep_few;
+  {
+    std::lock_guard<std::mutex> lk(c->mu);
+    keep = c->shape;
+    keep_few = c->shape_few;
+  }
   double best_ms = 1e300;
   for (const auto& v : variants)
     for (int ppu : ppus) {

@@ -51,7 +51,6 @@ __device__ __forceinline__ V3 v3(float4 a) { return V3{a.x, a.y, a.z}; }
 #define GAS __attribute__((address_space(1)))
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ V3 v3(f32x4 a) { return V3{a.x, a.y, a.z}; }
-__device__ __forceinline__ GAS f32x4* global_f4(float4* p) { return (GAS f32x4*)p; }
 
 // sprod (geo4.h:130-132)
 __device__ __forceinline__ float dot3(const V3& u, const V3& v) {
@@ -912,7 +911,8 @@ struct Lds {
 // A lane's iteration history R[k] (x, y, z) and combs[k] (w: p | q << 16);
 // only iterations that do not separate touch it.  The first n entries are in
 // LDS (as many as fit beside the launch's resident blocks, history_entries),
-// the others in global memory, where a wave's entries are one 16 KB block.
+// the others in global memory, where a wave's kMaxIter entries are one 10 KB
+// block.
 // Lanes are adjacent in both.  Every iteration reads all entries before it,
 // two at a time: in memory, with entry k of all lanes of the launch together,
 // each read was a trip to the L2 and often to another page.  (3,001 points of
